@@ -591,8 +591,9 @@ int wf_batch_set_int(int* p, int n, int value, void* stream);
  *   WF_TUNE_SWEEP2_ICH_F64/F32  i-planes per workgroup of the two-sweep kernel
  *   WF_TUNE_SWEEP_PAIRS_F64/F32 pairs of sweeps of this level as 1 = two
  *                               one-sweep launches, 2 = one two-sweep launch
- *                               (built-in: 2 for FP64 levels of >= 2^23
- *                               cells, else 1)
+ * A level with none of the SWEEP tile, ICH and PAIRS knobs set takes the
+ * built-in smoother: blocks relaxed several times per launch on levels of
+ * fewer than 1.75e6 (FP64) or 3.5e6 (FP32) cells, two-sweep launches above.
  *   WF_TUNE_PROJ_ICH            i-planes per workgroup of wf_calvel3_calmas
  *                               (raised where needed to keep the workgroup
  *                               count within the reduction's partial slots)

@@ -23,6 +23,7 @@
 
 #include "batch.h"
 #include "mg_common.h"
+#include "relax_block.h"
 
 namespace wf {
 
@@ -1197,6 +1198,23 @@ sweep2_kernel(const T* __restrict__ pin, T* __restrict__ pout, const T* __restri
   sweep2_body<T, TJ, TK>(pin, pout, rhs, d, c0, c1, c2, ich, this_blk());
 }
 
+// ns sweeps of a level by overlapping blocks of RI x rj x rk cells, a thread per
+// (j, k) column (relax_block.h); tiles in x-fastest order, an XCD's share of
+// them contiguous.  The occupancy range keeps the register budget the block
+// was laid out for (FP32 94, FP64 124 VGPRs at RI = 16) without asking for
+// more waves than that leaves.
+template <class T, int RI, int PL, int NT, bool PART>
+__global__ void __launch_bounds__(NT)
+    __attribute__((amdgpu_waves_per_eu(NT / 256, sizeof(T) == 4 ? 5 : 4)))
+relax_block_kernel(const T* __restrict__ pin, T* pout, const T* __restrict__ rhs, MgDev d, T c0,
+                   T c1, T c2, int ns, int rj, int rk, int tj, int tk) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int b = xcd_linear(blockIdx.x, gridDim.x);
+  relax_block_body<T, RI, PL, PART>(pin, pout, rhs, d, c0, c1, c2, ns, rj, rk,
+                                    Blk{b % tk, (b / tk) % tj, b / (tk * tj)},
+                                    reinterpret_cast<T*>(smem_raw));
+}
+
 // n sweeps of RBGS on one small level held in LDS by one workgroup
 // (multigrid.py:289-299 with the refill folded in).  The real cells of phi
 // live in LDS; ring terms carry zero coefficients and are skipped.  rhs is
@@ -1806,6 +1824,17 @@ int max_lds() {
   return g_max_lds;
 }
 
+int cu_count() {
+  static const int n = [] {
+    int dev = 0, v = 256;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+      v = 256;
+    return v;
+  }();
+  return n;
+}
+
 template <class T>
 int launch_rbgs(const wf_mg_level& L, int color, int write_ring, hipStream_t s) {
   const MgDev d = mg_dev(L);
@@ -1950,8 +1979,15 @@ int launch_sweep2(const wf_mg_level& L, const void* pin, void* pout, hipStream_t
   // the kernel's plane offsets within a chunk ((ich + 8) planes) stay below 2^30
   const int64_t pb = d.s0 * (int64_t)sizeof(T);
   if ((int64_t)9 * pb >= ((int64_t)1 << 30)) return WF_EINVAL;
-  int ich = tuned > 0 ? tuned
-                      : (int)std::max<int64_t>(4, std::min<int64_t>(32, tiles * d.n0 / 1024));
+  // Chunks that fill the chip once: a CU holds three (FP32) or two (FP64)
+  // workgroups of the 8 x 64 and 16 x 32 tiles, and a chunk of ich planes runs
+  // ich + 9 iterations, so the fewest chunks that occupy it lose the least to
+  // their fill.  Six sweeps, 16 x 32 tiles: FP64 128^3 85 us with 8-plane
+  // chunks (512 workgroups) against 89 with 16, 256^3 404 with 64 (512)
+  // against 428 with 32; FP32 256^3 212 with 43 (768).
+  const int64_t slots = (sizeof(T) == 8 ? 2 : TJ * TK == 512 ? 3 : 2) * (int64_t)cu_count();
+  const int64_t nch = std::max<int64_t>(std::max<int64_t>(1, slots / tiles), div_up(d.n0, 64));
+  int ich = tuned > 0 ? tuned : std::max(4, div_up(d.n0, nch));
   ich = (int)std::min<int64_t>(ich, ((int64_t)1 << 30) / pb - 8);
   const dim3 grid(kt, jt, div_up(d.n0, ich));
   hipLaunchKernelGGL((sweep2_kernel<T, TJ, TK>), grid, dim3(256), 0, s, (const T*)pin, (T*)pout,
@@ -1972,15 +2008,143 @@ int sweep2_t(const wf_mg_level& L, const void* pin, void* pout, hipStream_t s) {
                    : launch_sweep2<T, 16, 32>(L, pin, pout, s);
 }
 
+// Relaxation by overlapping blocks (relax_block_kernel): the block shapes, and
+// the choice of shape and sweeps per launch for a level.
+//
+// A launch costs `base` us up to 256 blocks (one per CU) and `more` ns for each
+// further block, both measured (six sweeps, back to back, 24^3 .. 256^3); the
+// plan with the least total is taken.  Blocks of 16^3 cells (256 threads)
+// relax three times per launch while they fit the CUs once and twice above;
+// FP32 levels of many blocks take 32 x 32 columns (1024 threads, a halo of 4
+// in 32 instead of in 16), of 16 planes while they fit the CUs once, else 20.
+struct BlockShape {
+  int ri, rjk, ns;   // planes, rows and columns, sweeps per launch
+  double base, more; // us, ns per block past 256
+};
+template <class T>
+constexpr BlockShape BLOCK_SHAPES[] = {
+    {16, 16, 3, sizeof(T) == 4 ? 6.75 : 7.3, sizeof(T) == 4 ? 8.0 : 14.0},
+    {16, 16, 2, sizeof(T) == 4 ? 5.85 : 6.5, sizeof(T) == 4 ? 7.5 : 9.5},
+    {12, 16, 2, sizeof(T) == 4 ? 5.0 : 5.95, sizeof(T) == 4 ? 5.7 : 8.0},
+    {16, 32, 2, sizeof(T) == 4 ? 11.7 : 1e9, 35.0},
+    {20, 32, 2, sizeof(T) == 4 ? 14.6 : 1e9, 45.0},
+};
+struct BlockPlan {
+  int ri = 0, rj = 0, rk = 0;
+  bool part = false;
+  int launches = 0;
+};
+
+template <class T, int RI, int RJK, bool PART>
+int launch_relax_block(const wf_mg_level& L, const void* pin, void* pout, int ns, int rj, int rk,
+                       hipStream_t s) {
+  constexpr int PL = RJK == 16 ? 320 : 1152;  // (RJK + 2)(RJK + 1) words, whole bank rows
+  constexpr int NT = RJK * RJK;
+  constexpr size_t lds = (size_t)RI * PL * sizeof(T);
+  auto kern = relax_block_kernel<T, RI, PL, NT, PART>;
+  if constexpr (lds > 65536) {
+    static const hipError_t set = hipFuncSetAttribute(
+        (const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    WF_TRY(set);
+  }
+  const MgDev d = mg_dev(L);
+  T c0, c1, c2;
+  inv_h2(L, c0, c1, c2);
+  const int h = 2 * ns;
+  const int ti = relax_block_tiles(d.n0, RI, h), tj = relax_block_tiles(d.n1, rj, h),
+            tk = relax_block_tiles(d.n2, rk, h);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(ti * tj * tk)), dim3((unsigned)div_up(rj * rk, 64) * 64),
+                     lds, s, (const T*)pin, (T*)pout, (const T*)L.rhs, d, c0, c1, c2, ns, rj, rk,
+                     tj, tk);
+  WF_LAUNCHED();
+  return 0;
+}
+
+// The plan for n sweeps; even: the launches come in even numbers (the result
+// in phi).  False where blocks don't apply: a level tuned to another kernel,
+// one streaming is faster on, a level without tmp that is more than one block.
+template <class T>
+bool block_plan(const wf_mg_level& L, int n, bool even, BlockPlan& P) {
+  constexpr bool f64 = sizeof(T) == 8;
+  if (n < 1 || L.n1 < 2 || L.n2 < 2) return false;
+  for (int knob : f64 ? std::initializer_list<int>{WF_TUNE_SWEEP_TILE_F64, WF_TUNE_SWEEP_ICH_F64,
+                                                   WF_TUNE_SWEEP_PAIRS_F64}
+                      : std::initializer_list<int>{WF_TUNE_SWEEP_TILE_F32, WF_TUNE_SWEEP_ICH_F32,
+                                                   WF_TUNE_SWEEP_PAIRS_F32})
+    if (tune_get(knob, L.n0, L.n1, L.n2)) return false;
+  // Streaming two sweeps per launch is faster above (us per six sweeps, blocks
+  // against two-sweep launches): FP32 144^3 73 / 95, 160^3 104 / 95; FP64
+  // 112^3 69 / 80, 128^3 96 / 85.
+  const int64_t cells = (int64_t)L.n0 * L.n1 * L.n2;
+  if (cells >= (f64 ? 1750000 : 3500000)) return false;
+  const MgDev d = mg_dev(L);
+  if (d.s0 * (int64_t)sizeof(T) * 24 >= ((int64_t)1 << 30)) return false;  // lane offsets
+  if (L.n0 <= 16 && L.n1 <= 16 && L.n2 <= 16) {  // one block: every sweep in one launch, in place
+    P.ri = L.n0 <= 8 ? 8 : L.n0 <= 12 ? 12 : 16;
+    P.part = L.n0 < P.ri;
+    P.rj = L.n1;
+    P.rk = L.n2;
+    P.launches = 1;
+    return true;
+  }
+  if (!L.tmp || (even && n < 2)) return false;
+  double best = 0;
+  for (const BlockShape& S : BLOCK_SHAPES<T>) {
+    BlockPlan Q;
+    Q.ri = S.ri;
+    if (L.n0 < 16 && S.rjk == 16) {  // one block along i
+      if (S.ri == 12) continue;
+      Q.ri = L.n0 <= 8 ? 8 : L.n0 <= 12 ? 12 : 16;
+    }
+    if (S.rjk == 32 && L.n0 < S.ri) continue;
+    Q.part = L.n0 < Q.ri;
+    Q.rj = std::min(L.n1, S.rjk);
+    Q.rk = std::min(L.n2, S.rjk);
+    Q.launches = div_up(n, S.ns);
+    if (even) Q.launches += Q.launches & 1;
+    if (Q.launches > n) continue;
+    const int h = 2 * div_up(n, Q.launches);
+    const double blocks = (double)relax_block_tiles(L.n0, Q.ri, h) *
+                          relax_block_tiles(L.n1, Q.rj, h) * relax_block_tiles(L.n2, Q.rk, h);
+    const double cost = Q.launches * (S.base + 1e-3 * S.more * std::max(0.0, blocks - 256.0));
+    if (P.launches == 0 || cost < best) {
+      P = Q;
+      best = cost;
+    }
+  }
+  return P.launches > 0;
+}
+
+template <class T>
+int relax_block(const wf_mg_level& L, const BlockPlan& P, const void* pin, void* pout, int ns,
+                hipStream_t s) {
+  if (std::max(P.rj, P.rk) > 16) {
+    if constexpr (sizeof(T) == 4)
+      return P.ri == 16 ? launch_relax_block<T, 16, 32, false>(L, pin, pout, ns, P.rj, P.rk, s)
+                        : launch_relax_block<T, 20, 32, false>(L, pin, pout, ns, P.rj, P.rk, s);
+    return WF_EINVAL;
+  }
+  switch (P.ri) {
+    case 8: return launch_relax_block<T, 8, 16, true>(L, pin, pout, ns, P.rj, P.rk, s);
+    case 12:
+      return P.part ? launch_relax_block<T, 12, 16, true>(L, pin, pout, ns, P.rj, P.rk, s)
+                    : launch_relax_block<T, 12, 16, false>(L, pin, pout, ns, P.rj, P.rk, s);
+    default:
+      return P.part ? launch_relax_block<T, 16, 16, true>(L, pin, pout, ns, P.rj, P.rk, s)
+                    : launch_relax_block<T, 16, 16, false>(L, pin, pout, ns, P.rj, P.rk, s);
+  }
+}
+
 // nsweeps RBGS sweeps of L.  Pairs of sweeps run as two-sweep launches
 // (phi -> tmp, then tmp -> phi, ...); with allow_swap an odd number of them
 // may leave the result in tmp, which *swapped reports (the caller then
 // treats tmp as the level's phi); without it the pairs go in even numbers
 // and the rest as one-sweep launches, so the result is in phi.
 // Which smoother relax_t runs for nsweeps sweeps of level L.
-enum class RelaxPath { LDS2, LDS_RHS, LDS, SWEEPS };
+enum class RelaxPath { BLOCKS, LDS2, LDS_RHS, LDS, SWEEPS };
 template <class T>
-RelaxPath relax_path(const wf_mg_level& L, int nsweeps) {
+RelaxPath relax_path(const wf_mg_level& L, int nsweeps, bool even, BlockPlan& P) {
+  if (block_plan<T>(L, nsweeps, even, P)) return RelaxPath::BLOCKS;
   const size_t cells = (size_t)L.n0 * L.n1 * L.n2;
   const size_t lds = (size_t)max_lds();
   // levels whose zero-ringed copy fits LDS: all sweeps in one workgroup
@@ -1993,11 +2157,13 @@ RelaxPath relax_path(const wf_mg_level& L, int nsweeps) {
   if (cells <= LDS_RELAX_MAX_CELLS && cells * sizeof(T) <= lds) return RelaxPath::LDS;
   return RelaxPath::SWEEPS;
 }
-// True when relax_t's first launch for nsweeps sweeps of L is a full-sweep
-// kernel, which can take a zero iterate without reading it (zero_start).
+// True when relax_t's first launch for nsweeps sweeps of L is a full-sweep or
+// block kernel, which can take a zero iterate without reading it (zero_start).
 template <class T>
 bool relax_zero_start_ok(const wf_mg_level& L, int nsweeps) {
-  return nsweeps >= 2 && L.tmp && relax_path<T>(L, nsweeps) == RelaxPath::SWEEPS;
+  BlockPlan P;
+  const RelaxPath p = relax_path<T>(L, nsweeps, true, P);
+  return nsweeps >= 2 && L.tmp && (p == RelaxPath::BLOCKS || p == RelaxPath::SWEEPS);
 }
 
 // zero_start: the iterate in L.phi is to be taken as zero (the caller has
@@ -2008,7 +2174,22 @@ int relax_t(const wf_mg_level& L, int nsweeps, hipStream_t s, bool allow_swap = 
   if (swapped) *swapped = false;
   if (nsweeps <= 0) return 0;
   const size_t cells = (size_t)L.n0 * L.n1 * L.n2;
-  switch (relax_path<T>(L, nsweeps)) {
+  BlockPlan P;
+  switch (relax_path<T>(L, nsweeps, !allow_swap, P)) {
+    case RelaxPath::BLOCKS: {
+      const void* in = zero_start ? nullptr : L.phi;
+      if (P.launches == 1 && L.n0 <= 16 && L.n1 <= 16 && L.n2 <= 16)
+        return relax_block<T>(L, P, in, L.phi, nsweeps, s);  // one block, in place
+      wf_mg_level C = L;
+      for (int q = 0; q < P.launches; ++q) {
+        const int ns = nsweeps / P.launches + (q < nsweeps % P.launches);
+        WF_TRY((hipError_t)relax_block<T>(C, P, in, C.tmp, ns, s));
+        std::swap(C.phi, C.tmp);
+        in = C.phi;
+      }
+      if (swapped) *swapped = C.phi != L.phi;
+      return 0;
+    }
     case RelaxPath::LDS2:
       return launch_relax_lds2<T>(L, nsweeps, s);
     case RelaxPath::LDS_RHS:
@@ -2029,8 +2210,8 @@ int relax_t(const wf_mg_level& L, int nsweeps, hipStream_t s, bool allow_swap = 
   int q = 0;
   const int pairs = tune_get(sizeof(T) == 8 ? WF_TUNE_SWEEP_PAIRS_F64 : WF_TUNE_SWEEP_PAIRS_F32,
                              L.n0, L.n1, L.n2);
-  // built-in: two-sweep launches where they measured faster (FP64, >= 2^23 cells)
-  if (C.tmp && (pairs == 2 || (pairs == 0 && sizeof(T) == 8 && cells >= ((size_t)1 << 23)))) {
+  // built-in: two-sweep launches on the levels too large for blocks (block_plan)
+  if (C.tmp && (pairs == 2 || (pairs == 0 && cells >= (sizeof(T) == 8 ? 1750000u : 3500000u)))) {
     int npair = nsweeps / 2;
     if (!allow_swap) npair &= ~1;
     for (int f = 0; f < npair; ++f) {

@@ -307,6 +307,17 @@ def _tune_level(lev, T, reps, out):
                 "x".join(map(str, n3)), "f64" if f64 else "f32", tile, ich)] = round(t, 2)
             if best is None or t < best[0]:
                 best = (t, tile, ich)
+    # the built-in smoother (blocks of several sweeps per launch on the smaller
+    # levels), a V-cycle phase of six sweeps on each side of it, per sweep
+    def relax12():
+        copy(lev.phi, keep_phi)
+        _hip.call("wf_mg_relax", C.byref(d), 12, current_stream())
+    set_shape(ktile, n3, 0)
+    set_shape(kich, n3, 0)
+    t_builtin = (T.us(relax12, reps) - t_copy) / 12
+    out["timings_us"]["sweep %s %s built-in" % (
+        "x".join(map(str, n3)), "f64" if f64 else "f32")] = round(t_builtin, 2)
+    ntuned = len(out["entries"])
     set_shape(ktile, n3, best[1])
     set_shape(kich, n3, best[2])
     out["entries"] += [(ktile, tuple(n3), best[1]), (kich, tuple(n3), best[2])]
@@ -350,6 +361,10 @@ def _tune_level(lev, T, reps, out):
     else:
         set_shape(kpairs, n3, 1)
         out["entries"].append((kpairs, tuple(n3), 1))
+    if t_builtin <= min(t_single, best2[0]) / 4:  # leave the level to the built-in choice
+        for knob, _, _ in out["entries"][ntuned:]:
+            set_shape(knob, n3, 0)
+        del out["entries"][ntuned:]
     copy(lev.phi, keep_phi)
     copy(lev.tmp, keep_tmp)
 
