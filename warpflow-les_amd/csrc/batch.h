@@ -91,6 +91,7 @@ enum PlanKind : int {
   PK_CDE,           // u's edge planes 0 and ni-2: 8 x 32 (j, k) tiles x 2
   PK_XG,            // w's cross-ghost cells of each real plane, 256 per item
   PK_MEMBER,        // one item per member
+  PK_COP,           // 32-row blocks of the coarsest level's operator
   PK_LCELLS0,       // 64x4 blocks over level-l real cells, l = 0 .. 7
   PK_SWEEP0 = PK_LCELLS0 + BATCH_MAX_LEVELS,  // fused-sweep tiles of level l
   PK_COUNT = PK_SWEEP0 + BATCH_MAX_LEVELS
@@ -111,7 +112,7 @@ struct Batch {
   int64_t field_elems = 0;
   int64_t level_elems[BATCH_MAX_LEVELS] = {};
   int64_t cop_elems = 0;
-  int max_coarse_cells = 0, max_lds_cells[BATCH_MAX_LEVELS] = {};
+  int max_lds_cells[BATCH_MAX_LEVELS] = {};
   int lds = 0;  // dynamic LDS bytes available to one workgroup
   BView view() const { return BView{mem_dev, nmem}; }
 };

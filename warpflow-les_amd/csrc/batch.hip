@@ -75,6 +75,10 @@ int member_count(int kind, const MemDev& M) {
       return ((2 * (n2 + 3) + 4 * n1 + 255) / 256) * n0;
     case PK_MEMBER:
       return 1;
+    case PK_COP: {
+      const int* c = M.ln[M.nlev - 1];
+      return (c[0] * c[1] * c[2] + 31) / 32;
+    }
     default:
       break;
   }
@@ -119,7 +123,7 @@ int create(const wf_member* mem, int nmem, int nlev, Batch** out) {
   B->nlev = nlev;
   B->mem_host = new MemDev[nmem];
   int64_t foff = 0, loff[BATCH_MAX_LEVELS] = {}, coff = 0;
-  int red = 0, sum = 0, maxc = 0;
+  int red = 0, sum = 0;
   for (int m = 0; m < nmem; ++m) {
     const wf_member& a = mem[m];
     MemDev& M = B->mem_host[m];
@@ -159,7 +163,6 @@ int create(const wf_member* mem, int nmem, int nlev, Batch** out) {
     } else {
       M.coff = -1;
     }
-    maxc = std::max(maxc, cc);
     M.red0 = red;
     red += red_blocks(a.n0, a.n1, a.n2);
     M.sum0 = sum;
@@ -168,7 +171,6 @@ int create(const wf_member* mem, int nmem, int nlev, Batch** out) {
   B->field_elems = foff;
   for (int l = 0; l < nlev; ++l) B->level_elems[l] = loff[l];
   B->cop_elems = coff;
-  B->max_coarse_cells = maxc;
   B->nred = red;
   B->nsum = sum;
 

@@ -1410,77 +1410,140 @@ coarse_op_build_kernel(T* __restrict__ M, MgDev d, T c0, T c1, T c2, int nsweeps
 }
 
 // phi = M rhs on the real cells of a small level, plus face-ring images.
-// acc + m * r with one rounding, as both coarse-operator kernels accumulate
+// acc + m * r with one rounding, as the coarse-operator kernels accumulate
 __device__ inline float cop_fma(float m, float r, float acc) { return __builtin_fmaf(m, r, acc); }
 __device__ inline double cop_fma(double m, double r, double acc) {
   return __builtin_fma(m, r, acc);
 }
+// Rows [x*COP_ROWS, (x+1)*COP_ROWS) of the product, COP_ROWS rows making a
+// 128-byte line of each column.  A row is one lane's serial sum in column
+// order, a chain of ncell FMAs (2.4 ns each); what took the time was waiting for
+// M, 64 loads a row at a time (512 cells FP32 14.7 us, 2145 cells 62; batched, a
+// workgroup per member, 177 for a member of 1728).  Here waves that only fetch
+// bring COP_COLS columns a round trip into one of two LDS buffers, the round
+// trip after that already under way, while a wave of its own sums the other;
+// 16-byte LDS reads keep the sum near one instruction per FMA.  512 cells FP32
+// 5.8 us, 2145 cells 16; FP64 512 cells 6.5 (14.0).
+constexpr int COP_COLS = 256;
 template <class T>
-__device__ inline void coarse_op_apply_body(const T* __restrict__ M, T* __restrict__ phi,
-                                            const T* __restrict__ rhs, const MgDev& d, T* r) {
-  const int n0 = d.n0, n1 = d.n1, n2 = d.n2;
-  const int ncell = n0 * n1 * n2;
-  const int nt = blockDim.x, tid = threadIdx.x;
-  for (int l = tid; l < ncell; l += nt) {
-    const int k = l % n2, j = (l / n2) % n1, i = l / (n1 * n2);
-    r[l] = rhs[mg_at(d, i, j, k)];
-  }
-  __syncthreads();
-  for (int row = tid; row < ncell; row += nt) {
-    // serial sum in column order; the loads of 16 columns are issued
-    // before their products so that one workgroup keeps them in flight
-    T acc = T(0);
-    int col = 0;
-    for (; col + 16 <= ncell; col += 16) {
-      T m[16];
+constexpr int COP_WAVES = sizeof(T) == 4 ? 8 : 4;  // fetching (FP64: 4 measured 10-20% below 8)
+template <class T>
+constexpr int COP_ROWS = 128 / (int)sizeof(T);
+template <class T>
+constexpr int COP_PITCH = COP_COLS + 16 / (int)sizeof(T);  // words of a row's chunk in LDS
+template <class T>
+constexpr size_t COP_LDS = 2 * sizeof(T) * (COP_ROWS<T> * COP_PITCH<T> + COP_COLS);
+template <class T>
+__device__ inline void coarse_op_rows_body(const T* __restrict__ M, T* __restrict__ phi,
+                                           const T* __restrict__ rhs, const MgDev& d, int x,
+                                           T* __restrict__ sm) {
+  constexpr int V = 16 / (int)sizeof(T);             // columns of a 16-byte LDS access
+  using TV = T __attribute__((ext_vector_type(V)));
+  constexpr int R = COP_ROWS<T>, PW = COP_PITCH<T>;
+  constexpr int NG = 64 * COP_WAVES<T> / R * V;         // columns the waves fetch per V loads
+  constexpr int NQ = COP_COLS / NG;                  // such groups of loads per chunk
+  constexpr int NB = R * PW + COP_COLS;              // words of a buffer: M's, then rhs's
+  constexpr int CB = 16;                             // columns read from LDS while CB are summed
+  static_assert(COP_COLS <= 64 * COP_WAVES<T>, "one right-hand side per thread and chunk");
+  static_assert(NG % (2 * CB) == 0, "the columns summed past the end are fetched zeros");
+  const int n1 = d.n1, n2 = d.n2;
+  const int ncell = d.n0 * n1 * n2;
+  const int tid = (int)threadIdx.x - 64;  // of the fetching waves
+  const bool sums = tid < 0;              // the first wave
+  const int rl = (int)threadIdx.x % R, row = x * R + rl;
+  const int cg = tid / R * V;             // this lane's first column of a group
+  const int cs = ncell * (int)sizeof(T);
+  const uint32_t off = (uint32_t)(cg * cs + row * (int)sizeof(T));
+  TV m[2][NQ];
+  T rv[2];
+  // Columns cb .. cb + COP_COLS - 1: buffer loads whose range ends with M, so
+  // that nothing is tested and columns past the end are zeros (rows past the
+  // end are summed and dropped).
+  auto fetch = [&](auto Wc, int cb) {
+    constexpr int W = decltype(Wc)::value;
+    const int left = min(COP_COLS, ncell - cb);
+    if (left <= 0) return;
+    const auto src = buf_rsrc(M + (size_t)cb * ncell, (uint32_t)(left * cs));
 #pragma unroll
-      for (int q = 0; q < 16; ++q) m[q] = M[(size_t)(col + q) * ncell + row];
+    for (int q = 0; q < NQ; ++q) {
+      if (q * NG >= left) break;
 #pragma unroll
-      for (int q = 0; q < 16; ++q) acc = cop_fma(m[q], r[col + q], acc);
+      for (int e = 0; e < V; ++e) m[W][q][e] = buf_ld<T>(src, off, (q * NG + e) * cs);
     }
-    for (; col < ncell; ++col) acc = cop_fma(M[(size_t)col * ncell + row], r[col], acc);
-    const int k = row % n2, j = (row / n2) % n1, i = row / (n1 * n2);
-    const int64_t x = mg_at(d, i, j, k);
-    phi[x] = acc;
-    ring_images(phi, d, i, j, k, x, acc);
-  }
-}
-// The rows of coarse_op_apply_body spread over one 64-thread workgroup per 64 rows, so that the
-// matrix streams through many CUs instead of one; each row is still one
-// thread's serial sum in column order (the bits of coarse_op_apply_body).
-template <class T>
-__global__ void __launch_bounds__(64)
-coarse_op_apply_rows_kernel(const T* __restrict__ M, T* __restrict__ phi,
-                            const T* __restrict__ rhs, MgDev d) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  T* r = reinterpret_cast<T*>(smem_raw);
-  const int n0 = d.n0, n1 = d.n1, n2 = d.n2;
-  const int ncell = n0 * n1 * n2;
-  const int tid = threadIdx.x;
-  for (int l = tid; l < ncell; l += 64) {
-    const int k = l % n2, j = (l / n2) % n1, i = l / (n1 * n2);
-    r[l] = rhs[mg_at(d, i, j, k)];
+    rv[W] = T(0);
+    if (tid < left) {
+      const int col = cb + tid;
+      const int k = col % n2, j = (col / n2) % n1, i = col / (n1 * n2);
+      rv[W] = rhs[mg_at(d, i, j, k)];
+    }
+  };
+  auto keep = [&](auto Wc, int cb) {
+    constexpr int W = decltype(Wc)::value;
+    T* const b = sm + W * NB;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      if (q * NG >= ncell - cb) break;
+      *reinterpret_cast<TV*>(b + rl * PW + q * NG + cg) = m[W][q];
+    }
+    if (tid < COP_COLS) b[R * PW + tid] = rv[W];
+  };
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+  if (!sums) {
+    fetch(I0{}, 0);
+    fetch(I1{}, COP_COLS);
+    keep(I0{}, 0);
+    fetch(I0{}, 2 * COP_COLS);
   }
   __syncthreads();
-  const int row = blockIdx.x * 64 + tid;
-  if (row >= ncell) return;
-  // CB columns' loads in flight before their products: the few workgroups
-  // of a coarse level wait for one memory round trip per CB columns
-  constexpr int CB = sizeof(T) == 4 ? 64 : 32;
   T acc = T(0);
-  int col = 0;
-  for (; col + CB <= ncell; col += CB) {
-    T m[CB];
+  auto step = [&](auto Wc, auto Vc, int cb) {  // sum buffer W, fill the other
+    constexpr int W = decltype(Wc)::value;
+    if (sums) {
+      const TV* const bm = reinterpret_cast<const TV*>(sm + W * NB + rl * PW);
+      const TV* const br = reinterpret_cast<const TV*>(sm + W * NB + R * PW);
+      TV a[2][CB / V], r[2][CB / V];
+      auto get = [&](int b, int c) {
 #pragma unroll
-    for (int q = 0; q < CB; ++q) m[q] = M[(size_t)(col + q) * ncell + row];
+        for (int q = 0; q < CB / V; ++q) {
+          a[b][q] = bm[c / V + q];
+          r[b][q] = br[c / V + q];
+        }
+      };
+      const int nc = min(COP_COLS, ncell - cb);
+      get(0, 0);
+      for (int c = 0; c < nc; c += 2 * CB) {
 #pragma unroll
-    for (int q = 0; q < CB; ++q) acc = cop_fma(m[q], r[col + q], acc);
+        for (int b = 0; b < 2; ++b) {
+          // (the last read of a full chunk is its first columns again)
+          get(b ^ 1, (c + (b + 1) * CB) % COP_COLS);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int q = 0; q < CB; ++q) acc = cop_fma(a[b][q / V][q % V], r[b][q / V][q % V], acc);
+        }
+      }
+    } else if (cb + COP_COLS < ncell) {
+      keep(Vc, cb + COP_COLS);
+      fetch(Vc, cb + 3 * COP_COLS);
+    }
+    __syncthreads();
+  };
+  for (int cb = 0; cb < ncell; cb += 2 * COP_COLS) {
+    step(I0{}, I1{}, cb);
+    if (cb + COP_COLS < ncell) step(I1{}, I0{}, cb + COP_COLS);
   }
-  for (; col < ncell; ++col) acc = cop_fma(M[(size_t)col * ncell + row], r[col], acc);
+  if ((int)threadIdx.x >= R || row >= ncell) return;
   const int k = row % n2, j = (row / n2) % n1, i = row / (n1 * n2);
-  const int64_t x = mg_at(d, i, j, k);
-  phi[x] = acc;
-  ring_images(phi, d, i, j, k, x, acc);
+  const int64_t xc = mg_at(d, i, j, k);
+  phi[xc] = acc;
+  ring_images(phi, d, i, j, k, xc, acc);
+}
+template <class T>
+__global__ void __launch_bounds__(64 * (COP_WAVES<T> + 1))
+coarse_op_rows_kernel(const T* __restrict__ M, T* __restrict__ phi, const T* __restrict__ rhs,
+                      MgDev d) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  coarse_op_rows_body<T>(M, phi, rhs, d, blockIdx.x, reinterpret_cast<T*>(smem_raw));
 }
 
 // Coarse operators of more than COARSE_OP_SERIAL_MAX_CELLS cells (a 20^3
@@ -1683,16 +1746,18 @@ batch_relax_lds_kernel(BView V, int l, float* phi, const float* rhs, int nsweeps
                               reinterpret_cast<float*>(smem_raw));
 }
 
-// phi = M rhs on the coarsest level l, one workgroup per member
-__global__ void __launch_bounds__(1024)
-batch_coarse_apply_kernel(BView V, int l, const float* cop, float* phi, const float* rhs,
-                          const int* active) {
+// phi = M rhs on the coarsest level l, a workgroup per member and COP_ROWS rows
+// (one per member took 177 us where a member's M is 1728^2, as long as that
+// member alone)
+__global__ void __launch_bounds__(64 * (COP_WAVES<float> + 1))
+batch_coarse_rows_kernel(BView V, Plan P, int l, const float* cop, float* phi, const float* rhs,
+                         const int* active) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  const int m = blockIdx.x;
-  if (active && !active[m]) return;
+  const int m = member_of(P.start, V.nmem, blockIdx.x);
+  if (active && !active[m]) return;  // uniform per workgroup
   const MemDev& M = V.mem[m];
-  coarse_op_apply_body<float>(cop + M.coff, phi + M.loff[l], rhs + M.loff[l], level_dev(M, l),
-                              reinterpret_cast<float*>(smem_raw));
+  coarse_op_rows_body<float>(cop + M.coff, phi + M.loff[l], rhs + M.loff[l], level_dev(M, l),
+                             blockIdx.x - P.start[m], reinterpret_cast<float*>(smem_raw));
 }
 
 int batch_lds_bytes() {
@@ -1709,8 +1774,8 @@ int batch_mg_init(int* lds_out) {
   const int lds = batch_lds_bytes();
   WF_TRY(hipFuncSetAttribute((const void*)batch_relax_lds_kernel,
                              hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-  WF_TRY(hipFuncSetAttribute((const void*)batch_coarse_apply_kernel,
-                             hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+  WF_TRY(hipFuncSetAttribute((const void*)batch_coarse_rows_kernel,
+                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)COP_LDS<float>));
   *lds_out = lds;
   return 0;
 }
@@ -1753,9 +1818,9 @@ int batch_vcycle(const Batch& B, float* const* phi, float* const* rhs, float* co
       WF_LAUNCHED();
     }
     if (l > 0 && l == nlev - 1 && cop) {
-      hipLaunchKernelGGL(batch_coarse_apply_kernel, dim3(B.nmem), dim3(1024),
-                         (size_t)B.max_coarse_cells * sizeof(float), s, V, l, cop, phi[l],
-                         (const float*)rhs[l], active);
+      const Plan& P = B.plan[PK_COP];
+      hipLaunchKernelGGL(batch_coarse_rows_kernel, dim3(P.total), dim3(64 * (COP_WAVES<float> + 1)),
+                         COP_LDS<float>, s, V, P, l, cop, phi[l], (const float*)rhs[l], active);
       WF_LAUNCHED();
       continue;
     }
@@ -2318,7 +2383,6 @@ template <class T>
 int coarse_op_apply_t(const wf_mg_level& L, hipStream_t s) {
   const MgDev d = mg_dev(L);
   const int ncell = d.n0 * d.n1 * d.n2;
-  const size_t bytes = (size_t)ncell * sizeof(T);
   if (ncell > COARSE_OP_MAX_CELLS) return WF_EINVAL;
   if (ncell > COARSE_OP_SERIAL_MAX_CELLS) {
     const int nch = cop_split_chunks(ncell), clen = div_up(ncell, nch);
@@ -2333,15 +2397,13 @@ int coarse_op_apply_t(const wf_mg_level& L, hipStream_t s) {
     WF_LAUNCHED();
     return 0;
   }
-  if (bytes > (size_t)max_lds()) return WF_EINVAL;
-  static bool attr_set = false;
-  if (!attr_set) {
-    WF_TRY(hipFuncSetAttribute((const void*)coarse_op_apply_rows_kernel<T>,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, max_lds()));
-    attr_set = true;
-  }
-  hipLaunchKernelGGL(coarse_op_apply_rows_kernel<T>, dim3((unsigned)div_up(ncell, 64)),
-                     dim3(64), bytes, s, (const T*)L.cop, (T*)L.phi, (const T*)L.rhs, d);
+  static const hipError_t set =
+      hipFuncSetAttribute((const void*)coarse_op_rows_kernel<T>,
+                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)COP_LDS<T>);
+  WF_TRY(set);
+  hipLaunchKernelGGL(coarse_op_rows_kernel<T>, dim3((unsigned)div_up(ncell, COP_ROWS<T>)),
+                     dim3(64 * (COP_WAVES<T> + 1)), COP_LDS<T>, s, (const T*)L.cop, (T*)L.phi,
+                     (const T*)L.rhs, d);
   WF_LAUNCHED();
   return 0;
 }
