@@ -41,3 +41,25 @@ def test_blocks_equal_one_sweep_launches(gpu, prec, n3):
     for n in (2, 3, 6, 7):
         want = relax(lev, phi, n, True)
         assert np.array_equal(relax(lev, phi, n, False), want), n
+
+
+# members whose levels are one block each (all sweeps in one launch), a few
+# blocks, and blocks of fewer planes than the kernel's
+@pytest.mark.parametrize("sizes,levels", [([(16, 12, 8), (12, 8, 16)], 2),
+                                          ([(20, 36, 24), (28, 12, 16), (36, 20, 44)], 2),
+                                          ([(56, 40, 24), (24, 72, 56)], 4)])
+def test_batched_blocks_equal_single_solvers(gpu, sizes, levels):
+    from warpflow import FlowSolver, build_topology
+    from warpflow.ensemble import Ensemble, MemberSpec, member_config
+    specs = [MemberSpec(n3, 200.0 + 100.0 * m, m + 1) for m, n3 in enumerate(sizes)]
+    ens = Ensemble(specs, 5e-4, mg_levels=levels)
+    for _ in range(2):
+        ens.step()
+    for m, sp in enumerate(specs):
+        cfg = member_config(sp, 5e-4, mg_levels=levels)
+        sol = FlowSolver(cfg, build_topology(cfg), "hip:0")
+        for _ in range(2):
+            sol.step()
+        for name in ("u", "v", "w", "p"):
+            assert np.array_equal(ens.field(name, m).numpy(), sol.f[name].numpy()), (m, name)
+    ens.close()

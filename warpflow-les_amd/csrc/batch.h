@@ -12,6 +12,8 @@
 // A per-member `active` mask (nullable) lets converged members skip the
 // projection iterations of the others inside one captured graph.
 #pragma once
+#include <vector>
+
 #include "wf_common.h"
 
 namespace wf {
@@ -29,6 +31,7 @@ struct MemDev {
   int nlev;
   int ln[BATCH_MAX_LEVELS][3];
   int64_t loff[BATCH_MAX_LEVELS];
+  float lc[BATCH_MAX_LEVELS][3];  // 1/h^2 of each level, as the single-domain path forms it
   int64_t coff;  // coarse-operator offset (elements) in the operator pool
   int red0;      // first reduction-partial slot of this member
   int sum0;      // first sum-partial slot of this member
@@ -93,8 +96,17 @@ enum PlanKind : int {
   PK_MEMBER,        // one item per member
   PK_COP,           // 32-row blocks of the coarsest level's operator
   PK_LCELLS0,       // 64x4 blocks over level-l real cells, l = 0 .. 7
-  PK_SWEEP0 = PK_LCELLS0 + BATCH_MAX_LEVELS,  // fused-sweep tiles of level l
-  PK_COUNT = PK_SWEEP0 + BATCH_MAX_LEVELS
+  PK_COUNT = PK_LCELLS0 + BATCH_MAX_LEVELS
+};
+
+// How a level of every member relaxes: one workgroup per item (member, block
+// coordinates x, y, z) of a table made at creation.
+struct BatchRelax {
+  const int4* item = nullptr;  // device
+  int total = 0;
+  bool single = false;  // every member is one block: all sweeps in one launch, in place
+  int rjk = 0, ns = 0;  // blocks: rows and columns, sweeps per launch
+  int ich = 0;          // > 0: two-sweep launches in chunks of ich planes instead
 };
 
 // Host side of a batch (defined in batch.hip).
@@ -104,6 +116,7 @@ struct Batch {
   MemDev* mem_host = nullptr;       // host copy
   Plan plan[PK_COUNT];
   int* plan_mem[PK_COUNT] = {};     // device start arrays
+  BatchRelax relax[BATCH_MAX_LEVELS];
   double* red_part = nullptr;       // 4 * nred reduction partials (device)
   int nred = 0;
   double* sum_part = nullptr;       // nsum sum partials (device)
@@ -113,7 +126,6 @@ struct Batch {
   int64_t level_elems[BATCH_MAX_LEVELS] = {};
   int64_t cop_elems = 0;
   int max_lds_cells[BATCH_MAX_LEVELS] = {};
-  int lds = 0;  // dynamic LDS bytes available to one workgroup
   BView view() const { return BView{mem_dev, nmem}; }
 };
 
@@ -129,15 +141,6 @@ __host__ __device__ inline void op_dims(int c, int n0, int n1, int n2, int& d0, 
   d1 = n1 - (c == 1);
   d2 = n2 - (c == 2);
 }
-// Fused-sweep tiles of a level (the single-domain tile choice).
-__host__ __device__ inline int sweep_tj(int n2) { return n2 > 32 ? 8 : 16; }
-__host__ __device__ inline int sweep_tk(int n2) { return n2 > 32 ? 64 : 32; }
-constexpr int BATCH_SWEEP_ICH = 8;
-__host__ __device__ inline int sweep_tiles(int n0, int n1, int n2) {
-  return ((n2 + sweep_tk(n2) - 1) / sweep_tk(n2)) * ((n1 + sweep_tj(n2) - 1) / sweep_tj(n2)) *
-         ((n0 + BATCH_SWEEP_ICH - 1) / BATCH_SWEEP_ICH);
-}
-
 // Batched launchers, one per source file (argument checks done by the C ABI).
 int batch_noise(const Batch& B, double* u, double* v, double* w, hipStream_t s);
 int batch_fill_vis(const Batch& B, double* vis, hipStream_t s);
@@ -173,9 +176,11 @@ int batch_bc_fill_n(const Batch& B, double* const* f, const int* which, int nf,
                     const int* active, hipStream_t s);
 int batch_vcycle(const Batch& B, float* const* phi, float* const* rhs, float* const* tmp,
                  const float* cop, int npre, int npost, int ncoarse, const int* active,
-                 hipStream_t s);
+                 hipStream_t s, bool zero0);
 int bc_blocks(int axis, int ni, int nj, int nk);
-int batch_mg_init(int* lds_out);
+int batch_mg_init();
+void batch_relax_plan(const MemDev* mem, int nmem, int l, BatchRelax& P,
+                      std::vector<int4>& items);
 int batch_mg_mixed(const Batch& B, float* const* phi, float* const* rhs, float* const* tmp,
                    const float* cop, const double* su, double* pp, int ncycles, int npre,
                    int npost, int ncoarse, int flags, const int* active, hipStream_t s);

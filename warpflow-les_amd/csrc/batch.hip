@@ -87,11 +87,6 @@ int member_count(int kind, const MemDev& M) {
     if (l >= M.nlev) return 0;
     return cells_blocks(M.ln[l][0], M.ln[l][1], M.ln[l][2]);
   }
-  if (kind >= PK_SWEEP0 && kind < PK_SWEEP0 + BATCH_MAX_LEVELS) {
-    const int l = kind - PK_SWEEP0;
-    if (l >= M.nlev) return 0;
-    return sweep_tiles(M.ln[l][0], M.ln[l][1], M.ln[l][2]);
-  }
   return 0;
 }
 
@@ -99,6 +94,8 @@ void batch_free(Batch* B) {
   if (!B) return;
   for (int k = 0; k < PK_COUNT; ++k)
     if (B->plan_mem[k]) (void)hipFree(B->plan_mem[k]);
+  for (int l = 0; l < BATCH_MAX_LEVELS; ++l)
+    if (B->relax[l].item) (void)hipFree(const_cast<int4*>(B->relax[l].item));
   if (B->mem_dev) (void)hipFree(B->mem_dev);
   if (B->red_part) (void)hipFree(B->red_part);
   if (B->sum_part) (void)hipFree(B->sum_part);
@@ -152,6 +149,8 @@ int create(const wf_member* mem, int nmem, int nlev, Batch** out) {
       M.ln[l][1] = a.n1 >> l;
       M.ln[l][2] = a.n2 >> l;
       M.loff[l] = loff[l];
+      const double f = (double)(1 << l), h[3] = {a.dx * f, a.dy * f, a.dz * f};
+      for (int d = 0; d < 3; ++d) M.lc[l][d] = (float)(1.0 / (h[d] * h[d]));
       loff[l] = align_up(loff[l] + (int64_t)(M.ln[l][0] + 2) * (M.ln[l][1] + 2) * (M.ln[l][2] + 2));
       const int cells = M.ln[l][0] * M.ln[l][1] * M.ln[l][2];
       B->max_lds_cells[l] = std::max(B->max_lds_cells[l], cells);
@@ -174,7 +173,7 @@ int create(const wf_member* mem, int nmem, int nlev, Batch** out) {
   B->nred = red;
   B->nsum = sum;
 
-  rc = batch_mg_init(&B->lds);
+  rc = batch_mg_init();
   if (rc) {
     batch_free(B);
     return rc;
@@ -210,6 +209,21 @@ int create(const wf_member* mem, int nmem, int nlev, Batch** out) {
       return rc;
     }
     P.start = B->plan_mem[k];
+  }
+  std::vector<int4> items;
+  for (int l = 0; l < nlev; ++l) {
+    BatchRelax& P = B->relax[l];
+    batch_relax_plan(B->mem_host, nmem, l, P, items);
+    void* p = nullptr;
+    if (fail(hipMalloc(&p, sizeof(int4) * items.size()))) {
+      batch_free(B);
+      return rc;
+    }
+    P.item = (const int4*)p;
+    if (fail(hipMemcpy(p, items.data(), sizeof(int4) * items.size(), hipMemcpyHostToDevice))) {
+      batch_free(B);
+      return rc;
+    }
   }
   *out = B;
   return 0;

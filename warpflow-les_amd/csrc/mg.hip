@@ -20,6 +20,7 @@
 // reference could observe it.
 #include <algorithm>
 #include <type_traits>
+#include <vector>
 
 #include "batch.h"
 #include "mg_common.h"
@@ -1210,7 +1211,7 @@ relax_block_kernel(const T* __restrict__ pin, T* pout, const T* __restrict__ rhs
                    T c1, T c2, int ns, int rj, int rk, int tj, int tk) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int b = xcd_linear(blockIdx.x, gridDim.x);
-  relax_block_body<T, RI, PL, PART>(pin, pout, rhs, d, c0, c1, c2, ns, rj, rk,
+  relax_block_body<T, RI, PL, PART>(pin, pout, rhs, d, c0, c1, c2, ns, 2 * ns, rj, rk,
                                     Blk{b % tk, (b / tk) % tj, b / (tk * tj)},
                                     reinterpret_cast<T*>(smem_raw));
 }
@@ -1712,38 +1713,57 @@ batch_prolong8_kernel(BView V, Plan P, int lf, const float* phic, float* phif,
   });
 }
 
-// one fused full sweep pout = S(pin) on level l, tile shape per member
-__global__ void __launch_bounds__(256)
-batch_sweep_kernel(BView V, Plan P, int l, const float* pin, float* pout, const float* rhs,
-                   const int* active) {
-  mg_items<true>(P, V, active, [&](int q, const MemDev& M) {
-    const MgDev d = level_dev(M, l);
-    float c0, c1, c2;
-    level_coef(M, l, c0, c1, c2);
-    const int TJ = sweep_tj(d.n2), TK = sweep_tk(d.n2);
-    const int kt = (d.n2 + TK - 1) / TK, jt = (d.n1 + TJ - 1) / TJ;
-    const Blk B{q % kt, (q / kt) % jt, q / (kt * jt)};
-    const int64_t o = M.loff[l];
-    if (TK == 64)
-      sweep_body<float, 8, 64>(pin + o, pout + o, rhs + o, d, c0, c1, c2, BATCH_SWEEP_ICH, B);
-    else
-      sweep_body<float, 16, 32>(pin + o, pout + o, rhs + o, d, c0, c1, c2, BATCH_SWEEP_ICH, B);
-  });
+// Batched relaxation of level l: an item (member, block coordinates) per
+// workgroup, from the level's table (BatchRelax), so that nothing is searched
+// or divided before the loads.
+__device__ inline bool relax_item(const BView& V, const int4* item, const int* active, int l,
+                                  const MemDev*& M, MgDev& d, Blk& B) {
+  const int4 it = item[xcd_linear(blockIdx.x, gridDim.x)];
+  if (active && !active[it.x]) return false;  // uniform per workgroup
+  M = &V.mem[it.x];
+  d = level_dev(*M, l);
+  B = Blk{it.y, it.z, it.w};
+  return true;
 }
-
-// nsweeps RBGS sweeps of level l, one LDS-resident workgroup per member
-__global__ void __launch_bounds__(1024)
-batch_relax_lds_kernel(BView V, int l, float* phi, const float* rhs, int nsweeps,
-                       const int* active) {
+// ns sweeps by overlapping blocks (relax_block.h) of RI planes; levels of
+// fewer planes than that run one part block
+template <int RJK, bool SMALL>
+__global__ void __launch_bounds__(RJK * RJK)
+    __attribute__((amdgpu_waves_per_eu(RJK * RJK / 256, 5)))
+batch_relax_block_kernel(BView V, const int4* item, int l, int ns, int h, const float* pin,
+                         float* pout, const float* rhs, const int* active) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  const int m = blockIdx.x;
-  if (active && !active[m]) return;  // uniform per workgroup
-  const MemDev& M = V.mem[m];
-  const MgDev d = level_dev(M, l);
-  float c0, c1, c2;
-  level_coef(M, l, c0, c1, c2);
-  relax_lds_body<float, true>(phi + M.loff[l], rhs + M.loff[l], d, c0, c1, c2, nsweeps,
-                              reinterpret_cast<float*>(smem_raw));
+  float* const sm = reinterpret_cast<float*>(smem_raw);
+  const MemDev* M;
+  MgDev d;
+  Blk B;
+  if (!relax_item(V, item, active, l, M, d, B)) return;
+  constexpr int PL = RJK == 16 ? 320 : 1152;
+  const float c0 = M->lc[l][0], c1 = M->lc[l][1], c2 = M->lc[l][2];
+  const int rj = min(d.n1, RJK), rk = min(d.n2, RJK);
+  const int64_t o = M->loff[l];
+  const float* const in = pin ? pin + o : nullptr;
+  if (d.n0 >= 16)
+    relax_block_body<float, 16, PL, false>(in, pout + o, rhs + o, d, c0, c1, c2, ns, h, rj, rk, B,
+                                           sm);
+  else if (SMALL && d.n0 <= 8)
+    relax_block_body<float, 8, PL, true>(in, pout + o, rhs + o, d, c0, c1, c2, ns, h, rj, rk, B,
+                                         sm);
+  else
+    relax_block_body<float, 16, PL, true>(in, pout + o, rhs + o, d, c0, c1, c2, ns, h, rj, rk, B,
+                                          sm);
+}
+// two sweeps in one pass over 16 x 32 tiles and chunks of ich planes
+__global__ void __launch_bounds__(256, 3)
+batch_sweep2_kernel(BView V, const int4* item, int l, int ich, const float* pin, float* pout,
+                    const float* rhs, const int* active) {
+  const MemDev* M;
+  MgDev d;
+  Blk B;
+  if (!relax_item(V, item, active, l, M, d, B)) return;
+  const int64_t o = M->loff[l];
+  sweep2_body<float, 16, 32>(pin ? pin + o : nullptr, pout + o, rhs + o, d, M->lc[l][0],
+                             M->lc[l][1], M->lc[l][2], ich, B);
 }
 
 // phi = M rhs on the coarsest level l, a workgroup per member and COP_ROWS rows
@@ -1760,52 +1780,130 @@ batch_coarse_rows_kernel(BView V, Plan P, int l, const float* cop, float* phi, c
                              blockIdx.x - P.start[m], reinterpret_cast<float*>(smem_raw));
 }
 
-int batch_lds_bytes() {
-  int dev = 0, v = 65536;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
-    v = 65536;
-  return v;
-}
-
-// Dynamic-LDS limits of the batched single-workgroup kernels, set once when a
-// batch is created (never inside a captured step).
-int batch_mg_init(int* lds_out) {
-  const int lds = batch_lds_bytes();
-  WF_TRY(hipFuncSetAttribute((const void*)batch_relax_lds_kernel,
-                             hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+// Dynamic-LDS limits of the batched kernels, set once when a batch is
+// created (never inside a captured step).
+int batch_mg_init() {
+  WF_TRY(hipFuncSetAttribute((const void*)batch_relax_block_kernel<32, false>,
+                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                             16 * 1152 * (int)sizeof(float)));
   WF_TRY(hipFuncSetAttribute((const void*)batch_coarse_rows_kernel,
                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)COP_LDS<float>));
-  *lds_out = lds;
   return 0;
 }
 
-// One batched V-cycle of the FP32 levels (vcycle_any's order).
-int batch_vcycle(const Batch& B, float* const* phi, float* const* rhs, float* const* tmp,
+// The relaxation of level l of every member: the tiles and the cheapest of the
+// launches below, costs as in BLOCK_SHAPES (us for the first 256 blocks, ns for
+// each further one; two-sweep launches: us per plane iteration of a round of
+// three workgroups per CU).
+void batch_relax_plan(const MemDev* mem, int nmem, int l, BatchRelax& P,
+                      std::vector<int4>& items) {
+  struct Shape {
+    int rjk, ns;
+    double base, more;
+  };
+  static const Shape shapes[] = {{16, 3, 6.75, 8.0}, {16, 2, 5.85, 7.5}, {32, 3, 12.9, 40.0},
+                                 {32, 2, 11.7, 35.0}};
+  auto blocks = [&](int m, int rjk, int h, int* t) {
+    const int* n = mem[m].ln[l];
+    t[0] = relax_block_tiles(n[0], n[0] <= 8 && rjk == 16 ? 8 : 16, h);
+    t[1] = relax_block_tiles(n[1], std::min(n[1], rjk), h);
+    t[2] = relax_block_tiles(n[2], std::min(n[2], rjk), h);
+    return (int64_t)t[0] * t[1] * t[2];
+  };
+  int t[3];
+  double best = 0;
+  P.single = true;
+  for (int m = 0; m < nmem; ++m)
+    for (int a = 0; a < 3; ++a) P.single = P.single && mem[m].ln[l][a] <= 16;
+  for (const Shape& S : shapes) {
+    int64_t nb = 0;
+    for (int m = 0; m < nmem; ++m) nb += blocks(m, S.rjk, 2 * S.ns, t);
+    // per six sweeps
+    const double cost = 6 / S.ns * (S.base + 1e-3 * S.more * std::max(0.0, (double)nb - 256.0));
+    if (P.ns == 0 || cost < best) {
+      best = cost;
+      P.rjk = S.rjk;
+      P.ns = S.ns;
+    }
+    if (P.single) break;
+  }
+  // two-sweep launches: the chunk of least total plane iterations
+  int nmax = 0;
+  for (int m = 0; m < nmem; ++m) nmax = std::max(nmax, mem[m].ln[l][0]);
+  const double slots = 3 * 256;
+  for (int ich = 8; ich <= 64 && !P.single; ich += 4) {
+    int64_t w = 0;
+    for (int m = 0; m < nmem; ++m) {
+      const int* n = mem[m].ln[l];
+      // the kernel's plane offsets within a chunk stay below 2^30
+      if ((int64_t)(ich + 9) * (n[1] + 2) * (n[2] + 2) * 4 >= ((int64_t)1 << 30)) w = INT32_MAX;
+      w += (int64_t)div_up(n[0], ich) * div_up(n[1], 16) * div_up(n[2], 32);
+    }
+    const double cost = 3 * (2.0 + 1.36 * std::max(1.0, w / slots) * (std::min(ich, nmax) + 9));
+    if (cost < best) {
+      best = cost;
+      P.ich = ich;
+    }
+  }
+  if (P.ich) P.ns = 2;
+  items.clear();
+  for (int m = 0; m < nmem; ++m) {
+    const int* n = mem[m].ln[l];
+    if (P.ich) {
+      t[0] = div_up(n[0], P.ich);
+      t[1] = div_up(n[1], 16);
+      t[2] = div_up(n[2], 32);
+    } else {
+      blocks(m, P.rjk, 2 * P.ns, t);
+    }
+    for (int z = 0; z < t[0]; ++z)
+      for (int y = 0; y < t[1]; ++y)
+        for (int x = 0; x < t[2]; ++x)
+          items.push_back(int4{m, x, y, z});
+  }
+  P.total = (int)items.size();
+}
+
+// One batched V-cycle of the FP32 levels (vcycle_any's order); zero0: level 0's
+// iterate is taken as zero without being read (its first relaxation has sweeps).
+int batch_vcycle(const Batch& B, float* const* phi_, float* const* rhs, float* const* tmp_,
                  const float* cop, int npre, int npost, int ncoarse, const int* active,
-                 hipStream_t s) {
+                 hipStream_t s, bool zero0) {
   const int nlev = B.nlev;
   const BView V = B.view();
-  const int lds = B.lds;
-  auto relax = [&](int l, int n) -> int {
+  // a level whose relaxation takes an odd number of launches leaves its
+  // iterate in tmp: the two swap, as in vcycle_any
+  float *phi[BATCH_MAX_LEVELS], *tmp[BATCH_MAX_LEVELS];
+  for (int l = 0; l < nlev; ++l) {
+    phi[l] = phi_[l];
+    tmp[l] = tmp_[l];
+  }
+  auto relax = [&](int l, int n, bool zero) -> int {
     if (n <= 0) return 0;
-    const size_t cells = (size_t)B.max_lds_cells[l];
-    if (cells <= 4096 && 2 * cells * sizeof(float) <= (size_t)lds) {
-      hipLaunchKernelGGL(batch_relax_lds_kernel, dim3(B.nmem), dim3(1024),
-                         2 * cells * sizeof(float), s, V, l, phi[l], (const float*)rhs[l], n,
-                         active);
+    const BatchRelax& P = B.relax[l];
+    if (n % 2 && B.max_lds_cells[l] > 4096) return WF_EINVAL;
+    const float* in = zero ? nullptr : phi[l];
+    const int launches = P.single ? 1 : div_up(n, P.ns);
+    for (int q = 0; q < launches; ++q) {
+      const int ns = n / launches + (q < n % launches);
+      float* const out = P.single ? phi[l] : tmp[l];
+      if (P.ich && ns == 2) {
+        hipLaunchKernelGGL(batch_sweep2_kernel, dim3(P.total), dim3(256), 0, s, V, P.item, l,
+                           P.ich, in, out, (const float*)rhs[l], active);
+      } else if (P.ich) {
+        return WF_EINVAL;  // (levels this large take even numbers of sweeps)
+      } else if (P.rjk == 16) {
+        hipLaunchKernelGGL((batch_relax_block_kernel<16, true>), dim3(P.total), dim3(256),
+                           16 * 320 * sizeof(float), s, V, P.item, l, ns, 2 * P.ns, in, out,
+                           (const float*)rhs[l], active);
+      } else {
+        hipLaunchKernelGGL((batch_relax_block_kernel<32, false>), dim3(P.total), dim3(1024),
+                           16 * 1152 * sizeof(float), s, V, P.item, l, ns, 2 * P.ns, in, out,
+                           (const float*)rhs[l], active);
+      }
       WF_LAUNCHED();
-      return 0;
-    }
-    if (n % 2) return WF_EINVAL;  // the fused form runs sweeps in pairs
-    const Plan& P = B.plan[PK_SWEEP0 + l];
-    for (int q = 0; q < n; q += 2) {
-      hipLaunchKernelGGL(batch_sweep_kernel, dim3(P.grid), dim3(256), 0, s, V, P, l,
-                         (const float*)phi[l], tmp[l], (const float*)rhs[l], active);
-      WF_LAUNCHED();
-      hipLaunchKernelGGL(batch_sweep_kernel, dim3(P.grid), dim3(256), 0, s, V, P, l,
-                         (const float*)tmp[l], phi[l], (const float*)rhs[l], active);
-      WF_LAUNCHED();
+      if (!P.single) std::swap(phi[l], tmp[l]);
+      in = phi[l];
     }
     return 0;
   };
@@ -1824,7 +1922,7 @@ int batch_vcycle(const Batch& B, float* const* phi, float* const* rhs, float* co
       WF_LAUNCHED();
       continue;
     }
-    const int r = relax(l, l < nlev - 1 ? npre : ncoarse);
+    const int r = relax(l, l < nlev - 1 ? npre : ncoarse, l == 0 && zero0);
     if (r) return r;
   }
   for (int l = nlev - 2; l >= 0; --l) {
@@ -1842,9 +1940,13 @@ int batch_vcycle(const Batch& B, float* const* phi, float* const* rhs, float* co
                          (const float*)phi[l + 1], phi[l], active);
     }
     WF_LAUNCHED();
-    const int r = relax(l, npost);
+    const int r = relax(l, npost, false);
     if (r) return r;
   }
+  for (int l = 0; l < nlev; ++l)
+    if (phi[l] != phi_[l])
+      WF_TRY(hipMemcpyAsync(phi_[l], phi[l], (size_t)B.level_elems[l] * sizeof(float),
+                            hipMemcpyDeviceToDevice, s));
   return 0;
 }
 

@@ -539,10 +539,14 @@ int batch_mg_mixed(const Batch& B, float* const* phi, float* const* rhs, float* 
       WF_LAUNCHED();
     }
     defect_formed = false;
-    const int lb = (int)std::min<int64_t>((B.level_elems[0] + 255) / 256, 8192);
-    hipLaunchKernelGGL(batch_fillf_kernel, dim3(lb), dim3(256), 0, s, phi[0], B.level_elems[0]);
-    WF_LAUNCHED();
-    const int r = batch_vcycle(B, phi, rhs, tmp, cop, npre, npost, ncoarse, active, s);
+    // phi0 = 0: taken unread by the first relaxation of level 0, if there is one
+    const bool zero0 = (B.nlev > 1 ? npre : ncoarse) > 0;
+    if (!zero0) {
+      const int lb = (int)std::min<int64_t>((B.level_elems[0] + 255) / 256, 8192);
+      hipLaunchKernelGGL(batch_fillf_kernel, dim3(lb), dim3(256), 0, s, phi[0], B.level_elems[0]);
+      WF_LAUNCHED();
+    }
+    const int r = batch_vcycle(B, phi, rhs, tmp, cop, npre, npost, ncoarse, active, s, zero0);
     if (r) return r;
     if (c == 0 && ncycles > 1) {
       // pp = 0 + e and the second cycle's defect in one pass

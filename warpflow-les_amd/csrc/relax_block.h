@@ -39,17 +39,18 @@ __host__ __device__ inline int relax_block_tiles(int n, int r, int h) {
   return r >= n ? 1 : 1 + (n - r + r - 2 * h - 1) / (r - 2 * h);
 }
 
-// PART: the level has fewer than RI planes (one block along i); the planes past
-// it stay zero under a zero reciprocal diagonal, kept per cell.
+// h: the halo the tiles were cut for, at least 2 ns.  PART: the level may have
+// fewer than RI planes (one block along i then); the planes past it stay zero
+// under a zero reciprocal diagonal, kept per cell.
 template <class T, int RI, int PL, bool PART>
 __device__ inline void relax_block_body(const T* __restrict__ pin, T* __restrict__ pout,
                                         const T* __restrict__ rhs, const MgDev& d, T c0, T c1,
-                                        T c2, int ns, int rj, int rk, Blk B, T* __restrict__ sm) {
+                                        T c2, int ns, int h, int rj, int rk, Blk B,
+                                        T* __restrict__ sm) {
   constexpr int NH = RI / 2;  // cells per colour and thread
   static_assert(RI % 2 == 0 && PL % 32 == 0, "whole pairs, whole bank rows");
   const int tid = threadIdx.x;
   const int n0 = d.n0, n1 = d.n1, n2 = d.n2;
-  const int h = 2 * ns;
   // block origin and the tile it writes, along one axis
   auto axis = [&](int b, int n, int r, int& o, int& lo, int& hi) {
     const int st = r - 2 * h;
