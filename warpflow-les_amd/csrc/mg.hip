@@ -1371,8 +1371,8 @@ relax_lds2_kernel(T* __restrict__ phi, const T* __restrict__ rhs, MgDev d, T c0,
 // sweeps in LDS from phi = 0 with rhs = e_col, the relax_lds_kernel
 // arithmetic; M is column-major (M[col * ncell + row]).
 template <class T>
-__device__ inline void coarse_op_build_body(T* __restrict__ M, const MgDev& d, T c0, T c1, T c2,
-                                            int nsweeps, int col, T* sp) {
+__device__ inline void coarse_op_sweeps(const MgDev& d, T c0, T c1, T c2, int nsweeps, int col,
+                                        T* sp) {
   const int n0 = d.n0, n1 = d.n1, n2 = d.n2;
   const int ncell = n0 * n1 * n2;
   const int nt = blockDim.x, tid = threadIdx.x;
@@ -1401,13 +1401,15 @@ __device__ inline void coarse_op_build_body(T* __restrict__ M, const MgDev& d, T
       __syncthreads();
     }
   }
-  for (int l = tid; l < ncell; l += nt) M[(size_t)col * ncell + l] = sp[l];
 }
 template <class T>
 __global__ void __launch_bounds__(256)
 coarse_op_build_kernel(T* __restrict__ M, MgDev d, T c0, T c1, T c2, int nsweeps) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  coarse_op_build_body<T>(M, d, c0, c1, c2, nsweeps, blockIdx.x, reinterpret_cast<T*>(smem_raw));
+  T* const sp = reinterpret_cast<T*>(smem_raw);
+  coarse_op_sweeps<T>(d, c0, c1, c2, nsweeps, blockIdx.x, sp);
+  const int ncell = d.n0 * d.n1 * d.n2;
+  for (int l = threadIdx.x; l < ncell; l += blockDim.x) M[(size_t)blockIdx.x * ncell + l] = sp[l];
 }
 
 // phi = M rhs on the real cells of a small level, plus face-ring images.
@@ -1599,6 +1601,153 @@ coarse_op_fold_kernel(const T* __restrict__ part, int nchunk, T* __restrict__ ph
   const int64_t x = mg_at(d, i, j, k);
   phi[x] = acc;
   ring_images(phi, d, i, j, k, x, acc);
+}
+
+// FP64 operators of more than COARSE_OP_SERIAL_MAX_CELLS cells and even extents
+// use the level's reflections.  Reflecting two axes at once keeps every cell's
+// colour when the extents are even, so the sweeps commute with the group of the
+// four elements below, and M splits into one block per character of it: with
+// the representatives i < n0/2, j < n1/2 (a quarter of the cells),
+//   b_c[q] = sum_e X[c][e] rhs[e q],    y_c = M_c b_c,
+//   phi[e p] = 1/4 sum_c X[c][e] y_c[p],
+//   M_c(p, q) = sum_e X[c][e] M(e p, q).
+// The last half-sweep of the sweeps M stands for forms the even cells from the
+// odd ones, so M_c keeps its odd rows only and one half-sweep finishes: N^2/8
+// entries instead of N^2, from a quarter of the columns.  20^3: 64 MB for 512,
+// apply 20 us for 116 (the 512 MB at 5.3 TB/s), build 19 ms for 71; the error
+// against 80-bit sweeps is that of the sweeps in FP64 (1.1-2.4e-15 at 20^3).
+constexpr int COP_SYM_ROWS = 256, COP_SYM_CHUNKS = 32;
+__device__ inline double cop_sign(int c, int e) {  // X[c][e]
+  return (c == 0 || e == 0 || c == e) ? 1.0 : -1.0;
+}
+// cell e q: e = 1 reflects axes 0 and 1, 2 axes 0 and 2, 3 axes 1 and 2
+__device__ inline void cop_orbit(const MgDev& d, int e, int i, int j, int k, int& a, int& b,
+                                 int& c) {
+  a = e == 1 || e == 2 ? d.n0 - 1 - i : i;
+  b = e == 1 || e == 3 ? d.n1 - 1 - j : j;
+  c = e >= 2 ? d.n2 - 1 - k : k;
+}
+// representative q (all of them), and odd representative r (half of them)
+__device__ inline void cop_rep(const MgDev& d, int q, int& i, int& j, int& k) {
+  const int h1 = d.n1 / 2;
+  k = q % d.n2;
+  j = q / d.n2 % h1;
+  i = q / d.n2 / h1;
+}
+__device__ inline void cop_odd_rep(const MgDev& d, int r, int& i, int& j, int& k) {
+  const int h1 = d.n1 / 2, h2 = d.n2 / 2;
+  j = r / h2 % h1;
+  i = r / h2 / h1;
+  k = 2 * (r % h2) + ((i + j + 1) & 1);
+}
+// Column q of every M_c: the sweeps on the unit rhs of representative q, in LDS.
+__global__ void __launch_bounds__(256)
+coarse_op_sym_build_kernel(double* __restrict__ M, MgDev d, double c0, double c1, double c2,
+                           int nsweeps, double* __restrict__ any) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  double* const sp = reinterpret_cast<double*>(smem_raw);
+  if (blockIdx.x == 0 && threadIdx.x == 0) *any = nsweeps > 0 ? 1.0 : 0.0;
+  int i, j, k;
+  cop_rep(d, blockIdx.x, i, j, k);
+  coarse_op_sweeps(d, c0, c1, c2, nsweeps, (i * d.n1 + j) * d.n2 + k, sp);
+  const int nq = d.n0 * d.n1 * d.n2 / 4, nr = nq / 2;
+  for (int r = threadIdx.x; r < nr; r += blockDim.x) {
+    cop_odd_rep(d, r, i, j, k);
+    double v[4];
+    for (int e = 0; e < 4; ++e) {
+      int a, b, c;
+      cop_orbit(d, e, i, j, k, a, b, c);
+      v[e] = sp[(a * d.n1 + b) * d.n2 + c];
+    }
+    for (int c = 0; c < 4; ++c) {
+      double m = 0.0;
+      for (int e = 0; e < 4; ++e) m += cop_sign(c, e) * v[e];
+      M[((size_t)c * nq + blockIdx.x) * nr + r] = m;
+    }
+  }
+}
+// part[c][y][row] = columns [y*clen, (y+1)*clen) of y_c; grid (row blocks,
+// column chunks, c)
+__global__ void __launch_bounds__(COP_SYM_ROWS)
+coarse_op_sym_split_kernel(const double* __restrict__ M, const double* __restrict__ rhs, MgDev d,
+                           int clen, double* __restrict__ part) {
+  __shared__ double b[COP_SPLIT_MAX_CLEN];
+  const int nq = d.n0 * d.n1 * d.n2 / 4, nr = nq / 2;
+  const int c = blockIdx.z, q0 = blockIdx.y * clen;
+  const int nc = min(clen, nq - q0);
+  for (int l = threadIdx.x; l < nc; l += COP_SYM_ROWS) {
+    int i, j, k, x, y, z;
+    cop_rep(d, q0 + l, i, j, k);
+    double v = 0.0;
+    for (int e = 0; e < 4; ++e) {
+      cop_orbit(d, e, i, j, k, x, y, z);
+      v += cop_sign(c, e) * rhs[mg_at(d, x, y, z)];
+    }
+    b[l] = v;
+  }
+  __syncthreads();
+  const int row = blockIdx.x * COP_SYM_ROWS + threadIdx.x;
+  if (row >= nr) return;
+  const double* __restrict__ m0 = M + ((size_t)c * nq + q0) * nr + row;
+  double acc = 0.0;
+  int l = 0;
+  for (; l + 16 <= nc; l += 16) {
+    double m[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) m[u] = m0[(size_t)(l + u) * nr];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) acc = cop_fma(m[u], b[l + u], acc);
+  }
+  for (; l < nc; ++l) acc = cop_fma(m0[(size_t)l * nr], b[l], acc);
+  part[((size_t)c * gridDim.y + blockIdx.y) * nr + row] = acc;
+}
+// y_c = its chunk sums in order, then the odd cells of phi (with their ring
+// images): 64 rows x 4 characters, then 64 rows x 4 orbit cells
+__global__ void __launch_bounds__(256)
+coarse_op_sym_fold_kernel(const double* __restrict__ part, int nchunk, double* __restrict__ phi,
+                          MgDev d) {
+  __shared__ double y[4][64];
+  const int nr = d.n0 * d.n1 * d.n2 / 8;
+  const int l = threadIdx.x & 63, c = threadIdx.x >> 6;
+  const int row = blockIdx.x * 64 + l;
+  if (row < nr) {
+    const double* p = part + (size_t)c * nchunk * nr + row;
+    double acc = 0.0;
+    for (int t = 0; t < nchunk; t += COP_SYM_CHUNKS) {
+      double v[COP_SYM_CHUNKS];
+#pragma unroll
+      for (int u = 0; u < COP_SYM_CHUNKS; ++u) v[u] = t + u < nchunk ? p[(size_t)(t + u) * nr] : 0.0;
+#pragma unroll
+      for (int u = 0; u < COP_SYM_CHUNKS; ++u) acc += v[u];
+    }
+    y[c][l] = acc;
+  }
+  __syncthreads();
+  if (row >= nr) return;
+  int i, j, k, a, b, z;
+  cop_odd_rep(d, row, i, j, k);
+  const int e = c;
+  double v = 0.0;
+  for (int q = 0; q < 4; ++q) v += cop_sign(q, e) * y[q][l];
+  v *= 0.25;
+  cop_orbit(d, e, i, j, k, a, b, z);
+  const int64_t x = mg_at(d, a, b, z);
+  phi[x] = v;
+  ring_images(phi, d, a, b, z, x, v);
+}
+
+// The even cells from the odd ones, a half-sweep of colour 1 (rbgs_kernel's
+// update); any: 0 where M stands for no sweeps at all, whose result is zero.
+__global__ void __launch_bounds__(256)
+coarse_op_sym_even_kernel(double* __restrict__ phi, const double* __restrict__ rhs, MgDev d,
+                          double c0, double c1, double c2, const double* __restrict__ any) {
+  int i, j, k;
+  if (!colour_cell(d, 1, i, j, k)) return;
+  const int64_t x = mg_at(d, i, j, k);
+  const Coef<double> c = mg_coef(d, i, j, k, c0, c1, c2);
+  const double v = *any != 0.0 ? (rhs[x] - nb_sum(phi, x, d, c)) * (1.0 / c.ap) : 0.0;
+  phi[x] = v;
+  ring_images(phi, d, i, j, k, x, v);
 }
 
 __global__ void __launch_bounds__(256)
@@ -2475,7 +2624,19 @@ inline int cop_split_chunks(int ncell) {
   while (div_up(ncell, nch) > COP_SPLIT_MAX_CLEN) ++nch;
   return nch;
 }
-inline size_t cop_elems(size_t ncell) {
+// the form by characters of the reflections (coarse_op_sym_*)
+inline bool cop_sym(const wf_mg_level& L) {
+  return L.prec == 8 && L.n0 % 2 == 0 && L.n1 % 2 == 0 && L.n2 % 2 == 0 &&
+         (int64_t)L.n0 * L.n1 * L.n2 > COARSE_OP_SERIAL_MAX_CELLS;
+}
+inline int cop_sym_chunks(int ncell) {
+  const int nq = ncell / 4;
+  return std::max(COP_SYM_CHUNKS, div_up(nq, COP_SPLIT_MAX_CLEN));
+}
+inline size_t cop_elems(const wf_mg_level& L) {
+  const size_t ncell = (size_t)L.n0 * L.n1 * L.n2;
+  if (cop_sym(L))  // the blocks, the chunk sums, and whether there were sweeps
+    return ncell * ncell / 8 + (size_t)cop_sym_chunks((int)ncell) * ncell / 2 + 1;
   size_t e = ncell * ncell;
   if (ncell > (size_t)COARSE_OP_SERIAL_MAX_CELLS) e += (size_t)cop_split_chunks((int)ncell) * ncell;
   return e;
@@ -2486,6 +2647,28 @@ int coarse_op_apply_t(const wf_mg_level& L, hipStream_t s) {
   const MgDev d = mg_dev(L);
   const int ncell = d.n0 * d.n1 * d.n2;
   if (ncell > COARSE_OP_MAX_CELLS) return WF_EINVAL;
+  if constexpr (sizeof(T) == 8) {
+    if (cop_sym(L)) {
+      const int nq = ncell / 4, nr = ncell / 8;
+      const int nch = cop_sym_chunks(ncell), clen = div_up(nq, nch);
+      double* part = (double*)L.cop + (size_t)ncell * ncell / 8;
+      hipLaunchKernelGGL(coarse_op_sym_split_kernel,
+                         dim3((unsigned)div_up(nr, COP_SYM_ROWS), (unsigned)nch, 4),
+                         dim3(COP_SYM_ROWS), 0, s, (const double*)L.cop, (const double*)L.rhs, d,
+                         clen, part);
+      WF_LAUNCHED();
+      hipLaunchKernelGGL(coarse_op_sym_fold_kernel, dim3((unsigned)div_up(nr, 64)), dim3(256), 0,
+                         s, (const double*)part, nch, (double*)L.phi, d);
+      WF_LAUNCHED();
+      double c0, c1, c2;
+      inv_h2(L, c0, c1, c2);
+      hipLaunchKernelGGL(coarse_op_sym_even_kernel, cell_grid(d.n0, d.n1, d.n2 / 2), dim3(64, 4),
+                         0, s, (double*)L.phi, (const double*)L.rhs, d, c0, c1, c2,
+                         (const double*)L.cop + cop_elems(L) - 1);
+      WF_LAUNCHED();
+      return 0;
+    }
+  }
   if (ncell > COARSE_OP_SERIAL_MAX_CELLS) {
     const int nch = cop_split_chunks(ncell), clen = div_up(ncell, nch);
     T* part = (T*)L.cop + (size_t)ncell * ncell;
@@ -2528,6 +2711,18 @@ int coarse_op_build_t(const wf_mg_level& L, int nsweeps, void* op, hipStream_t s
   }
   T c0, c1, c2;
   inv_h2(L, c0, c1, c2);
+  if constexpr (sizeof(T) == 8) {
+    if (cop_sym(L)) {
+      static const hipError_t set =
+          hipFuncSetAttribute((const void*)coarse_op_sym_build_kernel,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, max_lds());
+      WF_TRY(set);
+      hipLaunchKernelGGL(coarse_op_sym_build_kernel, dim3(ncell / 4), dim3(256), bytes, s,
+                         (double*)op, d, c0, c1, c2, nsweeps, (double*)op + cop_elems(L) - 1);
+      WF_LAUNCHED();
+      return 0;
+    }
+  }
   hipLaunchKernelGGL(coarse_op_build_kernel<T>, dim3(ncell), dim3(256), bytes, s, (T*)op, d, c0,
                      c1, c2, nsweeps);
   WF_LAUNCHED();
@@ -2654,7 +2849,7 @@ int wf_mg_coarse_op_bytes(const wf_mg_level* L, size_t* bytes) {
   const size_t ncell = (size_t)L->n0 * L->n1 * L->n2;
   if (ncell > (size_t)COARSE_OP_MAX_CELLS || ncell * L->prec > (size_t)max_lds())
     return WF_EINVAL;
-  *bytes = cop_elems(ncell) * (size_t)L->prec;
+  *bytes = cop_elems(*L) * (size_t)L->prec;
   return 0;
 }
 
