@@ -42,6 +42,7 @@ struct Plan {
   const int* start;
   int total;
   int grid;  // workgroups launched (<= total)
+  int ich;   // i-planes per item of the tile streams (PK_RED, PK_CD*, PK_WALE)
 };
 
 struct BView {
@@ -72,10 +73,9 @@ __device__ inline Blk cells_blk(int q, int d1, int d2) {
   return Blk{q % nx, (q / nx) % ny, q / (nx * ny)};
 }
 
-// Reduction items: 64 x 4 (k, j) tiles x i-chunks of RED_ICH planes.
-constexpr int BATCH_RED_ICH = 8;
-__host__ __device__ inline int red_blocks(int d0, int d1, int d2) {
-  return ((d2 + 63) / 64) * ((d1 + 3) / 4) * ((d0 + BATCH_RED_ICH - 1) / BATCH_RED_ICH);
+// Reduction items: 64 x 4 (k, j) tiles x i-chunks of ich planes.
+__host__ __device__ inline int red_blocks(int d0, int d1, int d2, int ich) {
+  return ((d2 + 63) / 64) * ((d1 + 3) / 4) * ((d0 + ich - 1) / ich);
 }
 
 // Work-item counts per member for each kind of batched launch.
@@ -89,7 +89,7 @@ enum PlanKind : int {
   PK_BC0,           // ghost-fill lines of the x, y, z axis launches
   PK_BC1,
   PK_BC2,
-  PK_WALE,          // WALE tiles (8 x 32 (j, k) x BATCH_CD_ICH planes) over the real cells;
+  PK_WALE,          // WALE tiles (8 x 32 (j, k) x ich planes) over the real cells;
                     // also the three-component conv+diff passes
   PK_CDE,           // u's edge planes 0 and ni-2: 8 x 32 (j, k) tiles x 2
   PK_XG,            // w's cross-ghost cells of each real plane, 256 per item
@@ -130,9 +130,8 @@ struct Batch {
 };
 
 // Convdiff tiles (8 x 32 (j, k) tiles x i-chunks): shared with convdiff.hip.
-constexpr int BATCH_CD_ICH = 16;
-__host__ __device__ inline int cd_tiles(int d0, int d1, int d2) {
-  return ((d2 + 31) / 32) * ((d1 + 7) / 8) * ((d0 + BATCH_CD_ICH - 1) / BATCH_CD_ICH);
+__host__ __device__ inline int cd_tiles(int d0, int d1, int d2, int ich) {
+  return ((d2 + 31) / 32) * ((d1 + 7) / 8) * ((d0 + ich - 1) / ich);
 }
 // Operator box of component c over n0 x n1 x n2 cells (solver.py:99-110).
 __host__ __device__ inline void op_dims(int c, int n0, int n1, int n2, int& d0, int& d1,

@@ -47,7 +47,7 @@ constexpr int64_t ALIGN = 32;  // elements: member arrays start on 256-byte (FP6
 
 int64_t align_up(int64_t x) { return (x + ALIGN - 1) / ALIGN * ALIGN; }
 
-int member_count(int kind, const MemDev& M) {
+int member_count(int kind, const MemDev& M, int ich) {
   const int n0 = M.g.ni, n1 = M.g.nj, n2 = M.g.nk;
   switch (kind) {
     case PK_CELLS:
@@ -55,20 +55,20 @@ int member_count(int kind, const MemDev& M) {
     case PK_RING:
       return cells_blocks(n0 + 2, n1 + 2, n2 + 2);
     case PK_RED:
-      return red_blocks(n0, n1, n2);
+      return red_blocks(n0, n1, n2, ich);
     case PK_CD0:
     case PK_CD1:
     case PK_CD2: {
       int d0, d1, d2;
       op_dims(kind - PK_CD0, n0, n1, n2, d0, d1, d2);
-      return cd_tiles(d0, d1, d2);
+      return cd_tiles(d0, d1, d2, ich);
     }
     case PK_BC0:
     case PK_BC1:
     case PK_BC2:
       return bc_blocks(kind - PK_BC0, n0, n1, n2);
     case PK_WALE:
-      return cd_tiles(n0, n1, n2);
+      return cd_tiles(n0, n1, n2, ich);
     case PK_CDE:
       return ((n2 + 31) / 32) * ((n1 + 7) / 8) * (n0 - 1 > 1 ? 2 : (n0 - 1 > 0 ? 1 : 0));
     case PK_XG:
@@ -162,10 +162,25 @@ int create(const wf_member* mem, int nmem, int nlev, Batch** out) {
     } else {
       M.coff = -1;
     }
-    M.red0 = red;
-    red += red_blocks(a.n0, a.n1, a.n2);
     M.sum0 = sum;
     sum += cells_blocks(a.n0, a.n1, a.n2);
+  }
+  // i-planes per item of the streams, as the single-domain launches choose
+  // them: the momentum passes two workgroups per CU, the projection four
+  int nmax = 0;
+  for (int m = 0; m < nmem; ++m) nmax = std::max(nmax, mem[m].n0);
+  auto chunk = [&](int kind, const ChunkCost& C) {
+    return pick_chunk(nmax, C, INT32_MAX, [&](int ich) {
+      int64_t w = 0;
+      for (int m = 0; m < nmem; ++m) w += member_count(kind, B->mem_host[m], ich);
+      return w;
+    });
+  };
+  const int cd_ich = chunk(PK_WALE, ChunkCost{2, {2.05, 3.0}});
+  const int red_ich = chunk(PK_RED, ChunkCost{4, {1.1, 1.75, 2.75, 3.7}});
+  for (int m = 0; m < nmem; ++m) {
+    B->mem_host[m].red0 = red;
+    red += red_blocks(mem[m].n0, mem[m].n1, mem[m].n2, red_ich);
   }
   B->field_elems = foff;
   for (int l = 0; l < nlev; ++l) B->level_elems[l] = loff[l];
@@ -197,8 +212,10 @@ int create(const wf_member* mem, int nmem, int nlev, Batch** out) {
   std::vector<int> start(nmem + 1);
   for (int k = 0; k < PK_COUNT; ++k) {
     start[0] = 0;
-    for (int m = 0; m < nmem; ++m) start[m + 1] = start[m] + member_count(k, B->mem_host[m]);
     Plan& P = B->plan[k];
+    P.ich = k == PK_RED ? red_ich : cd_ich;
+    for (int m = 0; m < nmem; ++m)
+      start[m + 1] = start[m] + member_count(k, B->mem_host[m], P.ich);
     P.total = start[nmem];
     // a persistent grid: at most 8 workgroups per CU, the most a CU holds
     P.grid = std::max(1, std::min(P.total, 8 * ncu));

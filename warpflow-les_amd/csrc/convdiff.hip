@@ -1240,7 +1240,7 @@ save_cross_ghosts_kernel(const double* __restrict__ w, double* __restrict__ wpre
 }
 
 // Ensemble form: a persistent grid over the (member, tile, chunk) items of
-// component C, chunks of BATCH_CD_ICH planes.
+// component C, chunks of P.ich planes.
 template <int C, bool SAVE>
 __global__ void __launch_bounds__(256)
 batch_convdiff_kernel(BView V, Plan P, const double* __restrict__ u,
@@ -1265,7 +1265,7 @@ batch_convdiff_kernel(BView V, Plan P, const double* __restrict__ u,
     K.ir12z = 1.0 / (12.0 * M.dz * M.dz);
     K.dta = M.dt * alpha;
     convdiff_body<C, SAVE>(u + M.off, v + M.off, w + M.off, SAVE ? nullptr : coo + M.off,
-                           vis + M.off, cstar + M.off, g, b, BATCH_CD_ICH, q % kt,
+                           vis + M.off, cstar + M.off, g, b, P.ich, q % kt,
                            (q / kt) % jt, q / (kt * jt), K, SAVE ? coo_save + M.off : nullptr);
     __syncthreads();  // LDS of this item is free for the next
   }
@@ -1286,7 +1286,7 @@ __device__ inline Coefs member_coefs(const MemDev& M, double alpha) {
 
 // Ensemble forms of the three-component passes: a persistent grid over the
 // (member, tile, chunk) items of PK_WALE (8 x 32 tiles over the real cells,
-// chunks of BATCH_CD_ICH planes), two workgroups per CU (the item loop's
+// chunks of P.ich planes), two workgroups per CU (the item loop's
 // member lookup pushes the first stage's form past 168 VGPRs as well).
 template <bool S2>
 __device__ inline void batch_convdiff3_items(BView V, Plan P, const double* u, const double* v,
@@ -1302,7 +1302,7 @@ __device__ inline void batch_convdiff3_items(BView V, Plan P, const double* u, c
     const int kt = (g.nk + TK - 1) / TK, jt = (g.nj + TJ - 1) / TJ;
     convdiff3_body<S2>(u + M.off, v + M.off, w + M.off, vis + M.off, S2 ? wpre + M.off : nullptr,
                        us + M.off, vs + M.off, ws + M.off, uoo + M.off, voo + M.off, woo + M.off,
-                       g, BATCH_CD_ICH, q % kt, (q / kt) % jt, q / (kt * jt),
+                       g, P.ich, q % kt, (q / kt) % jt, q / (kt * jt),
                        member_coefs(M, alpha));
     __syncthreads();  // LDS of this item is free for the next
   }
@@ -1519,10 +1519,11 @@ static int convdiff3_any_launch(const double* u, const double* v, const double* 
   using namespace cdv;
   const int kt = div_up(g.nk, TK), jt = div_up(g.nj, TJ);
   if (ich <= 0) ich = tune_get(wpre ? WF_TUNE_CD3S2_ICH : WF_TUNE_CD3_ICH, g.ni, g.nj, g.nk);
-  if (ich <= 0) {  // one round of workgroups (three per CU), >= 16 planes each
-    const int64_t tiles = (int64_t)kt * jt, slots = 768;
-    ich = (int)std::max<int64_t>(16, (tiles * g.ni + slots - 1) / slots);
-  }
+  // three workgroups per CU; us, built-in chunks before / by pick_chunk: 24^3
+  // 31 / 7, 64^3 32 / 12, 80^3 34 / 21, 176x240x208 284 / 225, 256^3 430 / 363
+  if (ich <= 0)
+    ich = pick_chunk(g.ni, ChunkCost{3, {2.05, 3.0, 4.15}}, INT32_MAX,
+                     [&](int c) { return (int64_t)kt * jt * div_up(g.ni, c); });
   const int nch = div_up(g.ni, ich);
   if ((int64_t)kt * jt * nch >= (int64_t)1 << 31) return WF_EINVAL;
   if (g.si * (int64_t)sizeof(double) >= ((int64_t)1 << 30)) return WF_EINVAL;  // buffer range

@@ -2140,17 +2140,6 @@ int max_lds() {
   return g_max_lds;
 }
 
-int cu_count() {
-  static const int n = [] {
-    int dev = 0, v = 256;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-      v = 256;
-    return v;
-  }();
-  return n;
-}
-
 template <class T>
 int launch_rbgs(const wf_mg_level& L, int color, int write_ring, hipStream_t s) {
   const MgDev d = mg_dev(L);

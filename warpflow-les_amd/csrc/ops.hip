@@ -951,7 +951,7 @@ batch_wale_kernel(BView V, Plan P, const double* u, const double* v, const doubl
   for_items<true>(P, V, nullptr, [&](int, int q, const MemDev& M) {
     const Box3 b = cells_box(M.g);
     const int kt = (b.d2 + WS_TK - 1) / WS_TK, jt = (b.d1 + WS_TJ - 1) / WS_TJ;
-    wale_stream_body(u + M.off, v + M.off, w + M.off, vis + M.off, M.g, b, BATCH_CD_ICH, q % kt,
+    wale_stream_body(u + M.off, v + M.off, w + M.off, vis + M.off, M.g, b, P.ich, q % kt,
                      (q / kt) % jt, q / (kt * jt), 1.0 / M.dx, 1.0 / M.dy, 1.0 / M.dz, M.rey,
                      M.ls);
   });
@@ -984,12 +984,12 @@ batch_calmas_kernel(BView V, Plan P, const double* u, const double* v, const dou
   for_items<true>(P, V, active, [&](int, int q, const MemDev& M) {
     const Box3 b = cells_box(M.g);
     calmas_body(u + M.off, v + M.off, w + M.off, su + M.off, M.g, b, cells_blk(q, b.d1, b.d2),
-                BATCH_RED_ICH, M.dx, M.dy, M.dz, M.dt, part, M.red0 + q);
+                P.ich, M.dx, M.dy, M.dz, M.dt, part, M.red0 + q);
   });
 }
 
 // The fused calvel/calmas pass per member on the reduction items (64 x 4
-// (k, j) tiles x BATCH_RED_ICH planes), so its partials fill the slots
+// (k, j) tiles x P.ich planes), so its partials fill the slots
 // batch_red_fold_kernel folds, as batch_calmas_kernel's do.
 __global__ void __launch_bounds__(256)
 batch_calvel3_calmas_kernel(BView V, Plan P, const double* us, const double* vs,
@@ -1003,7 +1003,7 @@ batch_calvel3_calmas_kernel(BView V, Plan P, const double* us, const double* vs,
                        1.0 / M.dt, M.dx, M.dy, M.dz};
     const double r = calvel3_calmas_body<4, 64>(
         us + M.off, vs + M.off, ws + M.off, p + M.off, u + M.off, v + M.off, w + M.off,
-        su + M.off, g, BATCH_RED_ICH, q % kt, (q / kt) % jt, q / (kt * jt), K);
+        su + M.off, g, P.ich, q % kt, (q / kt) % jt, q / (kt * jt), K);
     if (threadIdx.x == 0) part[M.red0 + q] = r;
   });
 }
@@ -1014,7 +1014,7 @@ batch_checkdt_kernel(BView V, Plan P, const double* u, const double* v, const do
   for_items<true>(P, V, nullptr, [&](int, int q, const MemDev& M) {
     const Box3 b = cells_box(M.g);
     checkdt_body(u + M.off, v + M.off, w + M.off, vis + M.off, M.g, b,
-                 cells_blk(q, b.d1, b.d2), BATCH_RED_ICH, M.dx, M.dy, M.dz, M.rsum, part,
+                 cells_blk(q, b.d1, b.d2), P.ich, M.dx, M.dy, M.dz, M.rsum, part,
                  stride, M.red0 + q);
   });
 }
@@ -1022,12 +1022,12 @@ batch_checkdt_kernel(BView V, Plan P, const double* u, const double* v, const do
 // One workgroup per member folds its reduction partials: out[m*nq + q] for
 // quantity q (bit q of min_mask: min, else max).
 __global__ void __launch_bounds__(1024)
-batch_red_fold_kernel(BView V, const double* part, int stride, int nq, int min_mask,
+batch_red_fold_kernel(BView V, Plan P, const double* part, int stride, int nq, int min_mask,
                       double* out, const int* active) {
   const int m = blockIdx.x;
   if (active && !active[m]) return;  // uniform per workgroup
   const MemDev& M = V.mem[m];
-  const int n = red_blocks(M.g.ni, M.g.nj, M.g.nk);
+  const int n = P.start[m + 1] - P.start[m];  // the member's PK_RED items
   __shared__ double sh[16];
   const int t = threadIdx.x;
   for (int q = 0; q < nq; ++q) {
@@ -1097,7 +1097,7 @@ int batch_calmas(const Batch& B, const double* u, const double* v, const double*
   hipLaunchKernelGGL(batch_calmas_kernel, dim3(P.grid), box_block(), 0, s, B.view(), P, u, v, w,
                      su, B.red_part, active);
   WF_LAUNCHED();
-  hipLaunchKernelGGL(batch_red_fold_kernel, dim3(B.nmem), dim3(1024), 0, s, B.view(),
+  hipLaunchKernelGGL(batch_red_fold_kernel, dim3(B.nmem), dim3(1024), 0, s, B.view(), P,
                      (const double*)B.red_part, B.nred, 1, 0, rmax, active);
   WF_LAUNCHED();
   return 0;
@@ -1110,7 +1110,7 @@ int batch_calvel3_calmas(const Batch& B, const double* us, const double* vs, con
   hipLaunchKernelGGL(batch_calvel3_calmas_kernel, dim3(P.grid), dim3(256), 0, s, B.view(), P, us,
                      vs, ws, p, u, v, w, su, B.red_part, alpha, active);
   WF_LAUNCHED();
-  hipLaunchKernelGGL(batch_red_fold_kernel, dim3(B.nmem), dim3(1024), 0, s, B.view(),
+  hipLaunchKernelGGL(batch_red_fold_kernel, dim3(B.nmem), dim3(1024), 0, s, B.view(), P,
                      (const double*)B.red_part, B.nred, 1, 0, rmax, active);
   WF_LAUNCHED();
   return 0;
@@ -1122,7 +1122,7 @@ int batch_checkdt(const Batch& B, const double* u, const double* v, const double
   hipLaunchKernelGGL(batch_checkdt_kernel, dim3(P.grid), box_block(), 0, s, B.view(), P, u, v, w,
                      vis, B.red_part, B.nred);
   WF_LAUNCHED();
-  hipLaunchKernelGGL(batch_red_fold_kernel, dim3(B.nmem), dim3(1024), 0, s, B.view(),
+  hipLaunchKernelGGL(batch_red_fold_kernel, dim3(B.nmem), dim3(1024), 0, s, B.view(), P,
                      (const double*)B.red_part, B.nred, 4, 8, out4, (const int*)nullptr);
   WF_LAUNCHED();
   return 0;
@@ -1357,9 +1357,12 @@ static int calvel3_calmas_launch(const double* ustar, const double* vstar, const
     if (e) return e;
     return wf_calmas(u, v, w, su, rmax_dev, g, g.ni, g.nj, g.nk, dx, dy, dz, dt, stream);
   }
-  // built-in: >= 2048 workgroups where the grid allows; at most RED_MAX_BLOCKS
+  // four workgroups per CU, at most RED_MAX_BLOCKS in all; us, built-in chunks
+  // before / by pick_chunk: 24^3 11.9 / 8.3, 80^3 15.9 / 14.3, 256^3 258 / 232
   int ich = tune_get(WF_TUNE_PROJ_ICH, g.ni, g.nj, g.nk);
-  if (ich <= 0) ich = (int)std::max<int64_t>(8, (tiles * g.ni + 2047) / 2048);
+  if (ich <= 0)
+    ich = pick_chunk(g.ni, ChunkCost{4, {1.1, 1.75, 2.75, 3.7}}, RED_MAX_BLOCKS,
+                     [&](int c) { return tiles * div_up(g.ni, c); });
   ich = std::max(ich, div_up(g.ni, (int)(RED_MAX_BLOCKS / tiles)));
   const int nch = div_up(g.ni, ich);
   RedGeom r;
@@ -1397,6 +1400,13 @@ int wf_calmas_of_calvel3(const double* ustar, const double* vstar, const double*
                                rhs32, g, dx, dy, dz, dt, alpha, stream, false);
 }
 
+// i-planes per workgroup of the WALE streams (four workgroups per CU); us with
+// checkdt, chunks before / by pick_chunk: 24^3 26.4 / 13.2, 80^3 27.5 / 21.6
+static int wale_chunk(int64_t tiles, int n0, int64_t limit) {
+  return pick_chunk(n0, ChunkCost{4, {1.04, 1.62, 2.18, 2.83}}, limit,
+                    [&](int c) { return tiles * div_up(n0, c); });
+}
+
 int wf_wale(const double* u, const double* v, const double* w, double* vis, wf_grid g,
             int d0, int d1, int d2, double dx, double dy, double dz, double rrey,
             double cw, double delta, void* stream) {
@@ -1404,7 +1414,7 @@ int wf_wale(const double* u, const double* v, const double* w, double* vis, wf_g
   if (!box_ok(g, b, 1, 1)) return WF_EINVAL;
   if (empty(b)) return 0;
   const int kt = div_up(b.d2, WS_TK), jt = div_up(b.d1, WS_TJ);
-  const int ich = (int)std::max<int64_t>(16, ((int64_t)kt * jt * b.d0 + 2047) / 2048);
+  const int ich = wale_chunk((int64_t)kt * jt, b.d0, INT32_MAX);
   hipLaunchKernelGGL(wale_stream_kernel, dim3(kt * jt, div_up(b.d0, ich)), dim3(256), 0,
                      S_(stream), u, v, w, vis, g, b, ich, kt, jt, 1.0 / dx, 1.0 / dy, 1.0 / dz,
                      rrey, cw * delta);
@@ -1461,7 +1471,7 @@ int wf_wale_checkdt(const double* u, const double* v, const double* w, double* v
   if (empty(b)) return 0;
   const int kt = div_up(b.d2, WS_TK), jt = div_up(b.d1, WS_TJ);
   const int64_t tiles = (int64_t)kt * jt;
-  int ich = (int)std::max<int64_t>(16, (tiles * b.d0 + 2047) / 2048);
+  int ich = wale_chunk(tiles, b.d0, RED_MAX_BLOCKS);
   if (tiles > RED_MAX_BLOCKS) {  // more tiles than partial slots: the two passes
     const int e = wf_checkdt(u, v, w, vis, out4_dev, g, dx, dy, dz, stream);
     if (e) return e;

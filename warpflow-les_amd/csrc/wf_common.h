@@ -76,6 +76,47 @@ inline int plane_chunk(int d0, int d1, int d2) {
 inline dim3 chunk_grid(int d0, int d1, int d2, int ich) {
   return dim3(div_up(d2, BX), div_up(d1, BY), div_up(d0, ich));
 }
+// i-planes per workgroup of a kernel that streams a (j, k) tile along i.  A
+// chunk of ich planes costs ich + 2 plane iterations (its prologue loads the
+// planes before it), and an iteration takes t[q-1] us with q workgroups on a CU,
+// measured: one workgroup waits for its loads, the most a CU holds (n) share
+// the memory's rate.  The chunk of the least total over the rounds of
+// workgroups is taken; small grids get chunks of one or two planes (24^3: a
+// chunk of 16 left six workgroups to walk 18 planes each, 32 us for 7).
+// tiles(ich): the launch's workgroups; limit: the most it may have.
+struct ChunkCost {
+  int n;
+  double t[4];
+};
+inline int cu_count() {
+  static const int n = [] {
+    int dev = 0, v = 256;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+      v = 256;
+    return v;
+  }();
+  return n;
+}
+template <class F>
+inline int pick_chunk(int n0, const ChunkCost& C, int64_t limit, F&& tiles) {
+  const int64_t cu = cu_count(), round = cu * C.n;
+  int best = n0;
+  double least = 0;
+  for (int ich = 1; ich <= n0; ich += ich < 16 ? 1 : ich < 64 ? 2 : 8) {
+    const int64_t w = tiles(ich);
+    if (w > limit && ich < n0) continue;
+    const int64_t rest = w % round;
+    const double cost = (ich + 2) * ((double)(w / round) * C.t[C.n - 1] +
+                                     (rest ? C.t[(rest - 1) / cu] : 0.0));
+    if (least == 0 || cost < least) {
+      least = cost;
+      best = ich;
+    }
+  }
+  return div_up(n0, div_up(n0, best));  // equal chunks
+}
+
 // f(B) for every plane B.z of this workgroup's chunk; SYNC: a barrier after
 // each plane, for bodies that reduce through LDS.
 template <bool SYNC = false, class F>
