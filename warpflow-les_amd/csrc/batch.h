@@ -86,9 +86,6 @@ enum PlanKind : int {
   PK_CD0,           // convdiff tiles, components u, v, w
   PK_CD1,
   PK_CD2,
-  PK_BC0,           // ghost-fill lines of the x, y, z axis launches
-  PK_BC1,
-  PK_BC2,
   PK_WALE,          // WALE tiles (8 x 32 (j, k) x ich planes) over the real cells;
                     // also the three-component conv+diff passes
   PK_CDE,           // u's edge planes 0 and ni-2: 8 x 32 (j, k) tiles x 2
@@ -117,6 +114,9 @@ struct Batch {
   Plan plan[PK_COUNT];
   int* plan_mem[PK_COUNT] = {};     // device start arrays
   BatchRelax relax[BATCH_MAX_LEVELS];
+  void* bc_fill = nullptr;          // ghost fills of every member (device; bcs.hip)
+  int2 *bc_x = nullptr, *bc_yz = nullptr;  // their items: (member, first x line), (member, plane)
+  int bc_nx = 0, bc_nyz = 0;
   double* red_part = nullptr;       // 4 * nred reduction partials (device)
   int nred = 0;
   double* sum_part = nullptr;       // nsum sum partials (device)
@@ -171,12 +171,12 @@ int batch_convdiff_u_edges(const Batch& B, const double* u, const double* v, con
                            hipStream_t s);
 int batch_save_cross_ghosts(const Batch& B, const double* w, double* wpre, hipStream_t s);
 int batch_bc_fill(const Batch& B, double* f, int which, const int* active, hipStream_t s);
-int batch_bc_fill_n(const Batch& B, double* const* f, const int* which, int nf,
+int batch_bc_fill_n(const Batch& B, double* const* f, const int* which, int nf, bool edges,
                     const int* active, hipStream_t s);
+int batch_bc_init(Batch& B);
 int batch_vcycle(const Batch& B, float* const* phi, float* const* rhs, float* const* tmp,
                  const float* cop, int npre, int npost, int ncoarse, const int* active,
                  hipStream_t s, bool zero0);
-int bc_blocks(int axis, int ni, int nj, int nk);
 int batch_mg_init();
 void batch_relax_plan(const MemDev* mem, int nmem, int l, BatchRelax& P,
                       std::vector<int4>& items);

@@ -63,10 +63,6 @@ int member_count(int kind, const MemDev& M, int ich) {
       op_dims(kind - PK_CD0, n0, n1, n2, d0, d1, d2);
       return cd_tiles(d0, d1, d2, ich);
     }
-    case PK_BC0:
-    case PK_BC1:
-    case PK_BC2:
-      return bc_blocks(kind - PK_BC0, n0, n1, n2);
     case PK_WALE:
       return cd_tiles(n0, n1, n2, ich);
     case PK_CDE:
@@ -96,6 +92,9 @@ void batch_free(Batch* B) {
     if (B->plan_mem[k]) (void)hipFree(B->plan_mem[k]);
   for (int l = 0; l < BATCH_MAX_LEVELS; ++l)
     if (B->relax[l].item) (void)hipFree(const_cast<int4*>(B->relax[l].item));
+  if (B->bc_fill) (void)hipFree(B->bc_fill);
+  if (B->bc_x) (void)hipFree(B->bc_x);
+  if (B->bc_yz) (void)hipFree(B->bc_yz);
   if (B->mem_dev) (void)hipFree(B->mem_dev);
   if (B->red_part) (void)hipFree(B->red_part);
   if (B->sum_part) (void)hipFree(B->sum_part);
@@ -227,6 +226,11 @@ int create(const wf_member* mem, int nmem, int nlev, Batch** out) {
     }
     P.start = B->plan_mem[k];
   }
+  rc = batch_bc_init(*B);
+  if (rc) {
+    batch_free(B);
+    return rc;
+  }
   std::vector<int4> items;
   for (int l = 0; l < nlev; ++l) {
     BatchRelax& P = B->relax[l];
@@ -311,8 +315,8 @@ int wf_batch_bc_fill(wf_batch b, double* f, int which, const int* active, void* 
   return batch_bc_fill(B_(b), f, which, active, (hipStream_t)stream);
 }
 
-int wf_batch_bc_fill_uvw(wf_batch b, double* u, double* v, double* w, const int* active,
-                         void* stream) {
+static int fill_uvw(wf_batch b, double* u, double* v, double* w, bool edges, const int* active,
+                    void* stream) {
   if (!ok(b) || !v || !w) return WF_EINVAL;
   double* f[3];
   int which[3], nf = 0;
@@ -324,7 +328,15 @@ int wf_batch_bc_fill_uvw(wf_batch b, double* u, double* v, double* w, const int*
   which[nf++] = 1;
   f[nf] = w;
   which[nf++] = 2;
-  return batch_bc_fill_n(B_(b), f, which, nf, active, (hipStream_t)stream);
+  return batch_bc_fill_n(B_(b), f, which, nf, edges, active, (hipStream_t)stream);
+}
+int wf_batch_bc_fill_uvw(wf_batch b, double* u, double* v, double* w, const int* active,
+                         void* stream) {
+  return fill_uvw(b, u, v, w, false, active, stream);
+}
+int wf_batch_bc_refill_uvw(wf_batch b, double* u, double* v, double* w, const int* active,
+                           void* stream) {
+  return fill_uvw(b, u, v, w, true, active, stream);
 }
 
 int wf_batch_convdiff(wf_batch b, int comp, const double* u, const double* v, const double* w,

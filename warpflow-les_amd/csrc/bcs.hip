@@ -28,14 +28,14 @@ struct BcOp {
 struct BcOps {
   BcOp op[4];
   int32_t n;
+  int32_t hoist;  // bc_ops_hoistable, set by the host
 };
 
 // Whether every source cell of the op list lies outside the ghost cells
 // written by the same or an earlier op (and every op has at most 3 layers):
 // then all sources can be loaded before the first store and the stores keep
 // their order, which leaves every cell with the value of the op-by-op walk.
-// Uniform over a launch (it depends on the ops only).
-__host__ __device__ inline bool bc_ops_hoistable(const BcOps& ops) {
+static inline bool bc_ops_hoistable(const BcOps& ops) {
   if (ops.n > 4) return false;
   for (int q = 0; q < ops.n; ++q) {
     const BcOp& o = ops.op[q];
@@ -53,13 +53,12 @@ __host__ __device__ inline bool bc_ops_hoistable(const BcOps& ops) {
 }
 
 // The ops of one (a, b) line along `axis`, low side then high side.  When
-// the ops allow it (bc_ops_hoistable) a thread issues all its loads before
+// the ops allow it (BcOps::hoist) a thread issues all its loads before
 // its first store, so a line costs one memory round trip instead of one per
 // layer and side (a load after a store to the same array cannot be moved
 // ahead of it by the compiler).
-__device__ inline void bc_line(double* __restrict__ f, const wf_grid& g, int axis, int a, int b,
-                               const BcOps& ops) {
-  int64_t base, s;
+__device__ inline void bc_line_base(const wf_grid& g, int axis, int a, int b, int64_t& base,
+                                    int64_t& s) {
   if (axis == 0) {
     base = at(g, 0, a, b);
     s = g.si;
@@ -70,36 +69,43 @@ __device__ inline void bc_line(double* __restrict__ f, const wf_grid& g, int axi
     base = at(g, a, b, 0);
     s = 1;
   }
-  if (bc_ops_hoistable(ops)) {
-    // every op field, destination and source value is in registers before
-    // the first store (a kernel-argument read placed after a store would
-    // wait for that store to complete)
-    double v[4][3];
-    int64_t dst[4][3];
-    bool on[4][3];
+}
+__device__ inline void bc_line_hoisted(double* __restrict__ f, const wf_grid& g, int axis, int a,
+                                       int b, const BcOps& ops) {
+  int64_t base, s;
+  bc_line_base(g, axis, a, b, base, s);
+  // every op field, destination and source value is in registers before
+  // the first store (a kernel-argument read placed after a store would
+  // wait for that store to complete)
+  double v[4][3];
+  int64_t dst[4][3];
+  bool on[4][3];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const BcOp o = ops.op[q];
-      const bool used = q < ops.n;
+  for (int q = 0; q < 4; ++q) {
+    const BcOp o = ops.op[q];
+    const bool used = q < ops.n;
 #pragma unroll
-      for (int m = 0; m < 3; ++m) {
-        on[q][m] = used && m < o.nlay;
-        dst[q][m] = base + (int64_t)(o.high ? o.g0 + m : o.g0 - m) * s;
-        // unconditional load (cell 0 of the line when no source is read), so
-        // no branch separates the loads
-        const bool src = on[q][m] && o.kind != 0;
-        const double x = f[base + (int64_t)(src ? (o.high ? o.s0 - m : o.s0 + m) : 0) * s];
-        v[q][m] = src ? o.val * x : o.val;
-      }
+    for (int m = 0; m < 3; ++m) {
+      on[q][m] = used && m < o.nlay;
+      dst[q][m] = base + (int64_t)(o.high ? o.g0 + m : o.g0 - m) * s;
+      // unconditional load (cell 0 of the line when no source is read), so
+      // no branch separates the loads
+      const bool src = on[q][m] && o.kind != 0;
+      const double x = f[base + (int64_t)(src ? (o.high ? o.s0 - m : o.s0 + m) : 0) * s];
+      v[q][m] = src ? o.val * x : o.val;
     }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-#pragma unroll
-      for (int m = 0; m < 3; ++m)
-        if (on[q][m]) f[dst[q][m]] = v[q][m];
-    }
-    return;
   }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+#pragma unroll
+    for (int m = 0; m < 3; ++m)
+      if (on[q][m]) f[dst[q][m]] = v[q][m];
+  }
+}
+__device__ inline void bc_line_walk(double* __restrict__ f, const wf_grid& g, int axis, int a,
+                                    int b, const BcOps& ops) {
+  int64_t base, s;
+  bc_line_base(g, axis, a, b, base, s);
   for (int q = 0; q < ops.n; ++q) {
     const BcOp o = ops.op[q];
     for (int m = 0; m < o.nlay; ++m) {
@@ -112,6 +118,13 @@ __device__ inline void bc_line(double* __restrict__ f, const wf_grid& g, int axi
       }
     }
   }
+}
+__device__ inline void bc_line(double* __restrict__ f, const wf_grid& g, int axis, int a, int b,
+                               const BcOps& ops) {
+  if (ops.hoist)
+    bc_line_hoisted(f, g, axis, a, b, ops);
+  else
+    bc_line_walk(f, g, axis, a, b, ops);
 }
 
 __global__ void __launch_bounds__(256)
@@ -189,8 +202,19 @@ struct BcYZ {
 // cache lines of 64 / ZLANES lines per access, where a thread per line
 // touches 64 (the ghosts and sources of a line share its first and last
 // lines).  A thread issues the loads of ZU groups before their stores.
+// The lane's ghost cell (threads t, t + blockDim.x, ... of a workgroup of a
+// multiple of ZLANES threads own the same one).
+struct BcLane {
+  int g, src;
+  double val;
+  bool on;
+};
+__device__ inline BcLane bc_lane(const BcCells& zc) {
+  const int c = threadIdx.x % ZLANES;
+  return BcLane{zc.g[c], zc.src[c], zc.val[c], c < zc.n};
+}
 __device__ inline void bc_zcells(double* __restrict__ f, const wf_grid& g, int i, int b0, int nb,
-                                 const BcCells& zc) {
+                                 const BcLane& L) {
   constexpr int ZU = 4;
   const int total = nb * ZLANES, nt = blockDim.x;
   for (int t0 = threadIdx.x; t0 < total; t0 += ZU * nt) {
@@ -199,15 +223,13 @@ __device__ inline void bc_zcells(double* __restrict__ f, const wf_grid& g, int i
     bool on[ZU];
 #pragma unroll
     for (int u = 0; u < ZU; ++u) {
-      const int t = t0 + u * nt, c = t % ZLANES;
-      on[u] = t < total && c < zc.n;
-      const int cc = on[u] ? c : 0;
+      const int t = t0 + u * nt;
+      on[u] = t < total && L.on;
       const int64_t base = at(g, i, b0 + (on[u] ? t / ZLANES : 0), 0);
-      dst[u] = base + zc.g[cc];
-      const int sc = zc.src[cc];
+      dst[u] = base + L.g;
       // unconditional load (cell 0 of the line for a constant ghost)
-      const double x = f[base + (sc >= 0 ? sc : 0)];
-      v[u] = sc >= 0 ? zc.val[cc] * x : zc.val[cc];
+      const double x = f[base + (on[u] && L.src >= 0 ? L.src : 0)];
+      v[u] = L.src >= 0 ? L.val * x : L.val;
     }
 #pragma unroll
     for (int u = 0; u < ZU; ++u)
@@ -230,10 +252,85 @@ __global__ void __launch_bounds__(1024) bc_yz_kernel(BcYZ A, wf_grid g) {
       for (int b = threadIdx.x; b < A.nbz[z]; b += blockDim.x)
         if (in_band(A.bz0[z] + b, A.yl[z], A.yh[z])) bc_line(A.f[z], g, 2, i, A.bz0[z] + b, A.oz[z]);
     } else if (A.zc[z].n > 0)
-      bc_zcells(A.f[z], g, i, A.bz0[z], A.nbz[z], A.zc[z]);
+      bc_zcells(A.f[z], g, i, A.bz0[z], A.nbz[z], bc_lane(A.zc[z]));
     else
       for (int b = threadIdx.x; b < A.nbz[z]; b += blockDim.x)
         bc_line(A.f[z], g, 2, i, A.bz0[z] + b, A.oz[z]);
+  }
+}
+
+
+// One member's fill `which`: the launch ranges and ops of each axis, the z
+// ghost cells, and the bands a refill skips by (all made by the host).
+struct BcFill {
+  int32_t a0[3], na[3], b0[3], nb[3];
+  BcOps ops[3];
+  BcCells zc;
+  int32_t lo[3], hi[3];
+  int32_t dep;  // some op reads its own axis's band: refills run in full
+};
+// Fields of a multi-field batched fill: blockIdx.y picks field z.
+struct BcFields {
+  double* f[3];
+  int which[3];
+};
+// The x ops of every member: 256 lines per item (member, first line), numbered
+// over the item's field's own range.
+__global__ void __launch_bounds__(256)
+batch_bc_x_kernel(BView V, const int2* item, const BcFill* fill, BcFields F, int edges,
+                  const int* active) {
+  const int2 it = item[blockIdx.x];
+  if (active && !active[it.x]) return;
+  const int z = blockIdx.y;
+  const BcFill& B = fill[it.x * 6 + F.which[z]];
+  const int q = it.y + (int)threadIdx.x, nb = B.nb[0];
+  if (q >= B.na[0] * nb) return;
+  const int a = B.a0[0] + q / nb, b = B.b0[0] + q % nb;
+  if (edges && !B.dep && !in_band(a, B.lo[1], B.hi[1]) && !in_band(b, B.lo[2], B.hi[2])) return;
+  const MemDev& M = V.mem[it.x];
+  bc_line(F.f[z] + M.off, M.g, 0, a, b, B.ops[0]);
+}
+// The y and z ops of every member, an item (member, plane) per workgroup, as
+// bc_yz_kernel runs them.
+__global__ void __launch_bounds__(256)
+batch_bc_yz_kernel(BView V, const int2* item, const BcFill* fill, BcFields F, int edges,
+                   const int* active) {
+  const int2 it = item[blockIdx.x];
+  if (active && !active[it.x]) return;  // uniform per workgroup
+  const int z = blockIdx.y, i = it.y;
+  const BcFill& B = fill[it.x * 6 + F.which[z]];
+  const wf_grid g = V.mem[it.x].g;
+  double* const f = F.f[z] + V.mem[it.x].off;
+  const bool part = edges && !B.dep && !in_band(i, B.lo[0], B.hi[0]);
+  const int ay = B.a0[1], nay = B.na[1], by = B.b0[1], nby = B.nb[1];
+  const int az = B.a0[2], naz = B.na[2], bz = B.b0[2], nbz = B.nb[2];
+  const int zl = B.lo[2], zh = B.hi[2], yl = B.lo[1], yh = B.hi[1];
+  // read before the first store (the walk, for grids of a few cells, reads
+  // its ops from memory)
+  const BcOps oy = B.ops[1], oz = B.ops[2];
+  const int nzc = B.zc.n;
+  const BcLane lane = bc_lane(B.zc);
+  if (i >= ay && i < ay + nay)
+    for (int b = threadIdx.x; b < nby; b += blockDim.x)
+      if (!part || in_band(by + b, zl, zh)) {
+        if (oy.hoist)
+          bc_line_hoisted(f, g, 1, i, by + b, oy);
+        else
+          bc_line_walk(f, g, 1, i, by + b, B.ops[1]);
+      }
+  __syncthreads();
+  if (i >= az && i < az + naz) {
+    if (part || nzc == 0) {
+      for (int b = threadIdx.x; b < nbz; b += blockDim.x)
+        if (!part || in_band(bz + b, yl, yh)) {
+          if (oz.hoist)
+            bc_line_hoisted(f, g, 2, i, bz + b, oz);
+          else
+            bc_line_walk(f, g, 2, i, bz + b, B.ops[2]);
+        }
+    } else {
+      bc_zcells(f, g, i, bz, nbz, lane);
+    }
   }
 }
 
@@ -281,13 +378,13 @@ static int launch_axis(double* f, const wf_grid& g, int axis, int a0, int na, in
   return 0;
 }
 
-__host__ __device__ inline BcOp C_(int high, int g0, double val, int nlay) {
+static BcOp C_(int high, int g0, double val, int nlay) {
   return BcOp{0, high, g0, 0, nlay, val};
 }
-__host__ __device__ inline BcOp L_(int high, int g0, int s0, double sign, int nlay) {
+static BcOp L_(int high, int g0, int s0, double sign, int nlay) {
   return BcOp{1, high, g0, s0, nlay, sign};
 }
-__host__ __device__ inline BcOps ops2(BcOp a, BcOp b) {
+static BcOps ops2(BcOp a, BcOp b) {
   BcOps o{};
   o.op[0] = a;
   o.op[1] = b;
@@ -300,9 +397,8 @@ __host__ __device__ inline BcOps ops2(BcOp a, BcOp b) {
 // (which = 0..5, bcs.py:201-311) on an N-ghost field of ni x nj x nk real
 // cells.  The reference uses one n for every axis; here each range uses its
 // own axis' count, identical for a cubic grid.  False for an unknown `which`.
-__host__ __device__ inline bool bc_axis_ops(int which, int axis, int N, int ni, int nj, int nk,
-                                            double param, int& a0, int& na, int& b0, int& nb,
-                                            BcOps& o) {
+static bool bc_axis_ops_of(int which, int axis, int N, int ni, int nj, int nk, double param,
+                           int& a0, int& na, int& b0, int& nb, BcOps& o) {
   a0 = b0 = N - 1;
   const int n3[3] = {ni, nj, nk};
   const int pa = axis == 0 ? nj : ni, pb = axis == 2 ? nj : nk;  // perpendicular counts
@@ -378,75 +474,12 @@ __host__ __device__ inline bool bc_axis_ops(int which, int axis, int N, int ni, 
   }
 }
 
-namespace wf {
-
-// Line blocks of one axis launch per member: 64 x 4 (b, a) blocks over the
-// widest range any fill uses ((perpendicular count + 6) per side).
-__host__ __device__ inline void bc_extent(int axis, int ni, int nj, int nk, int& namax,
-                                          int& nbmax) {
-  namax = (axis == 0 ? nj : ni) + 6;
-  nbmax = (axis == 2 ? nj : nk) + 6;
+static bool bc_axis_ops(int which, int axis, int N, int ni, int nj, int nk, double param, int& a0,
+                        int& na, int& b0, int& nb, BcOps& o) {
+  if (!bc_axis_ops_of(which, axis, N, ni, nj, nk, param, a0, na, b0, nb, o)) return false;
+  o.hoist = bc_ops_hoistable(o);
+  return true;
 }
-int bc_blocks(int axis, int ni, int nj, int nk) {
-  int na, nb;
-  bc_extent(axis, ni, nj, nk, na, nb);
-  return div_up(nb, 64) * div_up(na, 4);
-}
-
-// Fields of a multi-field batched fill: blockIdx.y picks field z.
-struct BcFields {
-  double* f[3];
-  int which[3];
-};
-
-__global__ void __launch_bounds__(256)
-batch_bc_kernel(BView V, Plan P, BcFields F, int axis, const int* active) {
-  double* __restrict__ f = F.f[blockIdx.y];
-  const int which = F.which[blockIdx.y];
-  for (int it = blockIdx.x; it < P.total; it += gridDim.x) {
-    const int m = member_of(P.start, V.nmem, it);
-    if (active && !active[m]) continue;
-    const int q = it - P.start[m];
-    const MemDev& M = V.mem[m];
-    const wf_grid g = M.g;
-    const double param = which == 0 ? M.ulid : (which == 3 ? M.rey : (double)g.npl);
-    int a0, na, b0, nb;
-    BcOps o{};
-    bc_axis_ops(which, axis, g.npl, g.ni, g.nj, g.nk, param, a0, na, b0, nb, o);
-    int namax, nbmax;
-    bc_extent(axis, g.ni, g.nj, g.nk, namax, nbmax);
-    const int nx = (nbmax + 63) / 64;
-    const int bb = (q % nx) * 64 + threadIdx.x, aa = (q / nx) * 4 + threadIdx.y;
-    if (aa < na && bb < nb) bc_line(f + M.off, g, axis, a0 + aa, b0 + bb, o);
-  }
-}
-
-// The three axis launches of the fills which[z] of fields f[z] (z < nf,
-// independent fields) over every (active) member: each launch covers the nf
-// fields, one per grid row, so the axes keep their order within each field.
-int batch_bc_fill_n(const Batch& B, double* const* f, const int* which, int nf,
-                    const int* active, hipStream_t s) {
-  if (nf < 1 || nf > 3) return WF_EINVAL;
-  BcFields F{};
-  for (int z = 0; z < nf; ++z) {
-    if (!f[z] || which[z] < 0 || which[z] > 5) return WF_EINVAL;
-    F.f[z] = f[z];
-    F.which[z] = which[z];
-  }
-  for (int axis = 0; axis < 3; ++axis) {
-    const Plan& P = B.plan[PK_BC0 + axis];
-    hipLaunchKernelGGL(batch_bc_kernel, dim3(P.grid, nf), dim3(64, 4), 0, s, B.view(), P, F,
-                       axis, active);
-    WF_LAUNCHED();
-  }
-  return 0;
-}
-
-int batch_bc_fill(const Batch& B, double* f, int which, const int* active, hipStream_t s) {
-  return batch_bc_fill_n(B, &f, &which, 1, active, s);
-}
-
-}  // namespace wf
 
 extern "C" {
 
@@ -455,6 +488,7 @@ int wf_bc_lin(double* fld, wf_grid g, int axis, int high, int g0, int s0, double
   BcOps o{};
   o.op[0] = L_(high != 0, g0, s0, sign, nlay);
   o.n = 1;
+  o.hoist = bc_ops_hoistable(o);
   return launch_axis(fld, g, axis, a0, na, b0, nb, o, (hipStream_t)stream);
 }
 
@@ -463,6 +497,7 @@ int wf_bc_const(double* fld, wf_grid g, int axis, int high, int g0, double val, 
   BcOps o{};
   o.op[0] = C_(high != 0, g0, val, nlay);
   o.n = 1;
+  o.hoist = bc_ops_hoistable(o);
   return launch_axis(fld, g, axis, a0, na, b0, nb, o, (hipStream_t)stream);
 }
 
@@ -540,6 +575,80 @@ static bool fill_bands(int which, double param, const wf_grid& g, int lo[3], int
   }
   return true;
 }
+
+}  // extern "C"
+
+namespace wf {
+
+// A batch's fills and their item lists, made once at creation.
+int batch_bc_init(Batch& B) {
+  std::vector<BcFill> fill(6 * (size_t)B.nmem);
+  std::vector<int2> x, yz;
+  for (int m = 0; m < B.nmem; ++m) {
+    const MemDev& M = B.mem_host[m];
+    int lines = 0;
+    for (int which = 0; which < 6; ++which) {
+      BcFill& D = fill[6 * (size_t)m + which];
+      D = BcFill{};
+      const double param = which == 0 ? M.ulid : which == 3 ? M.rey : (double)M.g.npl;
+      for (int axis = 0; axis < 3; ++axis)
+        if (!bc_axis_ops(which, axis, M.g.npl, M.g.ni, M.g.nj, M.g.nk, param, D.a0[axis],
+                         D.na[axis], D.b0[axis], D.nb[axis], D.ops[axis]) ||
+            !ops_ok(M.g, axis, D.a0[axis], D.na[axis], D.b0[axis], D.nb[axis], D.ops[axis]))
+          return WF_EINVAL;
+      D.zc = z_cells(D.ops[2]);
+      bool dep = false;
+      if (!fill_bands(which, param, M.g, D.lo, D.hi, &dep)) return WF_EINVAL;
+      D.dep = dep;
+      lines = std::max(lines, D.na[0] * D.nb[0]);
+    }
+    for (int q = 0; q < lines; q += 256) x.push_back(int2{m, q});
+    for (int i = 0; i < M.g.ni + 2 * M.g.npl; ++i) yz.push_back(int2{m, i});
+  }
+  B.bc_nx = (int)x.size();
+  B.bc_nyz = (int)yz.size();
+  const size_t nf = fill.size() * sizeof(BcFill), nx = x.size() * sizeof(int2),
+               ny = yz.size() * sizeof(int2);
+  WF_TRY(hipMalloc(&B.bc_fill, nf));
+  WF_TRY(hipMalloc((void**)&B.bc_x, nx));
+  WF_TRY(hipMalloc((void**)&B.bc_yz, ny));
+  WF_TRY(hipMemcpy(B.bc_fill, fill.data(), nf, hipMemcpyHostToDevice));
+  WF_TRY(hipMemcpy(B.bc_x, x.data(), nx, hipMemcpyHostToDevice));
+  WF_TRY(hipMemcpy(B.bc_yz, yz.data(), ny, hipMemcpyHostToDevice));
+  return 0;
+}
+
+// The fills which[z] of fields f[z] (z < nf, independent fields) over every
+// (active) member: an x launch, then a y-then-z launch, each over the nf
+// fields.  Three launches of an axis each, whose workgroups searched for their
+// member and formed the ops themselves, took 58 us apiece over a step of 64
+// members; these take 12 and 43.
+int batch_bc_fill_n(const Batch& B, double* const* f, const int* which, int nf, bool edges,
+                    const int* active, hipStream_t s) {
+  if (nf < 1 || nf > 3) return WF_EINVAL;
+  BcFields F{};
+  for (int z = 0; z < nf; ++z) {
+    if (!f[z] || which[z] < 0 || which[z] > 5) return WF_EINVAL;
+    F.f[z] = f[z];
+    F.which[z] = which[z];
+  }
+  const BcFill* fill = (const BcFill*)B.bc_fill;
+  hipLaunchKernelGGL(batch_bc_x_kernel, dim3(B.bc_nx, nf), dim3(256), 0, s, B.view(),
+                     (const int2*)B.bc_x, fill, F, (int)edges, active);
+  WF_LAUNCHED();
+  hipLaunchKernelGGL(batch_bc_yz_kernel, dim3(B.bc_nyz, nf), dim3(256), 0, s, B.view(),
+                     (const int2*)B.bc_yz, fill, F, (int)edges, active);
+  WF_LAUNCHED();
+  return 0;
+}
+
+int batch_bc_fill(const Batch& B, double* f, int which, const int* active, hipStream_t s) {
+  return batch_bc_fill_n(B, &f, &which, 1, false, active, s);
+}
+
+}  // namespace wf
+
+extern "C" {
 
 static int launch_yz(double* const* f, const int* which, const double* param, int nf,
                      const wf_grid& g, hipStream_t s, bool edges = false) {

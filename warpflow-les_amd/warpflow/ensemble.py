@@ -197,12 +197,13 @@ class Ensemble:
         self._call("wf_batch_bc_fill", self.pool[field].ptr, _BC[which or field],
                    active.ptr if active is not None else None, self.stream)
 
-    def _fill_uvw(self, with_u=True):
+    def _fill_uvw(self, with_u=True, again=False):
         """The fills of u (unless with_u is false), v and w for every member,
-        one launch per axis for the fields."""
+        each launch over the fields.  again: the fields were filled since
+        their last change (FlowSolver.refill_bc_uvw)."""
         P = self.pool
-        self._call("wf_batch_bc_fill_uvw", P["u"].ptr if with_u else None, P["v"].ptr,
-                   P["w"].ptr, None, self.stream)
+        self._call("wf_batch_bc_refill_uvw" if again else "wf_batch_bc_fill_uvw",
+                   P["u"].ptr if with_u else None, P["v"].ptr, P["w"].ptr, None, self.stream)
 
     def _calvel(self, alpha, active=None):
         P = self.pool
@@ -241,7 +242,7 @@ class Ensemble:
                            P["uoo"].ptr, P["voo"].ptr, P["woo"].ptr, P["vis"].ptr,
                            P["w_pre"].ptr, P["ustar"].ptr, P["vstar"].ptr, P["wstar"].ptr,
                            float(alpha), s)
-            self._fill_uvw()
+            self._fill_uvw(again=stage > 0)
             if stage + 1 < len(ALFARK):
                 self._calvel(alpha)
         # projection: reset the per-member loop state; every outer test opens
