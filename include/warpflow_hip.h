@@ -511,6 +511,10 @@ int wf_batch_wale(wf_batch b, const double* u, const double* v, const double* w,
 /* wf_checkdt: out4[4m .. 4m+3] = umax, vmax, wmax, dt limit of member m. */
 int wf_batch_checkdt(wf_batch b, const double* u, const double* v, const double* w,
                      const double* vis, double* out4, void* stream);
+/* wf_wale_checkdt: the two above in one pass over u, v, w (out4 from the vis
+ * that WALE replaces). */
+int wf_batch_wale_checkdt(wf_batch b, const double* u, const double* v, const double* w,
+                          double* vis, double* out4, void* stream);
 /* wf_bc_fill(which) with param = lid velocity (u), 1/Re (vis), 3 (p mirror). */
 int wf_batch_bc_fill(wf_batch b, double* f, int which, const int* active, void* stream);
 /* wf_bc_fill_uvw: the fills of u, v and w (u may be NULL: v and w only), each

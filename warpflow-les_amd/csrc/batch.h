@@ -27,6 +27,9 @@ struct MemDev {
   double dx, dy, dz, rey, ulid, noise, dt;
   double ls;    // WALE length scale cw * delta
   double rsum;  // 1/dx^2 + 1/dy^2 + 1/dz^2 (the checkdt viscous limit)
+  // 1/h, 1/h^2, 1/(24 h), 1/(12 h h) of each axis and 1/dt, formed here so that no
+  // workgroup opens with a chain of FP64 divisions
+  double r1[3], r2[3], r24[3], ir12[3], rdt;
   uint32_t seed;
   int nlev;
   int ln[BATCH_MAX_LEVELS][3];
@@ -40,9 +43,10 @@ struct MemDev {
 // A work-item list: start[m] .. start[m+1]-1 are member m's items.
 struct Plan {
   const int* start;
+  const int4* item;  // kinds with a tile shape (plan_tile): (member, k tile, j tile, chunk)
   int total;
-  int grid;  // workgroups launched (<= total)
-  int ich;   // i-planes per item of the tile streams (PK_RED, PK_CD*, PK_WALE)
+  int grid;  // workgroups launched by the grid-stride kinds (<= total)
+  int ich;   // i-planes per item
 };
 
 struct BView {
@@ -80,21 +84,42 @@ __host__ __device__ inline int red_blocks(int d0, int d1, int d2, int ich) {
 
 // Work-item counts per member for each kind of batched launch.
 enum PlanKind : int {
-  PK_CELLS = 0,     // 64x4 blocks over the real cells
+  PK_CELLS = 0,     // 64x4 tiles x ich planes over the real cells
   PK_RING,          // 64x4 blocks over real cells + 1 ring layer
   PK_RED,           // reduction tiles over the real cells
   PK_CD0,           // convdiff tiles, components u, v, w
   PK_CD1,
   PK_CD2,
-  PK_WALE,          // WALE tiles (8 x 32 (j, k) x ich planes) over the real cells;
-                    // also the three-component conv+diff passes
+  PK_MOM,           // 8 x 32 (j, k) tiles x ich planes over the real cells: the
+                    // three-component conv+diff passes
+  PK_STREAM,        // the same tiles, other chunks: WALE and calvel3_calmas
   PK_CDE,           // u's edge planes 0 and ni-2: 8 x 32 (j, k) tiles x 2
   PK_XG,            // w's cross-ghost cells of each real plane, 256 per item
   PK_MEMBER,        // one item per member
   PK_COP,           // 32-row blocks of the coarsest level's operator
-  PK_LCELLS0,       // 64x4 blocks over level-l real cells, l = 0 .. 7
+  PK_LCELLS0,       // 64x4 tiles over single planes of level l, l = 0 .. 7
   PK_COUNT = PK_LCELLS0 + BATCH_MAX_LEVELS
 };
+
+// The workgroup's entry of a plan with a table.  Nothing is searched or divided
+// before its loads: the grid-stride form's member search (a chain of six
+// dependent loads per 64 x 4 block) took half the time of a light field pass
+// (pp -= mean over 12.1 M cells: 75 us with it, 35 without).
+__device__ inline int4 plan_item(const Plan& P, int& w) {
+  w = xcd_linear(blockIdx.x, gridDim.x);
+  return P.item[w];
+}
+// f(member index, member, block) for every plane of the workgroup's item of a
+// 64 x 4 plan over n0(member) planes.
+template <class F>
+__device__ inline void item_planes(const Plan& P, const BView& V, const int* active, F&& f) {
+  int w;
+  const int4 it = plan_item(P, w);
+  if (active && !active[it.x]) return;  // uniform per workgroup
+  const MemDev& M = V.mem[it.x];
+  const int i1 = min(it.w * P.ich + P.ich, M.g.ni);
+  for (int i = it.w * P.ich; i < i1; ++i) f(it.x, M, Blk{it.y, it.z, i});
+}
 
 // How a level of every member relaxes: one workgroup per item (member, block
 // coordinates x, y, z) of a table made at creation.
@@ -147,6 +172,8 @@ int batch_wale(const Batch& B, const double* u, const double* v, const double* w
                hipStream_t s);
 int batch_checkdt(const Batch& B, const double* u, const double* v, const double* w,
                   const double* vis, double* out4, hipStream_t s);
+int batch_wale_checkdt(const Batch& B, const double* u, const double* v, const double* w,
+                       double* vis, double* out4, hipStream_t s);
 int batch_calvel3(const Batch& B, const double* us, const double* vs, const double* ws,
                   const double* p, double* u, double* v, double* w, double alpha,
                   const int* active, hipStream_t s);
@@ -154,7 +181,8 @@ int batch_calmas(const Batch& B, const double* u, const double* v, const double*
                  double* rmax, const int* active, hipStream_t s);
 int batch_calvel3_calmas(const Batch& B, const double* us, const double* vs, const double* ws,
                          const double* p, double* u, double* v, double* w, double* su,
-                         double* rmax, double alpha, const int* active, hipStream_t s);
+                         double* rmax, double alpha, float* r32, const int* active,
+                         hipStream_t s);
 int batch_add_ring(const Batch& B, double* p, const double* pp, const int* active,
                    hipStream_t s);
 int batch_convdiff(const Batch& B, int comp, const double* u, const double* v,

@@ -47,11 +47,31 @@ constexpr int64_t ALIGN = 32;  // elements: member arrays start on 256-byte (FP6
 
 int64_t align_up(int64_t x) { return (x + ALIGN - 1) / ALIGN * ALIGN; }
 
+// Chunks, j and k tiles of member M in a plan with an item table; false: a kind
+// without one.
+bool plan_tile(int kind, const MemDev& M, int ich, int t[3]) {
+  int tj = 4, tk = 64;
+  const int* n = M.ln[0];
+  if (kind == PK_MOM || kind == PK_STREAM) {
+    tj = 8;
+    tk = 32;
+  } else if (kind >= PK_LCELLS0 && kind < PK_LCELLS0 + BATCH_MAX_LEVELS) {
+    const int l = kind - PK_LCELLS0;
+    if (l >= M.nlev) return false;
+    n = M.ln[l];
+    ich = 1;
+  } else if (kind != PK_CELLS) {
+    return false;
+  }
+  t[0] = div_up(n[0], ich);
+  t[1] = div_up(n[1], tj);
+  t[2] = div_up(n[2], tk);
+  return true;
+}
+
 int member_count(int kind, const MemDev& M, int ich) {
   const int n0 = M.g.ni, n1 = M.g.nj, n2 = M.g.nk;
   switch (kind) {
-    case PK_CELLS:
-      return cells_blocks(n0, n1, n2);
     case PK_RING:
       return cells_blocks(n0 + 2, n1 + 2, n2 + 2);
     case PK_RED:
@@ -63,8 +83,6 @@ int member_count(int kind, const MemDev& M, int ich) {
       op_dims(kind - PK_CD0, n0, n1, n2, d0, d1, d2);
       return cd_tiles(d0, d1, d2, ich);
     }
-    case PK_WALE:
-      return cd_tiles(n0, n1, n2, ich);
     case PK_CDE:
       return ((n2 + 31) / 32) * ((n1 + 7) / 8) * (n0 - 1 > 1 ? 2 : (n0 - 1 > 0 ? 1 : 0));
     case PK_XG:
@@ -78,18 +96,16 @@ int member_count(int kind, const MemDev& M, int ich) {
     default:
       break;
   }
-  if (kind >= PK_LCELLS0 && kind < PK_LCELLS0 + BATCH_MAX_LEVELS) {
-    const int l = kind - PK_LCELLS0;
-    if (l >= M.nlev) return 0;
-    return cells_blocks(M.ln[l][0], M.ln[l][1], M.ln[l][2]);
-  }
-  return 0;
+  int t[3];
+  return plan_tile(kind, M, ich, t) ? t[0] * t[1] * t[2] : 0;
 }
 
 void batch_free(Batch* B) {
   if (!B) return;
   for (int k = 0; k < PK_COUNT; ++k)
     if (B->plan_mem[k]) (void)hipFree(B->plan_mem[k]);
+  for (int k = 0; k < PK_COUNT; ++k)
+    if (B->plan[k].item) (void)hipFree(const_cast<int4*>(B->plan[k].item));
   for (int l = 0; l < BATCH_MAX_LEVELS; ++l)
     if (B->relax[l].item) (void)hipFree(const_cast<int4*>(B->relax[l].item));
   if (B->bc_fill) (void)hipFree(B->bc_fill);
@@ -141,6 +157,14 @@ int create(const wf_member* mem, int nmem, int nlev, Batch** out) {
     M.dt = a.dt;
     M.ls = a.ls;
     M.rsum = 1.0 / (a.dx * a.dx) + 1.0 / (a.dy * a.dy) + 1.0 / (a.dz * a.dz);
+    const double h1[3] = {a.dx, a.dy, a.dz};
+    for (int d = 0; d < 3; ++d) {
+      M.r1[d] = 1.0 / h1[d];
+      M.r2[d] = 1.0 / (h1[d] * h1[d]);
+      M.r24[d] = 1.0 / (24.0 * h1[d]);
+      M.ir12[d] = 1.0 / (12.0 * h1[d] * h1[d]);
+    }
+    M.rdt = 1.0 / a.dt;
     M.seed = a.seed;
     M.nlev = nlev;
     for (int l = 0; l < nlev; ++l) {
@@ -165,7 +189,7 @@ int create(const wf_member* mem, int nmem, int nlev, Batch** out) {
     sum += cells_blocks(a.n0, a.n1, a.n2);
   }
   // i-planes per item of the streams, as the single-domain launches choose
-  // them: the momentum passes two workgroups per CU, the projection four
+  // them: the momentum passes three workgroups per CU, the projection four
   int nmax = 0;
   for (int m = 0; m < nmem; ++m) nmax = std::max(nmax, mem[m].n0);
   auto chunk = [&](int kind, const ChunkCost& C) {
@@ -175,11 +199,21 @@ int create(const wf_member* mem, int nmem, int nlev, Batch** out) {
       return w;
     });
   };
-  const int cd_ich = chunk(PK_WALE, ChunkCost{2, {2.05, 3.0}});
-  const int red_ich = chunk(PK_RED, ChunkCost{4, {1.1, 1.75, 2.75, 3.7}});
+  const ChunkCost proj{4, {1.1, 1.75, 2.75, 3.7}};
+  const int cd_ich = chunk(PK_MOM, ChunkCost{3, {2.05, 3.0, 4.15}});
+  const int red_ich = chunk(PK_RED, proj), stream_ich = chunk(PK_STREAM, proj);
+  // element passes: up to four planes per item while that leaves eight
+  // workgroups per CU
+  int el_ich = 1;
+  for (int ich : {2, 4}) {
+    int64_t w = 0;
+    for (int m = 0; m < nmem; ++m) w += member_count(PK_CELLS, B->mem_host[m], ich);
+    if (w >= 8 * 256) el_ich = ich;
+  }
   for (int m = 0; m < nmem; ++m) {
     B->mem_host[m].red0 = red;
-    red += red_blocks(mem[m].n0, mem[m].n1, mem[m].n2, red_ich);
+    red += std::max(red_blocks(mem[m].n0, mem[m].n1, mem[m].n2, red_ich),
+                    cd_tiles(mem[m].n0, mem[m].n1, mem[m].n2, stream_ich));
   }
   B->field_elems = foff;
   for (int l = 0; l < nlev; ++l) B->level_elems[l] = loff[l];
@@ -209,12 +243,26 @@ int create(const wf_member* mem, int nmem, int nlev, Batch** out) {
     return rc;
   }
   std::vector<int> start(nmem + 1);
+  std::vector<int4> items;
+  auto upload = [&](const int4** dst) {
+    void* p = nullptr;
+    if (fail(hipMalloc(&p, sizeof(int4) * items.size()))) return false;
+    *dst = (const int4*)p;
+    return !fail(hipMemcpy(p, items.data(), sizeof(int4) * items.size(), hipMemcpyHostToDevice));
+  };
   for (int k = 0; k < PK_COUNT; ++k) {
     start[0] = 0;
     Plan& P = B->plan[k];
-    P.ich = k == PK_RED ? red_ich : cd_ich;
-    for (int m = 0; m < nmem; ++m)
+    P.ich = k == PK_RED ? red_ich : k == PK_STREAM ? stream_ich : k == PK_CELLS ? el_ich : cd_ich;
+    items.clear();
+    for (int m = 0; m < nmem; ++m) {
       start[m + 1] = start[m] + member_count(k, B->mem_host[m], P.ich);
+      int t[3];
+      if (plan_tile(k, B->mem_host[m], P.ich, t))
+        for (int z = 0; z < t[0]; ++z)
+          for (int y = 0; y < t[1]; ++y)
+            for (int x = 0; x < t[2]; ++x) items.push_back(int4{m, x, y, z});
+    }
     P.total = start[nmem];
     // a persistent grid: at most 8 workgroups per CU, the most a CU holds
     P.grid = std::max(1, std::min(P.total, 8 * ncu));
@@ -225,23 +273,19 @@ int create(const wf_member* mem, int nmem, int nlev, Batch** out) {
       return rc;
     }
     P.start = B->plan_mem[k];
+    if (!items.empty() && !upload(&P.item)) {
+      batch_free(B);
+      return rc;
+    }
   }
   rc = batch_bc_init(*B);
   if (rc) {
     batch_free(B);
     return rc;
   }
-  std::vector<int4> items;
   for (int l = 0; l < nlev; ++l) {
-    BatchRelax& P = B->relax[l];
-    batch_relax_plan(B->mem_host, nmem, l, P, items);
-    void* p = nullptr;
-    if (fail(hipMalloc(&p, sizeof(int4) * items.size()))) {
-      batch_free(B);
-      return rc;
-    }
-    P.item = (const int4*)p;
-    if (fail(hipMemcpy(p, items.data(), sizeof(int4) * items.size(), hipMemcpyHostToDevice))) {
+    batch_relax_plan(B->mem_host, nmem, l, B->relax[l], items);
+    if (!upload(&B->relax[l].item)) {
       batch_free(B);
       return rc;
     }
@@ -302,6 +346,12 @@ int wf_batch_wale(wf_batch b, const double* u, const double* v, const double* w,
                   void* stream) {
   if (!ok(b) || !u || !v || !w || !vis) return WF_EINVAL;
   return batch_wale(B_(b), u, v, w, vis, (hipStream_t)stream);
+}
+
+int wf_batch_wale_checkdt(wf_batch b, const double* u, const double* v, const double* w,
+                          double* vis, double* out4, void* stream) {
+  if (!ok(b) || !u || !v || !w || !vis || !out4) return WF_EINVAL;
+  return batch_wale_checkdt(B_(b), u, v, w, vis, out4, (hipStream_t)stream);
 }
 
 int wf_batch_checkdt(wf_batch b, const double* u, const double* v, const double* w,
@@ -406,7 +456,7 @@ int wf_batch_calvel3_calmas(wf_batch b, const double* us, const double* vs, cons
                             const double* p, double* u, double* v, double* w, double* su,
                             double* rmax, double alpha, const int* active, void* stream) {
   if (!ok(b) || !us || !vs || !ws || !p || !u || !v || !w || !su || !rmax) return WF_EINVAL;
-  return batch_calvel3_calmas(B_(b), us, vs, ws, p, u, v, w, su, rmax, alpha, active,
+  return batch_calvel3_calmas(B_(b), us, vs, ws, p, u, v, w, su, rmax, alpha, nullptr, active,
                               (hipStream_t)stream);
 }
 

@@ -1239,6 +1239,19 @@ save_cross_ghosts_kernel(const double* __restrict__ w, double* __restrict__ wpre
   save_cross_body(w, wpre, g, blockIdx.x * blockDim.x + threadIdx.x, blockIdx.y);
 }
 
+// Coefficients of member M (as convdiff_launch forms them on the host).
+__device__ inline Coefs member_coefs(const MemDev& M, double alpha) {
+  Coefs K;
+  K.r24x = M.r24[0];
+  K.r24y = M.r24[1];
+  K.r24z = M.r24[2];
+  K.ir12x = M.ir12[0];
+  K.ir12y = M.ir12[1];
+  K.ir12z = M.ir12[2];
+  K.dta = M.dt * alpha;
+  return K;
+}
+
 // Ensemble form: a persistent grid over the (member, tile, chunk) items of
 // component C, chunks of P.ich planes.
 template <int C, bool SAVE>
@@ -1256,14 +1269,7 @@ batch_convdiff_kernel(BView V, Plan P, const double* __restrict__ u,
     op_dims(C, g.ni, g.nj, g.nk, d0, d1, d2);
     const Box3 b{g.npl, g.npl, g.npl, d0, d1, d2};
     const int kt = (d2 + TK - 1) / TK, jt = (d1 + TJ - 1) / TJ;
-    Coefs K;  // as convdiff_launch forms them on the host
-    K.r24x = 1.0 / (24.0 * M.dx);
-    K.r24y = 1.0 / (24.0 * M.dy);
-    K.r24z = 1.0 / (24.0 * M.dz);
-    K.ir12x = 1.0 / (12.0 * M.dx * M.dx);
-    K.ir12y = 1.0 / (12.0 * M.dy * M.dy);
-    K.ir12z = 1.0 / (12.0 * M.dz * M.dz);
-    K.dta = M.dt * alpha;
+    const Coefs K = member_coefs(M, alpha);
     convdiff_body<C, SAVE>(u + M.off, v + M.off, w + M.off, SAVE ? nullptr : coo + M.off,
                            vis + M.off, cstar + M.off, g, b, P.ich, q % kt,
                            (q / kt) % jt, q / (kt * jt), K, SAVE ? coo_save + M.off : nullptr);
@@ -1271,53 +1277,35 @@ batch_convdiff_kernel(BView V, Plan P, const double* __restrict__ u,
   }
 }
 
-// Coefficients of member M (as convdiff_launch forms them on the host).
-__device__ inline Coefs member_coefs(const MemDev& M, double alpha) {
-  Coefs K;
-  K.r24x = 1.0 / (24.0 * M.dx);
-  K.r24y = 1.0 / (24.0 * M.dy);
-  K.r24z = 1.0 / (24.0 * M.dz);
-  K.ir12x = 1.0 / (12.0 * M.dx * M.dx);
-  K.ir12y = 1.0 / (12.0 * M.dy * M.dy);
-  K.ir12z = 1.0 / (12.0 * M.dz * M.dz);
-  K.dta = M.dt * alpha;
-  return K;
-}
-
-// Ensemble forms of the three-component passes: a persistent grid over the
-// (member, tile, chunk) items of PK_WALE (8 x 32 tiles over the real cells,
-// chunks of P.ich planes), two workgroups per CU (the item loop's
-// member lookup pushes the first stage's form past 168 VGPRs as well).
+// Ensemble forms of the three-component passes: a workgroup per (member, tile,
+// chunk) item of PK_MOM, three workgroups per CU as in the single domain (12.1 M
+// cells: a grid-stride item loop, which left registers for two, 443 and 488 us;
+// here 433 and 426; rows of n + 6 doubles cost the rest of the single domain's
+// rate, whose rows are padded to whole cache lines).
 template <bool S2>
-__device__ inline void batch_convdiff3_items(BView V, Plan P, const double* u, const double* v,
-                                             const double* w, const double* vis,
-                                             const double* wpre, double* us, double* vs,
-                                             double* ws, double* uoo, double* voo, double* woo,
-                                             double alpha) {
-  for (int it = blockIdx.x; it < P.total; it += gridDim.x) {
-    const int m = member_of(P.start, V.nmem, it);
-    const int q = it - P.start[m];
-    const MemDev& M = V.mem[m];
-    const wf_grid g = M.g;
-    const int kt = (g.nk + TK - 1) / TK, jt = (g.nj + TJ - 1) / TJ;
-    convdiff3_body<S2>(u + M.off, v + M.off, w + M.off, vis + M.off, S2 ? wpre + M.off : nullptr,
-                       us + M.off, vs + M.off, ws + M.off, uoo + M.off, voo + M.off, woo + M.off,
-                       g, P.ich, q % kt, (q / kt) % jt, q / (kt * jt),
-                       member_coefs(M, alpha));
-    __syncthreads();  // LDS of this item is free for the next
-  }
+__device__ inline void batch_convdiff3_item(BView V, Plan P, const double* u, const double* v,
+                                            const double* w, const double* vis,
+                                            const double* wpre, double* us, double* vs,
+                                            double* ws, double* uoo, double* voo, double* woo,
+                                            double alpha) {
+  int q;
+  const int4 it = plan_item(P, q);
+  const MemDev& M = V.mem[it.x];
+  convdiff3_body<S2>(u + M.off, v + M.off, w + M.off, vis + M.off, S2 ? wpre + M.off : nullptr,
+                     us + M.off, vs + M.off, ws + M.off, uoo + M.off, voo + M.off, woo + M.off,
+                     M.g, P.ich, it.y, it.z, it.w, member_coefs(M, alpha));
 }
-__global__ void __launch_bounds__(256, 2)
+__global__ void __launch_bounds__(256, 3)
 batch_convdiff3_save_kernel(BView V, Plan P, const double* u, const double* v, const double* w,
                             const double* vis, double* us, double* vs, double* ws, double* uoo,
                             double* voo, double* woo, double alpha) {
-  batch_convdiff3_items<false>(V, P, u, v, w, vis, nullptr, us, vs, ws, uoo, voo, woo, alpha);
+  batch_convdiff3_item<false>(V, P, u, v, w, vis, nullptr, us, vs, ws, uoo, voo, woo, alpha);
 }
-__global__ void __launch_bounds__(256, 2)
+__global__ void __launch_bounds__(256, 3)
 batch_convdiff3_kernel(BView V, Plan P, const double* u, const double* v, const double* w,
                        const double* vis, const double* wpre, double* us, double* vs,
                        double* ws, double* uoo, double* voo, double* woo, double alpha) {
-  batch_convdiff3_items<true>(V, P, u, v, w, vis, wpre, us, vs, ws, uoo, voo, woo, alpha);
+  batch_convdiff3_item<true>(V, P, u, v, w, vis, wpre, us, vs, ws, uoo, voo, woo, alpha);
 }
 
 // u's planes 0 and ni-2 of every member (PK_CDE items: a tile and one of the
@@ -1362,12 +1350,12 @@ int batch_convdiff3(const Batch& B, const double* u, const double* v, const doub
                     const double* vis, const double* wpre, double* us, double* vs, double* ws,
                     double* uoo, double* voo, double* woo, double alpha, hipStream_t s) {
   using namespace cdv;
-  const Plan& P = B.plan[PK_WALE];
+  const Plan& P = B.plan[PK_MOM];
   if (wpre)
-    hipLaunchKernelGGL(batch_convdiff3_kernel, dim3(P.grid), dim3(NT), 0, s, B.view(), P, u, v,
+    hipLaunchKernelGGL(batch_convdiff3_kernel, dim3(P.total), dim3(NT), 0, s, B.view(), P, u, v,
                        w, vis, wpre, us, vs, ws, uoo, voo, woo, alpha);
   else
-    hipLaunchKernelGGL(batch_convdiff3_save_kernel, dim3(P.grid), dim3(NT), 0, s, B.view(), P, u,
+    hipLaunchKernelGGL(batch_convdiff3_save_kernel, dim3(P.total), dim3(NT), 0, s, B.view(), P, u,
                        v, w, vis, us, vs, ws, uoo, voo, woo, alpha);
   WF_LAUNCHED();
   return 0;

@@ -1807,59 +1807,42 @@ __device__ inline MgDev level_dev(const MemDev& M, int l) {
   d.s0 = (int64_t)(d.n1 + 2) * d.s1;
   return d;
 }
-// 1/h^2 of level l as the single-domain path forms it: (float)(1.0 / (h*h))
-// with h = spacing * 2^l.
-__device__ inline void level_coef(const MemDev& M, int l, float& c0, float& c1, float& c2) {
-  const double f = (double)(1 << l);
-  const double h0 = M.dx * f, h1 = M.dy * f, h2 = M.dz * f;
-  c0 = (float)(1.0 / (h0 * h0));
-  c1 = (float)(1.0 / (h1 * h1));
-  c2 = (float)(1.0 / (h2 * h2));
-}
-
-template <bool SYNC, class F>
-__device__ inline void mg_items(const Plan& P, const BView& V, const int* active, F&& f) {
-  for (int it = blockIdx.x; it < P.total; it += gridDim.x) {
-    const int m = member_of(P.start, V.nmem, it);
-    if (active && !active[m]) continue;
-    f(it - P.start[m], V.mem[m]);
-    if (SYNC) __syncthreads();
-  }
-}
-
 // restrict level lc-1 -> lc
 __global__ void __launch_bounds__(256)
 batch_restrict_kernel(BView V, Plan P, int lc, const float* phif, const float* rhsf,
                       float* phic, float* rhsc, const int* active) {
-  mg_items<false>(P, V, active, [&](int q, const MemDev& M) {
-    const MgDev f = level_dev(M, lc - 1), c = level_dev(M, lc);
-    float c0, c1, c2;
-    level_coef(M, lc - 1, c0, c1, c2);
-    restrict_body<float>(phif + M.loff[lc - 1], rhsf + M.loff[lc - 1], f, c0, c1, c2,
-                         phic + M.loff[lc], rhsc + M.loff[lc], c, cells_blk(q, c.n1, c.n2));
-  });
+  int w;
+  const int4 it = plan_item(P, w);
+  if (active && !active[it.x]) return;
+  const MemDev& M = V.mem[it.x];
+  const float* C = M.lc[lc - 1];
+  restrict_body<float>(phif + M.loff[lc - 1], rhsf + M.loff[lc - 1], level_dev(M, lc - 1), C[0],
+                       C[1], C[2], phic + M.loff[lc], rhsc + M.loff[lc], level_dev(M, lc),
+                       Blk{it.y, it.z, it.w});
 }
 
 // prolong level lf+1 -> lf
 __global__ void __launch_bounds__(256)
 batch_prolong_kernel(BView V, Plan P, int lf, const float* phic, float* phif,
                      const int* active) {
-  mg_items<false>(P, V, active, [&](int q, const MemDev& M) {
-    const MgDev c = level_dev(M, lf + 1), f = level_dev(M, lf);
-    prolong_body<float>(phic + M.loff[lf + 1], c, phif + M.loff[lf], f,
-                        cells_blk(q, f.n1, f.n2));
-  });
+  int w;
+  const int4 it = plan_item(P, w);
+  if (active && !active[it.x]) return;
+  const MemDev& M = V.mem[it.x];
+  prolong_body<float>(phic + M.loff[lf + 1], level_dev(M, lf + 1), phif + M.loff[lf],
+                      level_dev(M, lf), Blk{it.y, it.z, it.w});
 }
 // the same by 2 x 2 x 2 fine blocks (every member's level lf twice level
 // lf+1), items over the coarse cells
 __global__ void __launch_bounds__(256)
 batch_prolong8_kernel(BView V, Plan P, int lf, const float* phic, float* phif,
                       const int* active) {
-  mg_items<false>(P, V, active, [&](int q, const MemDev& M) {
-    const MgDev c = level_dev(M, lf + 1), f = level_dev(M, lf);
-    prolong8_body<float>(phic + M.loff[lf + 1], c, phif + M.loff[lf], f,
-                         cells_blk(q, c.n1, c.n2));
-  });
+  int w;
+  const int4 it = plan_item(P, w);
+  if (active && !active[it.x]) return;
+  const MemDev& M = V.mem[it.x];
+  prolong8_body<float>(phic + M.loff[lf + 1], level_dev(M, lf + 1), phif + M.loff[lf],
+                       level_dev(M, lf), Blk{it.y, it.z, it.w});
 }
 
 // Batched relaxation of level l: an item (member, block coordinates) per
@@ -2059,7 +2042,7 @@ int batch_vcycle(const Batch& B, float* const* phi_, float* const* rhs, float* c
   for (int l = 0; l < nlev; ++l) {
     if (l > 0) {
       const Plan& P = B.plan[PK_LCELLS0 + l];
-      hipLaunchKernelGGL(batch_restrict_kernel, dim3(P.grid), dim3(64, 4), 0, s, V, P, l,
+      hipLaunchKernelGGL(batch_restrict_kernel, dim3(P.total), dim3(64, 4), 0, s, V, P, l,
                          (const float*)phi[l - 1], (const float*)rhs[l - 1], phi[l], rhs[l],
                          active);
       WF_LAUNCHED();
@@ -2081,11 +2064,11 @@ int batch_vcycle(const Batch& B, float* const* phi_, float* const* rhs, float* c
         halves = halves && B.mem_host[m].ln[l][a] == 2 * B.mem_host[m].ln[l + 1][a];
     if (halves) {
       const Plan& P = B.plan[PK_LCELLS0 + l + 1];
-      hipLaunchKernelGGL(batch_prolong8_kernel, dim3(P.grid), dim3(64, 4), 0, s, V, P, l,
+      hipLaunchKernelGGL(batch_prolong8_kernel, dim3(P.total), dim3(64, 4), 0, s, V, P, l,
                          (const float*)phi[l + 1], phi[l], active);
     } else {
       const Plan& P = B.plan[PK_LCELLS0 + l];
-      hipLaunchKernelGGL(batch_prolong_kernel, dim3(P.grid), dim3(64, 4), 0, s, V, P, l,
+      hipLaunchKernelGGL(batch_prolong_kernel, dim3(P.total), dim3(64, 4), 0, s, V, P, l,
                          (const float*)phi[l + 1], phi[l], active);
     }
     WF_LAUNCHED();

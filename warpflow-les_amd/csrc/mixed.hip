@@ -420,24 +420,13 @@ __device__ inline MgDev level0_dev(const MemDev& M) {
   return d;
 }
 
-template <bool SYNC, class F>
-__device__ inline void mx_items(const Plan& P, const BView& V, const int* active, F&& f) {
-  for (int it = blockIdx.x; it < P.total; it += gridDim.x) {
-    const int m = member_of(P.start, V.nmem, it);
-    if (active && !active[m]) continue;
-    f(m, it - P.start[m], V.mem[m]);
-    if (SYNC) __syncthreads();
-  }
-}
-
 __global__ void __launch_bounds__(256)
 batch_defect_kernel(BView V, Plan P, const double* su, const double* pp, float* rhs0,
                     const int* active) {
-  mx_items<false>(P, V, active, [&](int, int q, const MemDev& M) {
+  item_planes(P, V, active, [&](int, const MemDev& M, Blk B) {
     const wf_grid& g = M.g;
     defect_body(su + M.off, pp ? pp + M.off : nullptr, g, rhs0 + M.loff[0], level0_dev(M),
-                1.0 / (M.dx * M.dx), 1.0 / (M.dy * M.dy), 1.0 / (M.dz * M.dz), nullptr,
-                nullptr, cells_blk(q, g.nj, g.nk));
+                M.r2[0], M.r2[1], M.r2[2], nullptr, nullptr, B);
   });
 }
 
@@ -461,25 +450,24 @@ __device__ inline void assign_defect_body(const double* __restrict__ b, double* 
 __global__ void __launch_bounds__(256)
 batch_assign_defect_kernel(BView V, Plan P, const double* su, double* pp, const float* phi0,
                            float* rhs0, const int* active) {
-  mx_items<false>(P, V, active, [&](int, int q, const MemDev& M) {
-    const wf_grid& g = M.g;
-    assign_defect_body(su + M.off, pp + M.off, g, phi0 + M.loff[0], rhs0 + M.loff[0],
-                       level0_dev(M), 1.0 / (M.dx * M.dx), 1.0 / (M.dy * M.dy),
-                       1.0 / (M.dz * M.dz), cells_blk(q, g.nj, g.nk));
+  item_planes(P, V, active, [&](int, const MemDev& M, Blk B) {
+    assign_defect_body(su + M.off, pp + M.off, M.g, phi0 + M.loff[0], rhs0 + M.loff[0],
+                       level0_dev(M), M.r2[0], M.r2[1], M.r2[2], B);
   });
 }
 
 __global__ void __launch_bounds__(256)
 batch_update_kernel(BView V, Plan P, double* pp, const float* phi0, const int* active) {
-  mx_items<false>(P, V, active, [&](int, int q, const MemDev& M) {
-    update_body(pp + M.off, M.g, phi0 + M.loff[0], level0_dev(M), cells_blk(q, M.g.nj, M.g.nk));
+  item_planes(P, V, active, [&](int, const MemDev& M, Blk B) {
+    update_body(pp + M.off, M.g, phi0 + M.loff[0], level0_dev(M), B);
   });
 }
 
 __global__ void __launch_bounds__(256)
 batch_partials_kernel(BView V, Plan P, const double* f, double* part, const int* active) {
-  mx_items<true>(P, V, active, [&](int, int q, const MemDev& M) {
-    field_partials_body(f + M.off, M.g, part + M.sum0, cells_blk(q, M.g.nj, M.g.nk));
+  item_planes(P, V, active, [&](int, const MemDev& M, Blk B) {
+    field_partials_body(f + M.off, M.g, part + M.sum0, B);
+    __syncthreads();
   });
 }
 
@@ -495,8 +483,8 @@ batch_sum_fold_kernel(BView V, const double* part, double* out, const int* activ
 
 __global__ void __launch_bounds__(256)
 batch_shift_kernel(BView V, Plan P, double* pp, const double* mean, const int* active) {
-  mx_items<false>(P, V, active, [&](int m, int q, const MemDev& M) {
-    shift_body(pp + M.off, M.g, mean + m, cells_blk(q, M.g.nj, M.g.nk));
+  item_planes(P, V, active, [&](int m, const MemDev& M, Blk B) {
+    shift_body(pp + M.off, M.g, mean + m, B);
   });
 }
 
@@ -534,7 +522,7 @@ int batch_mg_mixed(const Batch& B, float* const* phi, float* const* rhs, float* 
   bool defect_formed = false;  // the fused first update formed this cycle's defect
   for (int c = 0; c < ncycles; ++c) {
     if (!defect_formed) {
-      hipLaunchKernelGGL(batch_defect_kernel, dim3(P.grid), dim3(64, 4), 0, s, V, P, su,
+      hipLaunchKernelGGL(batch_defect_kernel, dim3(P.total), dim3(64, 4), 0, s, V, P, su,
                          c == 0 ? (const double*)nullptr : (const double*)pp, rhs[0], active);
       WF_LAUNCHED();
     }
@@ -550,23 +538,23 @@ int batch_mg_mixed(const Batch& B, float* const* phi, float* const* rhs, float* 
     if (r) return r;
     if (c == 0 && ncycles > 1) {
       // pp = 0 + e and the second cycle's defect in one pass
-      hipLaunchKernelGGL(batch_assign_defect_kernel, dim3(P.grid), dim3(64, 4), 0, s, V, P, su,
+      hipLaunchKernelGGL(batch_assign_defect_kernel, dim3(P.total), dim3(64, 4), 0, s, V, P, su,
                          pp, (const float*)phi[0], rhs[0], active);
       defect_formed = true;
     } else {
-      hipLaunchKernelGGL(batch_update_kernel, dim3(P.grid), dim3(64, 4), 0, s, V, P, pp,
+      hipLaunchKernelGGL(batch_update_kernel, dim3(P.total), dim3(64, 4), 0, s, V, P, pp,
                          (const float*)phi[0], active);
     }
     WF_LAUNCHED();
   }
   if (flags & MIX_RESULT_MEAN) {
-    hipLaunchKernelGGL(batch_partials_kernel, dim3(P.grid), dim3(64, 4), 0, s, V, P,
+    hipLaunchKernelGGL(batch_partials_kernel, dim3(P.total), dim3(64, 4), 0, s, V, P,
                        (const double*)pp, B.sum_part, active);
     WF_LAUNCHED();
     hipLaunchKernelGGL(batch_sum_fold_kernel, dim3(B.nmem), dim3(1024), 0, s, V,
                        (const double*)B.sum_part, B.scal, active);
     WF_LAUNCHED();
-    hipLaunchKernelGGL(batch_shift_kernel, dim3(P.grid), dim3(64, 4), 0, s, V, P, pp,
+    hipLaunchKernelGGL(batch_shift_kernel, dim3(P.total), dim3(64, 4), 0, s, V, P, pp,
                        (const double*)B.scal, active);
     WF_LAUNCHED();
   }

@@ -600,11 +600,11 @@ constexpr int WS_NL = (WS_RN + 255) / 256;  // staged values per thread per fiel
 
 // CHK: the checkdt reductions of the same cells in the same pass (max |u|,
 // |v|, |w| and min dtvisc with the vis read before it is overwritten), from
-// the values staged for WALE, into part[q * RED_MAX_BLOCKS + slot].
+// the values staged for WALE, into part[q * stride + slot].
 struct ChkArgs {
   double dx, dy, dz, rsum;  // with the rdx, rdy, rdz of the WALE gradients
   double* part;
-  int slot;
+  int stride, slot;
 };
 template <bool CHK = false>
 __device__ inline void wale_stream_body(const double* __restrict__ u,
@@ -620,10 +620,10 @@ __device__ inline void wale_stream_body(const double* __restrict__ u,
   const int i0 = chunk * ich, i1 = min(i0 + ich, b.d0);
   if (i0 >= i1) {  // uniform per workgroup
     if (CHK && tid == 0) {
-      ck.part[0 * RED_MAX_BLOCKS + ck.slot] = 0.0;
-      ck.part[1 * RED_MAX_BLOCKS + ck.slot] = 0.0;
-      ck.part[2 * RED_MAX_BLOCKS + ck.slot] = 0.0;
-      ck.part[3 * RED_MAX_BLOCKS + ck.slot] = 1.0e10;
+      ck.part[0 * ck.stride + ck.slot] = 0.0;
+      ck.part[1 * ck.stride + ck.slot] = 0.0;
+      ck.part[2 * ck.stride + ck.slot] = 0.0;
+      ck.part[3 * ck.stride + ck.slot] = 1.0e10;
     }
     return;
   }
@@ -727,10 +727,10 @@ __device__ inline void wale_stream_body(const double* __restrict__ u,
     __syncthreads();
     xmax = block_max(xmax);
     if (tid == 0) {
-      ck.part[0 * RED_MAX_BLOCKS + ck.slot] = mu;
-      ck.part[1 * RED_MAX_BLOCKS + ck.slot] = mv;
-      ck.part[2 * RED_MAX_BLOCKS + ck.slot] = mw;
-      ck.part[3 * RED_MAX_BLOCKS + ck.slot] = dtvisc_of_max(xmax);
+      ck.part[0 * ck.stride + ck.slot] = mu;
+      ck.part[1 * ck.stride + ck.slot] = mv;
+      ck.part[2 * ck.stride + ck.slot] = mw;
+      ck.part[3 * ck.stride + ck.slot] = dtvisc_of_max(xmax);
     }
   }
 }
@@ -756,7 +756,7 @@ wale_checkdt_kernel(const double* __restrict__ u, const double* __restrict__ v,
   const int L = xcd_linear(blockIdx.x + blockIdx.y * gridDim.x, nb);
   wale_stream_body<true>(u, v, w, vis, g, b, ich, L % kt, (L / kt) % jt, L / (kt * jt), rdx,
                          rdy, rdz, rrey, ls,
-                         ChkArgs{dx, dy, dz, rsum, g_red_part,
+                         ChkArgs{dx, dy, dz, rsum, g_red_part, RED_MAX_BLOCKS,
                                  (int)(blockIdx.x + blockIdx.y * gridDim.x)});
 }
 
@@ -909,11 +909,12 @@ noise_kernel(double* __restrict__ u, double* __restrict__ v, double* __restrict_
 }
 
 // ---------------------------------------------------------------------------
-// Batched (ensemble) kernels: a persistent grid walks the work items of a
-// plan; each item is one block of one member, run through the same body as
-// the single-domain kernel on that member's arrays.  Members whose `active`
-// flag is 0 are skipped.  SYNC: a barrier after every item, for bodies that
-// use LDS.
+// Batched (ensemble) kernels: each item of a plan is one block of one member,
+// run through the same body as the single-domain kernel on that member's
+// arrays: a workgroup per table entry (item_planes, plan_item) or, for the
+// kinds without a table, a persistent grid that walks the items.  Members whose
+// `active` flag is 0 are skipped.  SYNC: a barrier after every item, for bodies
+// that use LDS.
 // ---------------------------------------------------------------------------
 template <bool SYNC, class F>
 __device__ inline void for_items(const Plan& P, const BView& V, const int* active, F&& f) {
@@ -931,41 +932,39 @@ __device__ inline Box3 cells_box(const wf_grid& g) {
 
 __global__ void __launch_bounds__(256)
 batch_noise_kernel(BView V, Plan P, double* u, double* v, double* w) {
-  for_items<false>(P, V, nullptr, [&](int, int q, const MemDev& M) {
-    const Box3 b = cells_box(M.g);
-    noise_body(u + M.off, v + M.off, w + M.off, M.noise, M.seed, M.g, b,
-               cells_blk(q, b.d1, b.d2));
+  item_planes(P, V, nullptr, [&](int, const MemDev& M, Blk B) {
+    noise_body(u + M.off, v + M.off, w + M.off, M.noise, M.seed, M.g, cells_box(M.g), B);
   });
 }
 
 __global__ void __launch_bounds__(256) batch_fill_vis_kernel(BView V, Plan P, double* vis) {
-  for_items<false>(P, V, nullptr, [&](int, int q, const MemDev& M) {
-    const Box3 b = cells_box(M.g);
-    fill_box_body(vis + M.off, M.rey, M.g, b, cells_blk(q, b.d1, b.d2));
+  item_planes(P, V, nullptr, [&](int, const MemDev& M, Blk B) {
+    fill_box_body(vis + M.off, M.rey, M.g, cells_box(M.g), B);
   });
 }
 
+// WALE over the stream items, CHK: with the checkdt partials of the same cells
+// (one pass over u, v, w: 12.1 M cells, 283 us as two passes, 190 as one).
+template <bool CHK>
 __global__ void __launch_bounds__(256)
 batch_wale_kernel(BView V, Plan P, const double* u, const double* v, const double* w,
-                  double* vis) {
-  for_items<true>(P, V, nullptr, [&](int, int q, const MemDev& M) {
-    const Box3 b = cells_box(M.g);
-    const int kt = (b.d2 + WS_TK - 1) / WS_TK, jt = (b.d1 + WS_TJ - 1) / WS_TJ;
-    wale_stream_body(u + M.off, v + M.off, w + M.off, vis + M.off, M.g, b, P.ich, q % kt,
-                     (q / kt) % jt, q / (kt * jt), 1.0 / M.dx, 1.0 / M.dy, 1.0 / M.dz, M.rey,
-                     M.ls);
-  });
+                  double* vis, double* part, int stride) {
+  int q;
+  const int4 it = plan_item(P, q);
+  const MemDev& M = V.mem[it.x];
+  wale_stream_body<CHK>(u + M.off, v + M.off, w + M.off, vis + M.off, M.g, cells_box(M.g), P.ich,
+                        it.y, it.z, it.w, M.r1[0], M.r1[1], M.r1[2], M.rey, M.ls,
+                        ChkArgs{M.dx, M.dy, M.dz, M.rsum, part, stride,
+                                M.red0 + q - P.start[it.x]});
 }
 
 __global__ void __launch_bounds__(256)
 batch_calvel3_kernel(BView V, Plan P, const double* us, const double* vs, const double* ws,
                      const double* p, double* u, double* v, double* w, double alpha,
                      const int* active) {
-  for_items<false>(P, V, active, [&](int, int q, const MemDev& M) {
-    const Box3 b = cells_box(M.g);
+  item_planes(P, V, active, [&](int, const MemDev& M, Blk B) {
     calvel3_body(us + M.off, vs + M.off, ws + M.off, p + M.off, u + M.off, v + M.off,
-                 w + M.off, M.g, b, cells_blk(q, b.d1, b.d2), 1.0 / M.dx, 1.0 / M.dy, 1.0 / M.dz,
-                 M.dt * alpha);
+                 w + M.off, M.g, cells_box(M.g), B, M.r1[0], M.r1[1], M.r1[2], M.dt * alpha);
   });
 }
 
@@ -988,24 +987,26 @@ batch_calmas_kernel(BView V, Plan P, const double* u, const double* v, const dou
   });
 }
 
-// The fused calvel/calmas pass per member on the reduction items (64 x 4
-// (k, j) tiles x P.ich planes), so its partials fill the slots
-// batch_red_fold_kernel folds, as batch_calmas_kernel's do.
+// The fused calvel/calmas pass per member, the single-domain tiles and load
+// depth on the stream items (12.1 M cells 250 us, 3.1 TB/s: rows of n + 6
+// doubles start anywhere in a cache line; 0.5 M cells 15.6 -> 13.3 us against
+// the 64 x 4 tiles of an item loop); r32 (nullable): su as level 0's FP32
+// right-hand side as well.
 __global__ void __launch_bounds__(256)
 batch_calvel3_calmas_kernel(BView V, Plan P, const double* us, const double* vs,
                             const double* ws, const double* p, double* u, double* v, double* w,
-                            double* su, double* part, double alpha, const int* active) {
-  for_items<true>(P, V, active, [&](int, int q, const MemDev& M) {
-    const wf_grid& g = M.g;
-    const int kt = (g.nk + 63) / 64, jt = (g.nj + 3) / 4;
-    const pj::Consts K{1.0 / M.dx, 1.0 / M.dy, 1.0 / M.dz, M.dt * alpha,
-                       1.0 / (24.0 * M.dx), 1.0 / (24.0 * M.dy), 1.0 / (24.0 * M.dz),
-                       1.0 / M.dt, M.dx, M.dy, M.dz};
-    const double r = calvel3_calmas_body<4, 64>(
-        us + M.off, vs + M.off, ws + M.off, p + M.off, u + M.off, v + M.off, w + M.off,
-        su + M.off, g, P.ich, q % kt, (q / kt) % jt, q / (kt * jt), K);
-    if (threadIdx.x == 0) part[M.red0 + q] = r;
-  });
+                            double* su, double* part, double alpha, float* r32,
+                            const int* active) {
+  int q;
+  const int4 it = plan_item(P, q);
+  if (active && !active[it.x]) return;  // uniform per workgroup
+  const MemDev& M = V.mem[it.x];
+  const pj::Consts K{M.r1[0], M.r1[1], M.r1[2], M.dt * alpha, M.r24[0], M.r24[1], M.r24[2],
+                     M.rdt, M.dx, M.dy, M.dz};
+  const double r = calvel3_calmas_body<PJ_TJ, PJ_TK, true, 2>(
+      us + M.off, vs + M.off, ws + M.off, p + M.off, u + M.off, v + M.off, w + M.off,
+      su + M.off, M.g, P.ich, it.y, it.z, it.w, K, r32 ? r32 + M.loff[0] : nullptr);
+  if (threadIdx.x == 0) part[M.red0 + q - P.start[it.x]] = r;
 }
 
 __global__ void __launch_bounds__(256)
@@ -1019,7 +1020,7 @@ batch_checkdt_kernel(BView V, Plan P, const double* u, const double* v, const do
   });
 }
 
-// One workgroup per member folds its reduction partials: out[m*nq + q] for
+// One workgroup per member folds its reduction partials, one per item of P: out[m*nq + q] for
 // quantity q (bit q of min_mask: min, else max).
 __global__ void __launch_bounds__(1024)
 batch_red_fold_kernel(BView V, Plan P, const double* part, int stride, int nq, int min_mask,
@@ -1027,7 +1028,7 @@ batch_red_fold_kernel(BView V, Plan P, const double* part, int stride, int nq, i
   const int m = blockIdx.x;
   if (active && !active[m]) return;  // uniform per workgroup
   const MemDev& M = V.mem[m];
-  const int n = P.start[m + 1] - P.start[m];  // the member's PK_RED items
+  const int n = P.start[m + 1] - P.start[m];
   __shared__ double sh[16];
   const int t = threadIdx.x;
   for (int q = 0; q < nq; ++q) {
@@ -1051,23 +1052,35 @@ batch_red_fold_kernel(BView V, Plan P, const double* part, int stride, int nq, i
 
 int batch_noise(const Batch& B, double* u, double* v, double* w, hipStream_t s) {
   const Plan& P = B.plan[PK_CELLS];
-  hipLaunchKernelGGL(batch_noise_kernel, dim3(P.grid), box_block(), 0, s, B.view(), P, u, v, w);
+  hipLaunchKernelGGL(batch_noise_kernel, dim3(P.total), box_block(), 0, s, B.view(), P, u, v, w);
   WF_LAUNCHED();
   return 0;
 }
 
 int batch_fill_vis(const Batch& B, double* vis, hipStream_t s) {
   const Plan& P = B.plan[PK_CELLS];
-  hipLaunchKernelGGL(batch_fill_vis_kernel, dim3(P.grid), box_block(), 0, s, B.view(), P, vis);
+  hipLaunchKernelGGL(batch_fill_vis_kernel, dim3(P.total), box_block(), 0, s, B.view(), P, vis);
   WF_LAUNCHED();
   return 0;
 }
 
 int batch_wale(const Batch& B, const double* u, const double* v, const double* w, double* vis,
                hipStream_t s) {
-  const Plan& P = B.plan[PK_WALE];
-  hipLaunchKernelGGL(batch_wale_kernel, dim3(P.grid), dim3(256), 0, s, B.view(), P, u, v, w,
-                     vis);
+  const Plan& P = B.plan[PK_STREAM];
+  hipLaunchKernelGGL(batch_wale_kernel<false>, dim3(P.total), dim3(256), 0, s, B.view(), P, u, v,
+                     w, vis, (double*)nullptr, 0);
+  WF_LAUNCHED();
+  return 0;
+}
+
+int batch_wale_checkdt(const Batch& B, const double* u, const double* v, const double* w,
+                       double* vis, double* out4, hipStream_t s) {
+  const Plan& P = B.plan[PK_STREAM];
+  hipLaunchKernelGGL(batch_wale_kernel<true>, dim3(P.total), dim3(256), 0, s, B.view(), P, u, v,
+                     w, vis, B.red_part, B.nred);
+  WF_LAUNCHED();
+  hipLaunchKernelGGL(batch_red_fold_kernel, dim3(B.nmem), dim3(1024), 0, s, B.view(), P,
+                     (const double*)B.red_part, B.nred, 4, 8, out4, (const int*)nullptr);
   WF_LAUNCHED();
   return 0;
 }
@@ -1076,7 +1089,7 @@ int batch_calvel3(const Batch& B, const double* us, const double* vs, const doub
                   const double* p, double* u, double* v, double* w, double alpha,
                   const int* active, hipStream_t s) {
   const Plan& P = B.plan[PK_CELLS];
-  hipLaunchKernelGGL(batch_calvel3_kernel, dim3(P.grid), box_block(), 0, s, B.view(), P, us, vs,
+  hipLaunchKernelGGL(batch_calvel3_kernel, dim3(P.total), box_block(), 0, s, B.view(), P, us, vs,
                      ws, p, u, v, w, alpha, active);
   WF_LAUNCHED();
   return 0;
@@ -1105,10 +1118,11 @@ int batch_calmas(const Batch& B, const double* u, const double* v, const double*
 
 int batch_calvel3_calmas(const Batch& B, const double* us, const double* vs, const double* ws,
                          const double* p, double* u, double* v, double* w, double* su,
-                         double* rmax, double alpha, const int* active, hipStream_t s) {
-  const Plan& P = B.plan[PK_RED];
-  hipLaunchKernelGGL(batch_calvel3_calmas_kernel, dim3(P.grid), dim3(256), 0, s, B.view(), P, us,
-                     vs, ws, p, u, v, w, su, B.red_part, alpha, active);
+                         double* rmax, double alpha, float* r32, const int* active,
+                         hipStream_t s) {
+  const Plan& P = B.plan[PK_STREAM];
+  hipLaunchKernelGGL(batch_calvel3_calmas_kernel, dim3(P.total), dim3(256), 0, s, B.view(), P, us,
+                     vs, ws, p, u, v, w, su, B.red_part, alpha, r32, active);
   WF_LAUNCHED();
   hipLaunchKernelGGL(batch_red_fold_kernel, dim3(B.nmem), dim3(1024), 0, s, B.view(), P,
                      (const double*)B.red_part, B.nred, 1, 0, rmax, active);

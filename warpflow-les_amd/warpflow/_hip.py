@@ -71,6 +71,7 @@ _SIGS = {
     "wf_batch_init_noise": [_P, _P, _P, _P, _P],
     "wf_batch_fill_vis": [_P, _P, _P],
     "wf_batch_wale": [_P, _P, _P, _P, _P, _P],
+    "wf_batch_wale_checkdt": [_P, _P, _P, _P, _P, _P, _P],
     "wf_batch_checkdt": [_P, _P, _P, _P, _P, _P, _P],
     "wf_batch_bc_fill": [_P, _P, _I, _P, _P],
     "wf_batch_convdiff": [_P, _I, _P, _P, _P, _P, _P, _P, C.c_double, _P],

@@ -214,14 +214,15 @@ class Ensemble:
     def _part_a_head(self):
         """compute_dt, SGS and both RK2 stages (the first storing uoo, voo, woo)."""
         P, s = self.pool, self.stream
-        self._call("wf_batch_checkdt", P["u"].ptr, P["v"].ptr, P["w"].ptr, P["vis"].ptr,
-                   self.out4.ptr, s)
         # no copies u -> uoo: the first stage's conv+diff stores them on the
         # operator boxes (the cells the second stage reads)
         if self.sgs:
-            self._call("wf_batch_wale", P["u"].ptr, P["v"].ptr, P["w"].ptr, P["vis"].ptr, s)
+            self._call("wf_batch_wale_checkdt", P["u"].ptr, P["v"].ptr, P["w"].ptr,
+                       P["vis"].ptr, self.out4.ptr, s)
             self._fill("vis")
         else:
+            self._call("wf_batch_checkdt", P["u"].ptr, P["v"].ptr, P["w"].ptr, P["vis"].ptr,
+                       self.out4.ptr, s)
             self._call("wf_batch_fill_vis", P["vis"].ptr, s)
         for stage, alpha in enumerate(ALFARK):
             if stage == 0:
