@@ -571,6 +571,19 @@ int wf_batch_mg_solve_mixed(wf_batch b, float* const* phi, float* const* rhs, fl
                             const float* cop, const double* su, double* pp, int ncycles,
                             int n_pre, int n_post, int n_coarse, int flags, const int* active,
                             void* stream);
+/* wf_batch_mg_solve_mixed with level 0's right-hand side already (float)su (as
+ * wf_batch_project_test leaves it), then wf_batch_add_ring: p += pp. */
+int wf_batch_mg_correct(wf_batch b, float* const* phi, float* const* rhs, float* const* tmp,
+                        const float* cop, const double* su, double* pp, double* p, int ncycles,
+                        int n_pre, int n_post, int n_coarse, int flags, const int* active,
+                        void* stream);
+/* Outer test of iteration it >= 1: wf_batch_calvel3_calmas, which also leaves
+ * (float)su in level 0's right-hand side rhs0, and wf_batch_project_mask.  it = 1
+ * starts the loop: every member takes part and becomes active (or leaves). */
+int wf_batch_project_test(wf_batch b, const double* us, const double* vs, const double* ws,
+                          const double* p, double* u, double* v, double* w, double* su,
+                          float* rhs0, double* rmax, double alpha, double eps, int it,
+                          int* active, int* iters, int* status, void* stream);
 /* Outer-loop bookkeeping of solver.py:185-197 for iteration it: each active
  * member records iters[m] = it, then leaves when rmax[m] < eps and it > 1;
  * rmax[m] > 10 sets status[m] = 1 (diverged) and leaves. */

@@ -40,6 +40,8 @@ struct MemDev {
   int sum0;      // first sum-partial slot of this member
 };
 
+constexpr int BATCH_ICH = 4;  // most planes per item of the element passes
+
 // A work-item list: start[m] .. start[m+1]-1 are member m's items.
 struct Plan {
   const int* start;
@@ -53,6 +55,15 @@ struct BView {
   const MemDev* mem;
   int nmem;
 };
+
+// Member m's part of the outer loop's break test (solver.py:185-197).
+__device__ inline void loop_test(int m, double r, double eps, int it, int* __restrict__ active,
+                                 int* __restrict__ iters, int* __restrict__ status) {
+  iters[m] = it;
+  const bool diverged = !(r <= 10.0), leaves = diverged || (r < eps && it > 1);
+  if (diverged && !(r < eps && it > 1)) status[m] = 1;
+  active[m] = leaves ? 0 : 1;
+}
 
 // Largest m with start[m] <= w (start[0] = 0, start[nmem] = total > w).
 __device__ inline int member_of(const int* __restrict__ start, int nmem, int w) {
@@ -165,6 +176,16 @@ __host__ __device__ inline void op_dims(int c, int n0, int n1, int n2, int& d0, 
   d1 = n1 - (c == 1);
   d2 = n2 - (c == 2);
 }
+// The outer loop's break test of iteration it (> 0) in the projection's fold:
+// each member that takes part records iters[m] = it and leaves the loop when
+// rmax[m] < eps and it > 1, or, with status[m] = 1, when rmax[m] > 10 or NaN.
+// it = 1 starts the loop: every member takes part.
+struct BatchTest {
+  int it = 0;
+  double eps = 0.0;
+  int *active = nullptr, *iters = nullptr, *status = nullptr;
+};
+
 // Batched launchers, one per source file (argument checks done by the C ABI).
 int batch_noise(const Batch& B, double* u, double* v, double* w, hipStream_t s);
 int batch_fill_vis(const Batch& B, double* vis, hipStream_t s);
@@ -182,7 +203,7 @@ int batch_calmas(const Batch& B, const double* u, const double* v, const double*
 int batch_calvel3_calmas(const Batch& B, const double* us, const double* vs, const double* ws,
                          const double* p, double* u, double* v, double* w, double* su,
                          double* rmax, double alpha, float* r32, const int* active,
-                         hipStream_t s);
+                         hipStream_t s, const BatchTest& test = BatchTest{});
 int batch_add_ring(const Batch& B, double* p, const double* pp, const int* active,
                    hipStream_t s);
 int batch_convdiff(const Batch& B, int comp, const double* u, const double* v,
@@ -211,5 +232,9 @@ void batch_relax_plan(const MemDev* mem, int nmem, int l, BatchRelax& P,
 int batch_mg_mixed(const Batch& B, float* const* phi, float* const* rhs, float* const* tmp,
                    const float* cop, const double* su, double* pp, int ncycles, int npre,
                    int npost, int ncoarse, int flags, const int* active, hipStream_t s);
+int batch_mg_correct(const Batch& B, float* const* phi, float* const* rhs, float* const* tmp,
+                     const float* cop, const double* su, double* pp, double* p, int ncycles,
+                     int npre, int npost, int ncoarse, int flags, const int* active,
+                     hipStream_t s);
 
 }  // namespace wf

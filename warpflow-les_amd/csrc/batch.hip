@@ -22,14 +22,7 @@ __global__ void batch_mask_kernel(int nmem, const double* __restrict__ rmax, dou
                                   int* __restrict__ status) {
   const int m = blockIdx.x * blockDim.x + threadIdx.x;
   if (m >= nmem || !active[m]) return;
-  iters[m] = it;
-  const double r = rmax[m];
-  if (r < eps && it > 1) {
-    active[m] = 0;
-  } else if (!(r <= 10.0)) {
-    active[m] = 0;
-    status[m] = 1;
-  }
+  loop_test(m, rmax[m], eps, it, active, iters, status);
 }
 
 __global__ void batch_set_int_kernel(int* __restrict__ p, int n, int v) {
@@ -205,7 +198,7 @@ int create(const wf_member* mem, int nmem, int nlev, Batch** out) {
   // element passes: up to four planes per item while that leaves eight
   // workgroups per CU
   int el_ich = 1;
-  for (int ich : {2, 4}) {
+  for (int ich = 2; ich <= BATCH_ICH; ich *= 2) {
     int64_t w = 0;
     for (int m = 0; m < nmem; ++m) w += member_count(PK_CELLS, B->mem_host[m], ich);
     if (w >= 8 * 256) el_ich = ich;
@@ -296,6 +289,19 @@ int create(const wf_member* mem, int nmem, int nlev, Batch** out) {
 
 bool ok(wf_batch b) { return b != nullptr; }
 Batch& B_(wf_batch b) { return *reinterpret_cast<Batch*>(b); }
+
+bool mg_args_ok(wf_batch b, float* const* phi, float* const* rhs, float* const* tmp,
+                const float* cop, int ncycles, int n_pre, int n_post, int n_coarse, int flags) {
+  if (!ok(b) || !phi || !rhs || !tmp || ncycles < 0 || n_pre < 0 || n_post < 0 || n_coarse < 0 ||
+      (flags & ~2))
+    return false;
+  const Batch& B = B_(b);
+  for (int l = 0; l < B.nlev; ++l)
+    if (!phi[l] || !rhs[l] || !tmp[l]) return false;
+  for (int m = 0; cop && m < B.nmem; ++m)
+    if (B.mem_host[m].coff < 0) return false;
+  return true;
+}
 
 }  // namespace
 
@@ -470,17 +476,33 @@ int wf_batch_mg_solve_mixed(wf_batch b, float* const* phi, float* const* rhs, fl
                             const float* cop, const double* su, double* pp, int ncycles,
                             int n_pre, int n_post, int n_coarse, int flags, const int* active,
                             void* stream) {
-  if (!ok(b) || !phi || !rhs || !tmp || !su || !pp || ncycles < 0 || n_pre < 0 ||
-      n_post < 0 || n_coarse < 0 || (flags & ~2))
+  if (!mg_args_ok(b, phi, rhs, tmp, cop, ncycles, n_pre, n_post, n_coarse, flags) || !su || !pp)
     return WF_EINVAL;
-  const Batch& B = B_(b);
-  for (int l = 0; l < B.nlev; ++l)
-    if (!phi[l] || !rhs[l] || !tmp[l]) return WF_EINVAL;
-  if (cop)
-    for (int m = 0; m < B.nmem; ++m)
-      if (B.mem_host[m].coff < 0) return WF_EINVAL;
-  return batch_mg_mixed(B, phi, rhs, tmp, cop, su, pp, ncycles, n_pre, n_post, n_coarse, flags,
+  return batch_mg_mixed(B_(b), phi, rhs, tmp, cop, su, pp, ncycles, n_pre, n_post, n_coarse, flags,
                         active, (hipStream_t)stream);
+}
+
+int wf_batch_mg_correct(wf_batch b, float* const* phi, float* const* rhs, float* const* tmp,
+                        const float* cop, const double* su, double* pp, double* p, int ncycles,
+                        int n_pre, int n_post, int n_coarse, int flags, const int* active,
+                        void* stream) {
+  if (!mg_args_ok(b, phi, rhs, tmp, cop, ncycles, n_pre, n_post, n_coarse, flags) || !su || !pp ||
+      !p)
+    return WF_EINVAL;
+  return batch_mg_correct(B_(b), phi, rhs, tmp, cop, su, pp, p, ncycles, n_pre, n_post, n_coarse,
+                          flags, active, (hipStream_t)stream);
+}
+
+int wf_batch_project_test(wf_batch b, const double* us, const double* vs, const double* ws,
+                          const double* p, double* u, double* v, double* w, double* su,
+                          float* rhs0, double* rmax, double alpha, double eps, int it,
+                          int* active, int* iters, int* status, void* stream) {
+  if (!ok(b) || !us || !vs || !ws || !p || !u || !v || !w || !su || !rhs0 || !rmax || it < 1 ||
+      !active || !iters || !status)
+    return WF_EINVAL;
+  return batch_calvel3_calmas(B_(b), us, vs, ws, p, u, v, w, su, rmax, alpha, rhs0,
+                              it > 1 ? active : nullptr, (hipStream_t)stream,
+                              BatchTest{it, eps, active, iters, status});
 }
 
 int wf_batch_project_mask(wf_batch b, const double* rmax, double eps, int it, int* active,

@@ -1024,7 +1024,7 @@ batch_checkdt_kernel(BView V, Plan P, const double* u, const double* v, const do
 // quantity q (bit q of min_mask: min, else max).
 __global__ void __launch_bounds__(1024)
 batch_red_fold_kernel(BView V, Plan P, const double* part, int stride, int nq, int min_mask,
-                      double* out, const int* active) {
+                      double* out, const int* active, BatchTest test) {
   const int m = blockIdx.x;
   if (active && !active[m]) return;  // uniform per workgroup
   const MemDev& M = V.mem[m];
@@ -1045,6 +1045,7 @@ batch_red_fold_kernel(BView V, Plan P, const double* part, int stride, int nq, i
       double r = sh[0];
       for (int w = 1; w < 16; ++w) r = mn ? nan_min(r, sh[w]) : nan_max(r, sh[w]);
       out[m * nq + q] = r;
+      if (test.it) loop_test(m, r, test.eps, test.it, test.active, test.iters, test.status);
     }
     __syncthreads();
   }
@@ -1080,7 +1081,7 @@ int batch_wale_checkdt(const Batch& B, const double* u, const double* v, const d
                      w, vis, B.red_part, B.nred);
   WF_LAUNCHED();
   hipLaunchKernelGGL(batch_red_fold_kernel, dim3(B.nmem), dim3(1024), 0, s, B.view(), P,
-                     (const double*)B.red_part, B.nred, 4, 8, out4, (const int*)nullptr);
+                     (const double*)B.red_part, B.nred, 4, 8, out4, (const int*)nullptr, BatchTest{});
   WF_LAUNCHED();
   return 0;
 }
@@ -1111,7 +1112,7 @@ int batch_calmas(const Batch& B, const double* u, const double* v, const double*
                      su, B.red_part, active);
   WF_LAUNCHED();
   hipLaunchKernelGGL(batch_red_fold_kernel, dim3(B.nmem), dim3(1024), 0, s, B.view(), P,
-                     (const double*)B.red_part, B.nred, 1, 0, rmax, active);
+                     (const double*)B.red_part, B.nred, 1, 0, rmax, active, BatchTest{});
   WF_LAUNCHED();
   return 0;
 }
@@ -1119,13 +1120,13 @@ int batch_calmas(const Batch& B, const double* u, const double* v, const double*
 int batch_calvel3_calmas(const Batch& B, const double* us, const double* vs, const double* ws,
                          const double* p, double* u, double* v, double* w, double* su,
                          double* rmax, double alpha, float* r32, const int* active,
-                         hipStream_t s) {
+                         hipStream_t s, const BatchTest& test) {
   const Plan& P = B.plan[PK_STREAM];
   hipLaunchKernelGGL(batch_calvel3_calmas_kernel, dim3(P.total), dim3(256), 0, s, B.view(), P, us,
                      vs, ws, p, u, v, w, su, B.red_part, alpha, r32, active);
   WF_LAUNCHED();
   hipLaunchKernelGGL(batch_red_fold_kernel, dim3(B.nmem), dim3(1024), 0, s, B.view(), P,
-                     (const double*)B.red_part, B.nred, 1, 0, rmax, active);
+                     (const double*)B.red_part, B.nred, 1, 0, rmax, active, test);
   WF_LAUNCHED();
   return 0;
 }
@@ -1137,7 +1138,7 @@ int batch_checkdt(const Batch& B, const double* u, const double* v, const double
                      vis, B.red_part, B.nred);
   WF_LAUNCHED();
   hipLaunchKernelGGL(batch_red_fold_kernel, dim3(B.nmem), dim3(1024), 0, s, B.view(), P,
-                     (const double*)B.red_part, B.nred, 4, 8, out4, (const int*)nullptr);
+                     (const double*)B.red_part, B.nred, 4, 8, out4, (const int*)nullptr, BatchTest{});
   WF_LAUNCHED();
   return 0;
 }

@@ -81,6 +81,9 @@ _SIGS = {
     "wf_batch_calvel3_calmas": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, C.c_double, _P, _P],
     "wf_batch_add_ring": [_P, _P, _P, _P, _P],
     "wf_batch_mg_solve_mixed": [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P],
+    "wf_batch_mg_correct": [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P],
+    "wf_batch_project_test": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, C.c_double, C.c_double,
+                              _I, _P, _P, _P, _P],
     "wf_batch_project_mask": [_P, _P, C.c_double, _I, _P, _P, _P, _P],
     "wf_batch_set_int": [_P, _I, _I, _P],
     "wf_tune_set": [_I, _I, _I, _I, _I],

@@ -246,34 +246,33 @@ class Ensemble:
             self._fill_uvw(again=stage > 0)
             if stage + 1 < len(ALFARK):
                 self._calvel(alpha)
-        # projection: reset the per-member loop state; every outer test opens
-        # with the calvel/calmas pair in one pass, so a calvel of its own runs
-        # here only when no test does (solver.py:178-212)
+        # projection: the first outer test resets the per-member loop state, and
+        # every test opens with the calvel/calmas pair in one pass, so a calvel
+        # and a reset of their own run here only when no test does
+        # (solver.py:178-212)
         if self.maxcy < 1:
             self._calvel(1.0)
-        _hip.call("wf_batch_set_int", self.active.ptr, self.nmem, 1, s)
-        _hip.call("wf_batch_set_int", self.iters.ptr, self.nmem, 0, s)
+            _hip.call("wf_batch_set_int", self.active.ptr, self.nmem, 1, s)
+            _hip.call("wf_batch_set_int", self.iters.ptr, self.nmem, 0, s)
 
     def _outer_test(self, it):
         """calvel + calmas in one pass and the break test of outer iteration
         `it` (solver.py:185-197) for the active members."""
         P = self.pool
-        self._call("wf_batch_calvel3_calmas", P["ustar"].ptr, P["vstar"].ptr, P["wstar"].ptr,
-                   P["p"].ptr, P["u"].ptr, P["v"].ptr, P["w"].ptr, P["su"].ptr, self.rmax.ptr,
-                   1.0, self.active.ptr, self.stream)
-        self._call("wf_batch_project_mask", self.rmax.ptr, self.eps, int(it), self.active.ptr,
-                   self.iters.ptr, self.status.ptr, self.stream)
+        self._call("wf_batch_project_test", P["ustar"].ptr, P["vstar"].ptr, P["wstar"].ptr,
+                   P["p"].ptr, P["u"].ptr, P["v"].ptr, P["w"].ptr, P["su"].ptr,
+                   self.lpool["rhs"][0].ptr, self.rmax.ptr, 1.0, self.eps, int(it),
+                   self.active.ptr, self.iters.ptr, self.status.ptr, self.stream)
 
     def _outer_rest(self, it):
-        """MG solve, p += pp, p ghosts for the active members; after the last
-        allowed iteration `it` also the calvel that closes it (the next test
+        """MG solve (from the right-hand side the outer test left), p += pp, p
+        ghosts for the active members; after the last allowed iteration `it` also the calvel that closes it (the next test
         would otherwise run it)."""
         P, s, a = self.pool, self.stream, self.active.ptr
-        self._call("wf_batch_mg_solve_mixed", self._lptr["phi"], self._lptr["rhs"],
+        self._call("wf_batch_mg_correct", self._lptr["phi"], self._lptr["rhs"],
                    self._lptr["tmp"], self.cop.ptr if self.use_cop else None, P["su"].ptr,
-                   P["pp"].ptr, self.mixed_cycles, self.N_PRE, self.N_POST, self.N_COARSE, 2,
-                   a, s)
-        self._call("wf_batch_add_ring", P["p"].ptr, P["pp"].ptr, a, s)
+                   P["pp"].ptr, P["p"].ptr, self.mixed_cycles, self.N_PRE, self.N_POST,
+                   self.N_COARSE, 2, a, s)
         self._fill("p", "pbound", self.active)
         if it == self.maxcy:
             self._calvel(1.0, self.active)
