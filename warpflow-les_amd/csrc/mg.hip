@@ -25,6 +25,7 @@
 #include "batch.h"
 #include "mg_common.h"
 #include "relax_block.h"
+#include "relax_wg.h"
 
 namespace wf {
 
@@ -2701,9 +2702,60 @@ int coarse_op_build_t(const wf_mg_level& L, int nsweeps, void* op, hipStream_t s
   return 0;
 }
 
+// A one-workgroup leg (relax_wg.h).
+template <class T>
+int wg_leg(const wf_mg_level* lv, int l0, int l1, bool up, int ns, bool zero0, hipStream_t s) {
+  WgLevels<T> W{};
+  int nt = 64, lds = 0;
+  for (int l = l0; l <= l1 + 1; ++l) {
+    W.d[l] = mg_dev(lv[l]);
+    W.phi[l] = (T*)lv[l].phi;
+    W.rhs[l] = (T*)lv[l].rhs;
+    inv_h2(lv[l], W.c[l][0], W.c[l][1], W.c[l][2]);
+    if (l > l1) continue;
+    nt = std::max(nt, div_up(wg_threads(lv[l].n0, lv[l].n1, lv[l].n2), 64) * 64);
+    lds = std::max(lds, wg_lds(lv[l].n0, (int)sizeof(T)));
+  }
+  if (up)
+    hipLaunchKernelGGL((wg_leg_kernel<T, true>), dim3(1), dim3(nt), lds, s, W, l0, l1, ns, zero0);
+  else
+    hipLaunchKernelGGL((wg_leg_kernel<T, false>), dim3(1), dim3(nt), lds, s, W, l0, l1, ns, zero0);
+  WF_LAUNCHED();
+  return 0;
+}
+// First level of the one-workgroup legs, which end above the coarsest level's
+// operator; nlev: none.  A level joins where blocks would relax it (no launch
+// shape was tuned for it) and it fits, with all below.
+template <class T>
+int wg_first_t(const wf_mg_level* lv, int nlev, int npre, int npost) {
+  int first = nlev;
+  BlockPlan P;
+  for (int l = nlev - 2; l >= 0; --l) {
+    if (!wg_fits(lv[l].n0, lv[l].n1, lv[l].n2) || !block_plan<T>(lv[l], npre, false, P) ||
+        !block_plan<T>(lv[l], npost, false, P))
+      break;
+    first = l;
+  }
+  return first;
+}
+int wg_first(const wf_mg_level* lv, int nlev, int npre, int npost, int ncoarse) {
+  const wf_mg_level& C = lv[nlev - 1];
+  if (nlev < 2 || nlev > WG_MAX_LEVELS || npre < 1 || npost < 1 || ncoarse < 1 || !C.cop ||
+      C.cop_sweeps != ncoarse)
+    return nlev;
+  return C.prec == 8 ? wg_first_t<double>(lv, nlev, npre, npost)
+                     : wg_first_t<float>(lv, nlev, npre, npost);
+}
+
 template <class Relax>
 int vcycle_levels(const wf_mg_level* lv, int nlev, int npre, int npost, int ncoarse,
                   hipStream_t s, Relax&& relax_l, bool zero0 = false) {
+  const int lw = wg_first(lv, nlev, npre, npost, ncoarse);
+  auto leg = [&](bool up) {
+    const bool z = lw > 0 || zero0;
+    return lv[lw].prec == 8 ? wg_leg<double>(lv, lw, nlev - 2, up, up ? npost : npre, z, s)
+                            : wg_leg<float>(lv, lw, nlev - 2, up, up ? npost : npre, z, s);
+  };
   for (int l = 0; l < nlev; ++l) {
     if (l > 0) {
       const int r = lv[l].prec == 8 ? restrict_t<double>(lv[l - 1], lv[l], s)
@@ -2716,10 +2768,17 @@ int vcycle_levels(const wf_mg_level* lv, int nlev, int npre, int npost, int ncoa
       if (r) return r;
       continue;
     }
+    if (l == lw) {
+      int r = leg(false);
+      if (!r) r = coarse_op_apply_any(lv[nlev - 1], s);
+      if (!r) r = leg(true);
+      if (r) return r;
+      break;
+    }
     const int r = relax_l(l, l < nlev - 1 ? npre : ncoarse, l == 0 && zero0);
     if (r) return r;
   }
-  for (int l = nlev - 2; l >= 0; --l) {
+  for (int l = std::min(lw, nlev - 1) - 1; l >= 0; --l) {
     const int r = lv[l].prec == 8 ? prolong_t<double>(lv[l + 1], lv[l], s)
                                   : prolong_t<float>(lv[l + 1], lv[l], s);
     if (r) return r;
