@@ -34,6 +34,7 @@ def vcycle(mg, phi, rhs, per_level):
     ((24, 24, 24), 3), ((4, 4, 4), 2), ((16, 16, 16), 3), ((12, 20, 16), 2), ((20, 24, 28), 3),
     ((32, 32, 32), 3), ((32, 8, 8), 2), ((8, 32, 32), 2), ((6, 2, 18), 2), ((2, 16, 14), 2),
     ((48, 40, 64), 4), ((88, 60, 52), 3), ((64, 56, 60), 3), ((10, 34, 30), 2), ((72, 16, 48), 4),
+    ((112, 96, 104), 2),
 ])
 @pytest.mark.parametrize("sweeps", [(6, 6), (1, 3)])
 def test_legs_equal_levels(n3, levels, prec, sweeps):

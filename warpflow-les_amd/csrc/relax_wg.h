@@ -106,39 +106,8 @@ __device__ inline void wg_level(T* __restrict__ phi, const T* __restrict__ rhs, 
   T* const lo = sm + (oi + 1) * PL + wc;
   T* const lA = lo + f * PL;        // LDS words of the odd cells: lA[2 t PL]
   T* const lE = lo + (1 - f) * PL;  // and of the even ones
-  if constexpr (UP) {  // E += the interpolation of pc (prolong_body's sum)
-    if (work) {
-      const int pcb = (int)(dc.s0 * (int64_t)sizeof(T));
-      const auto dq = buf_rsrc(pc, 0x7fffffffu);
-      const int u0 = oi / 2 + 1 - f;  // array plane below the first even cell
-      const uint32_t o = (uint32_t)((((j + 1) >> 1) * (int)dc.s1 + ((k + 1) >> 1)) *
-                                        (int)sizeof(T) + u0 * pcb);
-      uint32_t oc[4];
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-        oc[c] = live ? o + (uint32_t)(((c >> 1) * (int)dc.s1 + (c & 1)) * (int)sizeof(T))
-                     : BUF_DEAD;
-      const T wx = fb ? T(0.25) : T(0.75), wy = j & 1 ? T(0.75) : T(0.25),
-              wz = k & 1 ? T(0.75) : T(0.25);
-      T w[8];
-#pragma unroll
-      for (int c = 0; c < 8; ++c)
-        w[c] = (c & 4 ? T(1) - wx : wx) * (c & 2 ? T(1) - wy : wy) * (c & 1 ? T(1) - wz : wz);
-      T q[NH + 1][4];
-#pragma unroll
-      for (int u = 0; u <= NH; ++u)
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-          q[u][c] = buf_ld<T>(dq, !PART || u0 + u <= dc.n0 + 1 ? oc[c] : BUF_DEAD, u * pcb);
-#pragma unroll
-      for (int t = 0; t < NH; ++t) {
-        T acc = T(0);
-#pragma unroll
-        for (int c = 0; c < 8; ++c) acc = fma(w[c], q[t + (c >> 2)][c & 3], acc);
-        const T v = E[t] + acc;
-        E[t] = live && (!PART || oi + 2 * t + 1 - f < n0) ? v : T(0);
-      }
-    }
+  if constexpr (UP) {
+    if (work) add_prolonged<T, NH>(E, pc, d, oi + 1 - f, j, k, live);
   }
   __syncthreads();
   if (work) {
