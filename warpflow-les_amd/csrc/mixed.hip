@@ -218,6 +218,8 @@ defect_stream_kernel(const double* __restrict__ b, const double* __restrict__ x,
 // separate update and defect.  Loads are grouped DEFECT_U planes at a time as
 // in defect_stream_kernel (plane indices past the chunk clamped onto plane
 // z1, which the (n+2)^3 level array holds).
+// U: planes loaded at a time.
+template <int U>
 __device__ inline void assign_defect_body(const double* __restrict__ b, double* __restrict__ x,
                                           const wf_grid& g, const float* __restrict__ e,
                                           float* __restrict__ r32, const MgDev& d, double c0,
@@ -228,14 +230,14 @@ __device__ inline void assign_defect_body(const double* __restrict__ b, double* 
   const int z0 = C.z * ich, z1 = min(z0 + ich, g.ni);
   const int64_t q0 = at(g, g.npl, j + g.npl, k + g.npl);  // real plane 0 of the column
   const int64_t m0 = mg_at(d, 0, j, k);
-  for (int i0 = z0; i0 < z1; i0 += DEFECT_U) {
-    double xc[DEFECT_U + 2], bv[DEFECT_U], xs[DEFECT_U], xn[DEFECT_U], xb[DEFECT_U],
-        xt[DEFECT_U];
+  for (int i0 = z0; i0 < z1; i0 += U) {
+    double xc[U + 2], bv[U], xs[U], xn[U], xb[U],
+        xt[U];
 #pragma unroll
-    for (int u = 0; u < DEFECT_U + 2; ++u)
+    for (int u = 0; u < U + 2; ++u)
       xc[u] = 0.0 + (double)e[m0 + (int64_t)min(i0 - 1 + u, z1) * d.s0];
 #pragma unroll
-    for (int u = 0; u < DEFECT_U; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int p = min(i0 + u, z1 - 1);
       const int64_t mq = m0 + (int64_t)p * d.s0;
       bv[u] = b[q0 + (int64_t)p * g.si];
@@ -245,7 +247,7 @@ __device__ inline void assign_defect_body(const double* __restrict__ b, double* 
       xt[u] = 0.0 + (double)e[mq + 1];
     }
 #pragma unroll
-    for (int u = 0; u < DEFECT_U; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int i = i0 + u;
       if (i < z1) {
         x[q0 + (int64_t)i * g.si] = xc[u + 1];
@@ -261,7 +263,7 @@ __global__ void __launch_bounds__(256)
 assign_defect_kernel(const double* __restrict__ b, double* __restrict__ x, wf_grid g,
                      const float* __restrict__ e, float* __restrict__ r32, MgDev d, double c0,
                      double c1, double c2, const double* __restrict__ mean, int ich) {
-  assign_defect_body(b, x, g, e, r32, d, c0, c1, c2, mean, ich, this_blk());
+  assign_defect_body<DEFECT_U>(b, x, g, e, r32, d, c0, c1, c2, mean, ich, this_blk());
 }
 
 // out = max(partials[0..n)), one 1024-thread workgroup, fixed order.
@@ -435,9 +437,14 @@ batch_assign_defect_kernel(BView V, Plan P, const double* su, double* pp, const 
   const int4 it = plan_item(P, w);
   if (active && !active[it.x]) return;
   const MemDev& M = V.mem[it.x];
-  assign_defect_body(su + M.off, pp + M.off, M.g, phi0 + M.loff[0], rhs0 + M.loff[0],
-                     level0_dev(M), M.r2[0], M.r2[1], M.r2[2], nullptr, P.ich,
-                     Blk{it.y, it.z, it.w});
+  auto run = [&](auto body) {
+    body(su + M.off, pp + M.off, M.g, phi0 + M.loff[0], rhs0 + M.loff[0], level0_dev(M), M.r2[0],
+         M.r2[1], M.r2[2], (const double*)nullptr, P.ich, Blk{it.y, it.z, it.w});
+  };
+  if (P.ich == 1)  // one plane per item: three more would be loaded for nothing
+    run(assign_defect_body<1>);
+  else
+    run(assign_defect_body<DEFECT_U>);
 }
 
 // pp = 0.0 + e (ASSIGN) or pp + e on the real cells; part (nullable): the block
@@ -475,6 +482,7 @@ batch_update_kernel(BView V, Plan P, double* pp, const float* phi0, double* part
   const int t = threadIdx.y * 64 + threadIdx.x;
 #pragma unroll
   for (int u = 0; u < BATCH_ICH; ++u) {
+    if (u >= np) break;  // uniform
     const double r = wave_sum(v[u]);
     if ((t & 63) == 0) ps[u][t >> 6] = r;
   }
