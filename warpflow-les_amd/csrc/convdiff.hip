@@ -148,6 +148,15 @@ __device__ inline double i4(double p1, double c0, double m1, double m2) {
 __device__ inline double d4(double sp, double sn, double sm, double smm, double r24h) {
   return (__builtin_fma(-27.0, sm, __builtin_fma(27.0, sn, -sp)) + smm) * r24h;
 }
+// The same by the rounded quotient: x / d24 = x r24h corrected by its exact
+// remainder (Markstein; x r24h itself where that is not finite).
+__device__ inline double d4q(double sp, double sn, double sm, double smm, double d24,
+                             double r24h) {
+  const double x = __builtin_fma(-27.0, sm, __builtin_fma(27.0, sn, -sp)) + smm;
+  const double q = x * r24h;
+  const double z = __builtin_fma(__builtin_fma(-q, d24, x), r24h, q);
+  return __builtin_isfinite(q) ? z : q;
+}
 // (-f[+2] + 16 f[+1] - 30 f[0] + 16 f[-1] - f[-2]) / (12 h^2)  (kernels.py:177-186)
 __device__ inline double l4(double p2, double p1, double c, double m1, double m2,
                             double ir12) {
@@ -167,6 +176,7 @@ struct Coefs {
   double r24x, r24y, r24z;     // 1 / (24 h)
   double ir12x, ir12y, ir12z;  // 1 / (12 h^2)
   double dta;                  // dt * alpha
+  double d24x, d24y, d24z;     // 24 h (the convective pass alone)
 };
 
 // Own-component region: plane i with a cross-shaped 3-cell halo.
@@ -192,7 +202,9 @@ struct Lay {  // regions of the two staged cross quantities
 // value c_oo is the component itself, taken from the thread's register
 // window instead of being loaded, and written to coo_save on the box -- the
 // cells the second stage reads as c_oo -- in place of a full-field copy.
-template <int C, bool SAVE = false>
+// DIFF = false: the convective update alone, c_oo - dt alpha N(c), with the
+// reference's quotients by 24 h rounded as quotients; vis is not read.
+template <int C, bool SAVE = false, bool DIFF = true>
 __device__ inline void convdiff_body(const double* __restrict__ u, const double* __restrict__ v,
                                      const double* __restrict__ w,
                                      const double* __restrict__ coo,
@@ -252,7 +264,7 @@ __device__ inline void convdiff_body(const double* __restrict__ u, const double*
   double fhalo = hs.on ? F[G.plane(i0 + 2) + hs.off] : 0.0;
   double cnew = 0.0;
   if constexpr (!SAVE) cnew = coo[G.plane(i0) + own.off];
-  double vnew = vis[G.plane(i0) + visoff];
+  double vnew = DIFF ? vis[G.plane(i0) + visoff] : 0.0;
 
   // C = 0: windows of v and w at the tile cell and at the halo position,
   // planes i-1 .. i+2 after the shift
@@ -348,7 +360,7 @@ __device__ inline void convdiff_body(const double* __restrict__ u, const double*
       fnew = F[G.plane(i + 4) + own.off];
       if (hs.on) fhalo = F[G.plane(i + 3) + hs.off];
       if constexpr (!SAVE) cnew = coo[G.plane(i + 1) + own.off];
-      vnew = vis[G.plane(i + 1) + visoff];
+      if constexpr (DIFF) vnew = vis[G.plane(i + 1) + visoff];
       if constexpr (C == 0) {
         const int64_t pn = G.plane(i + 3);
         van = FA[pn + ia.off];
@@ -369,11 +381,20 @@ __device__ inline void convdiff_body(const double* __restrict__ u, const double*
     auto Fo = [&](int dj, int dk) { return S[OwnR::idx(tj + dj, tk + dk)]; };
     const double c0 = f[3];
     double nsum;
+    auto dx4 = [&](double sp, double sn, double sm, double smm) {
+      return DIFF ? d4(sp, sn, sm, smm, K.r24x) : d4q(sp, sn, sm, smm, K.d24x, K.r24x);
+    };
+    auto dy4 = [&](double sp, double sn, double sm, double smm) {
+      return DIFF ? d4(sp, sn, sm, smm, K.r24y) : d4q(sp, sn, sm, smm, K.d24y, K.r24y);
+    };
+    auto dz4 = [&](double sp, double sn, double sm, double smm) {
+      return DIFF ? d4(sp, sn, sm, smm, K.r24z) : d4q(sp, sn, sm, smm, K.d24z, K.r24z);
+    };
     if constexpr (C == 0) {
       // x: conv_self(u) along x, rolled squares of I4x(u)
       const double a2 = i4(f[6], f[5], f[4], f[3]);
       const double s2 = a2 * a2;
-      const double tx = d4(s2, r1, r0, rm1, K.r24x);
+      const double tx = dx4(s2, r1, r0, rm1);
       rm1 = r0;
       r0 = r1;
       r1 = s2;
@@ -381,20 +402,21 @@ __device__ inline void convdiff_body(const double* __restrict__ u, const double*
       const double uy3 = Fo(3, 0), uy2 = Fo(2, 0), uy1 = Fo(1, 0);
       const double uym1 = Fo(-1, 0), uym2 = Fo(-2, 0), uym3 = Fo(-3, 0);
       const double ty =
-          d4(i4(uy3, uy2, uy1, c0) * A[IvR::idx(tj + 1, tk)],
+          dy4(i4(uy3, uy2, uy1, c0) * A[IvR::idx(tj + 1, tk)],
              i4(uy2, uy1, c0, uym1) * A[IvR::idx(tj, tk)],
              i4(uy1, c0, uym1, uym2) * A[IvR::idx(tj - 1, tk)],
-             i4(c0, uym1, uym2, uym3) * A[IvR::idx(tj - 2, tk)], K.r24y);
+             i4(c0, uym1, uym2, uym3) * A[IvR::idx(tj - 2, tk)]);
       // z: I4z(u) at columns m+1 times I4x(w) at (plane i+1, column m)
       const double uz3 = Fo(0, 3), uz2 = Fo(0, 2), uz1 = Fo(0, 1);
       const double uzm1 = Fo(0, -1), uzm2 = Fo(0, -2), uzm3 = Fo(0, -3);
       const double tz =
-          d4(i4(uz3, uz2, uz1, c0) * B[IwR::idx(tj, tk + 1)],
+          dz4(i4(uz3, uz2, uz1, c0) * B[IwR::idx(tj, tk + 1)],
              i4(uz2, uz1, c0, uzm1) * B[IwR::idx(tj, tk)],
              i4(uz1, c0, uzm1, uzm2) * B[IwR::idx(tj, tk - 1)],
-             i4(c0, uzm1, uzm2, uzm3) * B[IwR::idx(tj, tk - 2)], K.r24z);
+             i4(c0, uzm1, uzm2, uzm3) * B[IwR::idx(tj, tk - 2)]);
       nsum = tx + ty + tz;
-      if (live) {
+      if (live && !DIFF) cstar[G.plane(i) + own.off] = __builtin_fma(-K.dta, nsum, cur_coo);
+      if (live && DIFF) {
         const double lap = l4(f[5], f[4], c0, f[2], f[1], K.ir12x) +
                            l4(uy2, uy1, c0, uym1, uym2, K.ir12y) +
                            l4(uz2, uz1, c0, uzm1, uzm2, K.ir12z);
@@ -411,7 +433,7 @@ __device__ inline void convdiff_body(const double* __restrict__ u, const double*
         iu = i4(A[U2R::idx(tj, tk + 2)], A[U2R::idx(tj, tk + 1)], A[U2R::idx(tj, tk)],
                 A[U2R::idx(tj, tk - 1)]);
       const double q1 = i4(f[6], f[5], f[4], f[3]) * iu;
-      const double tx = d4(q1, r1, r0, rm1, K.r24x);
+      const double tx = dx4(q1, r1, r0, rm1);
       rm1 = r0;
       r0 = r1;
       r1 = q1;
@@ -424,29 +446,30 @@ __device__ inline void convdiff_body(const double* __restrict__ u, const double*
         // y: conv_self(v) along y
         const double p2 = i4(y3, y2, y1, c0), p1 = i4(y2, y1, c0, ym1);
         const double p0 = i4(y1, c0, ym1, ym2), m1 = i4(c0, ym1, ym2, ym3);
-        ty = d4(p2 * p2, p1 * p1, p0 * p0, m1 * m1, K.r24y);
+        ty = dy4(p2 * p2, p1 * p1, p0 * p0, m1 * m1);
         // z: I4z(v) at columns m+1 times I4y(w) across rows (+2 .. -1) at column m
         auto wq = [&](int m) {
           return i4(B[W1R::idx(tj + 2, tk + m)], B[W1R::idx(tj + 1, tk + m)],
                     B[W1R::idx(tj, tk + m)], B[W1R::idx(tj - 1, tk + m)]);
         };
-        tz = d4(i4(z3, z2, z1, c0) * wq(1), i4(z2, z1, c0, zm1) * wq(0),
-                i4(z1, c0, zm1, zm2) * wq(-1), i4(c0, zm1, zm2, zm3) * wq(-2), K.r24z);
+        tz = dz4(i4(z3, z2, z1, c0) * wq(1), i4(z2, z1, c0, zm1) * wq(0),
+                i4(z1, c0, zm1, zm2) * wq(-1), i4(c0, zm1, zm2, zm3) * wq(-2));
       } else {
         // y: I4y(w) at rows m+1 times I4z(v) across columns (+2 .. -1) at row m
         auto vq = [&](int m) {
           return i4(B[V2R::idx(tj + m, tk + 2)], B[V2R::idx(tj + m, tk + 1)],
                     B[V2R::idx(tj + m, tk)], B[V2R::idx(tj + m, tk - 1)]);
         };
-        ty = d4(i4(y3, y2, y1, c0) * vq(1), i4(y2, y1, c0, ym1) * vq(0),
-                i4(y1, c0, ym1, ym2) * vq(-1), i4(c0, ym1, ym2, ym3) * vq(-2), K.r24y);
+        ty = dy4(i4(y3, y2, y1, c0) * vq(1), i4(y2, y1, c0, ym1) * vq(0),
+                i4(y1, c0, ym1, ym2) * vq(-1), i4(c0, ym1, ym2, ym3) * vq(-2));
         // z: conv_self(w) along z
         const double p2 = i4(z3, z2, z1, c0), p1 = i4(z2, z1, c0, zm1);
         const double p0 = i4(z1, c0, zm1, zm2), m1 = i4(c0, zm1, zm2, zm3);
-        tz = d4(p2 * p2, p1 * p1, p0 * p0, m1 * m1, K.r24z);
+        tz = dz4(p2 * p2, p1 * p1, p0 * p0, m1 * m1);
       }
       nsum = tx + ty + tz;
-      if (live) {
+      if (live && !DIFF) cstar[G.plane(i) + own.off] = __builtin_fma(-K.dta, nsum, cur_coo);
+      if (live && DIFF) {
         const double lap = l4(f[5], f[4], c0, f[2], f[1], K.ir12x) +
                            l4(y2, y1, c0, ym1, ym2, K.ir12y) +
                            l4(z2, z1, c0, zm1, zm2, K.ir12z);
@@ -469,6 +492,18 @@ convdiff_kernel(const double* __restrict__ u, const double* __restrict__ v,
   const int L = xcd_linear(blockIdx.x + blockIdx.y * gridDim.x, nb);
   convdiff_body<C, SAVE>(u, v, w, coo, vis, cstar, g, b, ich, L % kt, (L / kt) % jt,
                          L / (kt * jt) * cstep, K, coo_save);
+}
+
+// The convective update alone.
+template <int C>
+__global__ void __launch_bounds__(256)
+conv_kernel(const double* __restrict__ u, const double* __restrict__ v,
+            const double* __restrict__ w, const double* __restrict__ coo,
+            double* __restrict__ cstar, wf_grid g, Box3 b, int ich, int kt, int jt, Coefs K) {
+  const int nb = kt * jt * gridDim.y;
+  const int L = xcd_linear(blockIdx.x + blockIdx.y * gridDim.x, nb);
+  convdiff_body<C, false, false>(u, v, w, coo, nullptr, cstar, g, b, ich, L % kt, (L / kt) % jt,
+                                 L / (kt * jt), K);
 }
 
 // ---------------------------------------------------------------------------
@@ -1411,6 +1446,34 @@ int batch_convdiff(const Batch& B, int comp, const double* u, const double* v,
 }
 
 // Launch of the fused operator on box b (checked by the caller).
+// conv4th alone on the fused pass's tiles: a thread per cell with every tap from
+// global memory took about fifty loads and three FP64 divisions, 25 us for 96 x 80
+// x 112 cells in the caches; here 14 us (the traffic's floor is 5).
+int conv_launch(int comp, const double* u, const double* v, const double* w, const double* coo,
+                double* cstar, const wf_grid& g, const Box3& b, double dx, double dy, double dz,
+                double dta, hipStream_t s) {
+  using namespace cdv;
+  const int kt = div_up(b.d2, TK), jt = div_up(b.d1, TJ);
+  const int64_t tiles = (int64_t)kt * jt;
+  const int ich = pick_chunk(b.d0, ChunkCost{4, {1.1, 1.75, 2.75, 3.7}}, INT32_MAX,
+                       [&](int c) { return tiles * div_up(b.d0, c); });
+  const int nch = div_up(b.d0, ich);
+  if (tiles * nch >= (int64_t)1 << 31 || nch > 65535) return WF_EINVAL;
+  Coefs K{};
+  K.d24x = 24.0 * dx;
+  K.d24y = 24.0 * dy;
+  K.d24z = 24.0 * dz;
+  K.r24x = 1.0 / K.d24x;
+  K.r24y = 1.0 / K.d24y;
+  K.r24z = 1.0 / K.d24z;
+  K.dta = dta;
+  auto k = comp == 0 ? conv_kernel<0> : comp == 1 ? conv_kernel<1> : conv_kernel<2>;
+  hipLaunchKernelGGL(k, dim3((unsigned)tiles, (unsigned)nch), dim3(NT), 0, s, u, v, w, coo, cstar,
+                     g, b, ich, kt, jt, K);
+  WF_LAUNCHED();
+  return 0;
+}
+
 int convdiff_launch(int comp, const double* u, const double* v, const double* w,
                     const double* coo, const double* vis, double* cstar, const wf_grid& g,
                     const Box3& b, double dx, double dy, double dz, double dta, int ich,

@@ -14,65 +14,6 @@
 
 namespace wf {
 
-// 4th-order midpoint interpolant along stride s at c (kernels.py:31-46):
-// (-f[c+s] + 9 f[c] + 9 f[c-s] - f[c-2s]) / 16
-__device__ inline double I4(const double* __restrict__ f, int64_t c, int64_t s) {
-  return (-f[c + s] + 9.0 * f[c] + 9.0 * f[c - s] - f[c - 2 * s]) / 16.0;
-}
-
-// Staggered 4-point derivative (kernels.py:69, :80, :281-286):
-// (-s[+] + 27 s[0] - 27 s[-] + s[--]) / (24 h)
-__device__ inline double D4(double sp, double sn, double sm, double smm, double h) {
-  return (-sp + 27.0 * sn - 27.0 * sm + smm) / (24.0 * h);
-}
-// The same with the division replaced by r24h = 1 / (24 h) formed once.
-__device__ inline double D4r(double sp, double sn, double sm, double smm, double r24h) {
-  return (-sp + 27.0 * sn - 27.0 * sm + smm) * r24h;
-}
-
-// d(c c)/dx_a for the component c living on axis a (kernels.py:64-69,
-// :103-108, :143-148).
-__device__ inline double conv_self(const double* __restrict__ c, int64_t x, int64_t sa,
-                                   double ha) {
-  const double p2 = I4(c, x + 2 * sa, sa), p1 = I4(c, x + sa, sa);
-  const double p0 = I4(c, x, sa), m1 = I4(c, x - sa, sa);
-  return D4(p2 * p2, p1 * p1, p0 * p0, m1 * m1, ha);
-}
-
-// d(c q)/dx_b for component c (axis a) and the component q along the cross
-// axis b: c is interpolated along b at b+2..b-1, q along a at a+1 and
-// b+1..b-2, so the derivative lands on c's face (kernels.py:71-87,
-// :110-127, :150-166).
-__device__ inline double conv_cross(const double* __restrict__ c,
-                                    const double* __restrict__ q, int64_t x,
-                                    int64_t sa, int64_t sb, double hb) {
-  const double sp1 = I4(c, x + 2 * sb, sb) * I4(q, x + sa + sb, sa);
-  const double sn = I4(c, x + sb, sb) * I4(q, x + sa, sa);
-  const double sm1 = I4(c, x, sb) * I4(q, x + sa - sb, sa);
-  const double sm2 = I4(c, x - sb, sb) * I4(q, x + sa - 2 * sb, sa);
-  return D4(sp1, sn, sm1, sm2, hb);
-}
-
-// N(c) = x-term + y-term + z-term, the reference's summation order for all
-// three components (kernels.py:89, :129, :168).
-template <int C>
-__device__ inline double conv_sum(const double* __restrict__ u,
-                                  const double* __restrict__ v,
-                                  const double* __restrict__ w, int64_t x,
-                                  const wf_grid& g, double dx, double dy, double dz) {
-  const int64_t sx = g.si, sy = g.sj, sz = 1;
-  if (C == 0) {
-    return conv_self(u, x, sx, dx) + conv_cross(u, v, x, sx, sy, dy) +
-           conv_cross(u, w, x, sx, sz, dz);
-  } else if (C == 1) {
-    return conv_cross(v, u, x, sy, sx, dx) + conv_self(v, x, sy, dy) +
-           conv_cross(v, w, x, sy, sz, dz);
-  } else {
-    return conv_cross(w, u, x, sz, sx, dx) + conv_cross(w, v, x, sz, sy, dy) +
-           conv_self(w, x, sz, dz);
-  }
-}
-
 // 4th-order Laplacian (kernels.py:177-186); r12xx = 12*dx*dx etc.
 __device__ inline double lap4(const double* __restrict__ f, int64_t x, const wf_grid& g,
                               double r12xx, double r12yy, double r12zz) {
@@ -90,20 +31,6 @@ __device__ inline double lap4(const double* __restrict__ f, int64_t x, const wf_
 template <int C>
 __device__ inline int64_t vis_offset(const wf_grid& g) {
   return C == 0 ? 0 : (C == 1 ? g.sj : 1);  // kernels.py:198, :211, :224
-}
-
-template <int C>
-__global__ void __launch_bounds__(256)
-conv4th_kernel(const double* __restrict__ u, const double* __restrict__ v,
-               const double* __restrict__ w, const double* __restrict__ coo,
-               double* __restrict__ cstar, wf_grid g, Box3 b, double dx, double dy,
-               double dz, double dta, int ich) {
-  for_planes(b.d0, ich, [&](Blk B) {
-    int i, j, k;
-    if (!box_thread(b, B, i, j, k)) return;
-    const int64_t x = at(g, i, j, k);
-    cstar[x] = coo[x] - dta * conv_sum<C>(u, v, w, x, g, dx, dy, dz);
-  });
 }
 
 template <int C>
@@ -1210,18 +1137,7 @@ int wf_conv4th(int comp, const double* u, const double* v, const double* w,
   const Box3 b = npl_box(g, d0, d1, d2);
   if (comp < 0 || comp > 2 || !box_ok(g, b, 3, 3)) return WF_EINVAL;
   if (empty(b)) return 0;
-  const double dta = dt * alpha;
-  if (comp == 0)
-    hipLaunchKernelGGL(conv4th_kernel<0>, CG(b), box_block(), 0, S_(stream), u, v, w,
-                       coo, cstar, g, b, dx, dy, dz, dta, CH(b));
-  else if (comp == 1)
-    hipLaunchKernelGGL(conv4th_kernel<1>, CG(b), box_block(), 0, S_(stream), u, v, w,
-                       coo, cstar, g, b, dx, dy, dz, dta, CH(b));
-  else
-    hipLaunchKernelGGL(conv4th_kernel<2>, CG(b), box_block(), 0, S_(stream), u, v, w,
-                       coo, cstar, g, b, dx, dy, dz, dta, CH(b));
-  WF_LAUNCHED();
-  return 0;
+  return conv_launch(comp, u, v, w, coo, cstar, g, b, dx, dy, dz, dt * alpha, S_(stream));
 }
 
 int wf_diff4th(int comp, const double* c, const double* vis, double* cstar, wf_grid g,
