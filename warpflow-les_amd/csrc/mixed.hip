@@ -40,6 +40,10 @@ inline dim3 field_grid(const wf_grid& g) {
 }
 inline int field_ich(const wf_grid& g) { return plane_chunk(g.ni, g.nj, g.nk); }
 inline dim3 field_cgrid(const wf_grid& g) { return chunk_grid(g.ni, g.nj, g.nk, field_ich(g)); }
+inline int64_t field_chunks(const wf_grid& g) {
+  const dim3 b = field_cgrid(g);
+  return (int64_t)b.x * b.y * b.z;
+}
 inline int64_t field_blocks(const wf_grid& g) {
   const dim3 b = field_grid(g);
   return (int64_t)b.x * b.y * b.z;
@@ -164,23 +168,28 @@ defect_kernel(const double* __restrict__ b, const double* __restrict__ x, wf_gri
                    [&](Blk B) { defect_body(b, x, g, r32, d, c0, c1, c2, mean, rmax, B); });
 }
 
-// The same defect (x given, no rmax), DEFECT_U planes at a time: a thread
+// The same defect (x given), DEFECT_U planes at a time: a thread
 // issues every load of its (j, k) column for U planes -- x at planes i0-1 ..
 // i0+U, b and the four in-plane neighbours of x at each plane -- before the
 // first use, so U planes of HBM reads are in flight per wait (the
 // plane-at-a-time walk waits on each plane's loads in turn).  Plane indices
 // past the chunk are clamped onto its last plane (x: onto plane z1, real or
 // the first ghost plane), so every load stays inside the field; their values
-// are not used.  Same addresses and the same bits as defect_kernel.
+// are not used.  Same addresses and the same bits as defect_kernel; RMAX: one
+// maximum per workgroup's chunk, at rmax[workgroup] (256^3, a plane at a time with
+// a barrier each: 111 us; here 98).
 constexpr int DEFECT_U = 4;
+template <bool RMAX>
 __global__ void __launch_bounds__(256)
 defect_stream_kernel(const double* __restrict__ b, const double* __restrict__ x, wf_grid g,
                      float* __restrict__ r32, MgDev d, double c0, double c1, double c2,
-                     const double* __restrict__ mean, int ich) {
+                     const double* __restrict__ mean, int ich, double* __restrict__ rmax) {
   const Blk C = this_blk();
   const int k = C.x * 64 + threadIdx.x, j = C.y * 4 + threadIdx.y;
-  if (k >= g.nk || j >= g.nj) return;  // no barriers below
-  const int z0 = C.z * ich, z1 = min(z0 + ich, g.ni);
+  const bool live = k < g.nk && j < g.nj;
+  if (!RMAX && !live) return;  // no barriers below
+  const int z0 = C.z * ich, z1 = live ? min(z0 + ich, g.ni) : z0;
+  double av = 0.0;
   const int64_t q0 = at(g, g.npl, j + g.npl, k + g.npl);  // real plane 0 of the column
   for (int i0 = z0; i0 < z1; i0 += DEFECT_U) {
     double xc[DEFECT_U + 2], bv[DEFECT_U], xs[DEFECT_U], xn[DEFECT_U], xb[DEFECT_U],
@@ -203,10 +212,21 @@ defect_stream_kernel(const double* __restrict__ b, const double* __restrict__ x,
       if (i < z1) {
         const Coef<double> c = mg_coef(d, i, j, k, c0, c1, c2);
         double r = defect_val(bv[u], c, xc[u + 1], xc[u], xc[u + 2], xs[u], xn[u], xb[u], xt[u]);
+        if (RMAX) av = nan_max(av, fabs(r));
         if (mean) r = r - *mean;
         r32[mg_at(d, i, j, k)] = (float)r;
       }
     }
+  }
+  if constexpr (RMAX) {
+    __shared__ double part[4];
+    const double m = wave_max(av);
+    const int t = threadIdx.y * 64 + threadIdx.x;
+    if ((t & 63) == 0) part[t >> 6] = m;
+    __syncthreads();
+    if (t == 0)
+      rmax[((int64_t)C.z * gridDim.y + C.y) * gridDim.x + C.x] =
+          nan_max(nan_max(part[0], part[1]), nan_max(part[2], part[3]));
   }
 }
 
@@ -272,7 +292,15 @@ max_fold_kernel(const double* __restrict__ partials, int64_t n, double* __restri
   __shared__ double s[16];
   const int t = threadIdx.x;
   double m = 0.0;
-  for (int64_t q = t; q < n; q += 1024) m = nan_max(m, partials[q]);
+  int64_t q = t;
+  for (; q + 7 * 1024 < n; q += 8 * 1024) {  // eight loads ahead, as fold_body
+    double a[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) a[e] = partials[q + e * 1024];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) m = nan_max(m, a[e]);
+  }
+  for (; q < n; q += 1024) m = nan_max(m, partials[q]);
   m = wave_max(m);
   if ((t & 63) == 0) s[t >> 6] = m;
   __syncthreads();
@@ -771,18 +799,19 @@ int wf_mg_solve_mixed(const wf_mg_level* levels, int nlev, const double* su, dou
         (c == 0 && (flags & MIX_RHS_READY) && !tol_mode && !(flags & MIX_DEFECT_MEAN));
     defect_formed = false;
     if (!rhs_ready) {
-      if (c > 0 && !tol_mode)
-        hipLaunchKernelGGL(defect_stream_kernel, field_cgrid(g), dim3(64, 4), 0, s, su, pp, g,
-                           (float*)L0.rhs, d0, c0, c1, c2, dmean, field_ich(g));
+      if (c > 0)
+        hipLaunchKernelGGL(tol_mode ? defect_stream_kernel<true> : defect_stream_kernel<false>,
+                           field_cgrid(g), dim3(64, 4), 0, s, su, pp, g, (float*)L0.rhs, d0, c0,
+                           c1, c2, dmean, field_ich(g), work + WORK_HEAD);
       else
         hipLaunchKernelGGL(defect_kernel, field_cgrid(g), dim3(64, 4), 0, s, su,
-                           c == 0 ? nullptr : pp, g, (float*)L0.rhs, d0, c0, c1, c2, dmean,
+                           (const double*)nullptr, g, (float*)L0.rhs, d0, c0, c1, c2, dmean,
                            tol_mode ? work + WORK_HEAD : nullptr, field_ich(g));
       WF_LAUNCHED();
     }
     if (tol_mode) {
       hipLaunchKernelGGL(max_fold_kernel, dim3(1), dim3(1024), 0, s, work + WORK_HEAD,
-                         field_blocks(g), rmax);
+                         c > 0 ? field_chunks(g) : field_blocks(g), rmax);
       WF_LAUNCHED();
       double h = 0.0;
       WF_TRY(hipMemcpyAsync(&h, rmax, sizeof(double), hipMemcpyDeviceToHost, s));

@@ -23,7 +23,9 @@ NPL_MG = 1
 SIDES = ("west", "east", "south", "north", "bottom", "top")
 # coarsest levels solved as phi = M rhs: up to 4096 cells each row of M is
 # summed serially by one thread (the form the batched solve shares); larger
-# ones, up to 16384 cells (M = 2 GiB in FP64), in row x column chunks
+# ones, up to 16384 cells, in row x column chunks (FP32, or odd extents: M = 2
+# GiB in FP64) or, in FP64 with even extents, by the level's reflections (an
+# eighth of that)
 COARSE_OPERATOR_MAX_CELLS = 16384
 COARSE_OPERATOR_SERIAL_MAX_CELLS = 4096
 
@@ -110,7 +112,7 @@ class Multigrid:
         # the coarsest solve as a matrix-vector product (M = the n_coarse
         # sweeps from zero) instead of 2 * n_coarse dependent half-sweeps in
         # one workgroup: 80^3 on 3 levels has a 20^3 coarsest level, whose 300
-        # sweeps took 0.67 ms per V-cycle against ~0.1 ms for the 512 MB M
+        # sweeps took 0.67 ms per V-cycle against 0.02 ms for M by reflections
         coarse = self.levels[-1]
         if len(self.levels) > 1 and np.prod(coarse.n3) <= COARSE_OPERATOR_MAX_CELLS:
             coarse.build_coarse_operator(self.n_coarse)
