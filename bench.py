@@ -286,7 +286,7 @@ def hot_kernels(a, s64, smx):
         L0, L1 = lv0.desc(), lv1.desc()
         knob = autotune.SWEEP_PAIRS_F64 if eb == 8 else autotune.SWEEP_PAIRS_F32
         pairs = autotune.get_shape(knob, lv0.n3)
-        two = pairs == 2 or (pairs == 0 and eb == 8 and cells >= 2 ** 23)
+        two = pairs == 2 or (pairs == 0 and cells >= (1750000 if eb == 8 else 3500000))
         ctype = "double" if eb == 8 else "float"
         kern = ("sweep2_kernel<%s> (two RBGS sweeps per launch)" % ctype if two
                 else "sweep_kernel<%s> (one RBGS sweep per launch)" % ctype)
