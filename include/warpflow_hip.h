@@ -393,11 +393,13 @@ int wf_mg_solve(const wf_mg_level* levels, int nlev, const double* su,
 
 /* Coarse operator of a small level: nsweeps RBGS sweeps started from
  * phi = 0 are a fixed linear map phi = M rhs of the level's real cells.
- * wf_mg_coarse_op_build forms M (column-major, ncell x ncell in the level
- * precision; ncell = n0*n1*n2 <= 4096) by running exactly those sweeps on
- * every unit rhs, one workgroup per column.  The V-cycle applies it to the
- * coarsest level, whose phi restriction has just zeroed, when the level's cop
- * is set and cop_sweeps equals the coarsest sweep count -- the same result as
+ * wf_mg_coarse_op_build forms M (ncell = n0*n1*n2 <= 16384 cells in the level
+ * precision: column-major, with a tail of chunk sums above 4096 cells; FP64
+ * levels above 4096 cells of even extents as the blocks of their reflections'
+ * characters, an eighth of ncell^2) by running exactly those sweeps on unit
+ * right-hand sides, one workgroup per column; wf_mg_coarse_op_bytes is the
+ * buffer's size.  The V-cycle applies it to the coarsest level when the level's
+ * cop is set and cop_sweeps equals the coarsest sweep count -- the same result as
  * the sweeps (multigrid.py:313-316) up to rounding, as one matrix-vector
  * product instead of 2*nsweeps dependent half-sweeps. */
 int wf_mg_coarse_op_bytes(const wf_mg_level* lev, size_t* bytes);
