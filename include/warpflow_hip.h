@@ -358,6 +358,16 @@ int wf_mg_refill(const wf_mg_level* lev, void* stream);
  * single-workgroup launch. */
 int wf_mg_relax(const wf_mg_level* lev, int nsweeps, void* stream);
 
+/* How wf_mg_relax runs nsweeps sweeps of lev (no arrays are touched):
+ * out[0] = one of WF_RELAX_*, out[1] = launches; blocks: out[2] = planes of a
+ * block, out[3] = 1 where the level may have fewer planes than that. */
+#define WF_RELAX_BLOCKS 1 /* overlapping blocks, several sweeps per launch */
+#define WF_RELAX_LDS 2    /* the level in one workgroup's LDS */
+#define WF_RELAX_SWEEP2 3 /* two-sweep launches, what is left in smaller ones */
+#define WF_RELAX_SWEEP 4  /* one-sweep launches */
+#define WF_RELAX_HALF 5   /* half-sweep launches */
+int wf_mg_relax_plan(const wf_mg_level* lev, int nsweeps, int32_t* out);
+
 /* _restrict, multigrid.py:93-119, followed by the coarse phi zeroing of
  * multigrid.py:312 (whole coarse array incl. the ring faces). */
 int wf_mg_restrict(const wf_mg_level* fine, const wf_mg_level* coarse,

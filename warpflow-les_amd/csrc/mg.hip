@@ -2340,6 +2340,8 @@ int launch_relax_block_t(const wf_mg_level& L, const void* pin, void* pout, int 
   constexpr int NT = RJK * RJK * NSEG;
   constexpr size_t lds = (size_t)(RI * NSEG + (NSEG > 1 ? 2 : 0)) * PL * sizeof(T);
   auto kern = relax_block_kernel<T, RI, NSEG, PL, NT, PART, PRO>;
+  // a whole block reads and writes all of its planes
+  if (PART ? L.n0 > RI * NSEG : L.n0 < RI * NSEG) return WF_EINVAL;
   if constexpr (lds > 65536) {
     static const hipError_t set = hipFuncSetAttribute(
         (const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -2414,7 +2416,8 @@ bool block_plan(const wf_mg_level& L, int n, bool even, BlockPlan& P) {
     // 32 x 32 columns fill a CU's registers: its second block waits for the first
     const double b = S.rjk == 32 ? std::ceil(blocks / 256.0) * 256.0 : blocks;
     const double cost = Q.launches * (S.base + 1e-3 * S.more * std::max(0.0, b - 256.0));
-    Q.seg = Q.part || (S.rjk == 16 && blocks <= 256);
+    // (eight planes: the part kernel, also where the level has all eight)
+    Q.seg = Q.part || Q.ri == 8 || (S.rjk == 16 && blocks <= 256);
     if (P.launches == 0 || cost < best) {
       P = Q;
       best = cost;
@@ -2423,25 +2426,33 @@ bool block_plan(const wf_mg_level& L, int n, bool even, BlockPlan& P) {
   return P.launches > 0;
 }
 
-template <class T>
-int relax_block(const wf_mg_level& L, const BlockPlan& P, const void* pin, void* pout, int ns,
-                const void* pc, hipStream_t s) {
+// The kernel of a plan: use(BlockKernel<...>{}).
+template <int RI_, int NSEG_, int RJK_, bool PART_>
+struct BlockKernel {
+  static constexpr int RI = RI_, NSEG = NSEG_, RJK = RJK_;
+  static constexpr bool PART = PART_;
+};
+template <class T, class F>
+int block_kernel(const BlockPlan& P, F&& use) {
   if (std::max(P.rj, P.rk) > 16) {
     if constexpr (sizeof(T) == 4)
-      return P.ri == 16
-                 ? launch_relax_block<T, 16, 1, 32, false>(L, pin, pout, ns, P.rj, P.rk, pc, s)
-                 : launch_relax_block<T, 20, 1, 32, false>(L, pin, pout, ns, P.rj, P.rk, pc, s);
+      return P.ri == 16 ? use(BlockKernel<16, 1, 32, false>{}) : use(BlockKernel<20, 1, 32, false>{});
     return WF_EINVAL;
   }
   const bool p = P.part;
-  auto run = [&](auto f) { return f(L, pin, pout, ns, P.rj, P.rk, pc, s); };
   if (!P.seg)
-    return run(P.ri == 12 ? launch_relax_block<T, 12, 1, 16, false>
-                          : launch_relax_block<T, 16, 1, 16, false>);
-  if (P.ri == 8) return run(launch_relax_block<T, 4, 2, 16, true>);
+    return P.ri == 12 ? use(BlockKernel<12, 1, 16, false>{}) : use(BlockKernel<16, 1, 16, false>{});
+  if (P.ri == 8) return use(BlockKernel<4, 2, 16, true>{});
   if (P.ri == 12)
-    return run(p ? launch_relax_block<T, 4, 3, 16, true> : launch_relax_block<T, 4, 3, 16, false>);
-  return run(p ? launch_relax_block<T, 4, 4, 16, true> : launch_relax_block<T, 4, 4, 16, false>);
+    return p ? use(BlockKernel<4, 3, 16, true>{}) : use(BlockKernel<4, 3, 16, false>{});
+  return p ? use(BlockKernel<4, 4, 16, true>{}) : use(BlockKernel<4, 4, 16, false>{});
+}
+template <class T>
+int relax_block(const wf_mg_level& L, const BlockPlan& P, const void* pin, void* pout, int ns,
+                const void* pc, hipStream_t s) {
+  return block_kernel<T>(P, [&](auto K) {
+    return launch_relax_block<T, K.RI, K.NSEG, K.RJK, K.PART>(L, pin, pout, ns, P.rj, P.rk, pc, s);
+  });
 }
 
 // nsweeps RBGS sweeps of L.  Pairs of sweeps run as two-sweep launches
@@ -2482,6 +2493,19 @@ template <class T>
 bool relax_prolong_ok(const wf_mg_level& L, int nsweeps) {
   BlockPlan P;
   return nsweeps > 0 && relax_path<T>(L, nsweeps, false, P) == RelaxPath::BLOCKS;
+}
+
+// Two-sweep launches of nsweeps sweeps by full-sweep kernels; without allow_swap
+// an even number of them.
+template <class T>
+int sweep_pairs(const wf_mg_level& L, int nsweeps, bool allow_swap) {
+  const size_t cells = (size_t)L.n0 * L.n1 * L.n2;
+  const int pairs = tune_get(sizeof(T) == 8 ? WF_TUNE_SWEEP_PAIRS_F64 : WF_TUNE_SWEEP_PAIRS_F32,
+                             L.n0, L.n1, L.n2);
+  // built-in: the levels too large for blocks (block_plan)
+  const bool two = pairs == 2 || (pairs == 0 && cells >= (sizeof(T) == 8 ? 1750000u : 3500000u));
+  if (!L.tmp || !two) return 0;
+  return allow_swap ? nsweeps / 2 : (nsweeps / 2) & ~1;
 }
 
 // zero_start: the iterate in L.phi is to be taken as zero (the caller has
@@ -2526,19 +2550,12 @@ int relax_t(const wf_mg_level& L, int nsweeps, hipStream_t s, bool allow_swap = 
     zero_start = false;
     return r;
   };
-  int q = 0;
-  const int pairs = tune_get(sizeof(T) == 8 ? WF_TUNE_SWEEP_PAIRS_F64 : WF_TUNE_SWEEP_PAIRS_F32,
-                             L.n0, L.n1, L.n2);
-  // built-in: two-sweep launches on the levels too large for blocks (block_plan)
-  if (C.tmp && (pairs == 2 || (pairs == 0 && cells >= (sizeof(T) == 8 ? 1750000u : 3500000u)))) {
-    int npair = nsweeps / 2;
-    if (!allow_swap) npair &= ~1;
-    for (int f = 0; f < npair; ++f) {
-      WF_TRY((hipError_t)sweep2_t<T>(C, src(C.phi), C.tmp, s));
-      std::swap(C.phi, C.tmp);
-    }
-    q = 2 * npair;
+  const int npair = sweep_pairs<T>(L, nsweeps, allow_swap);
+  for (int f = 0; f < npair; ++f) {
+    WF_TRY((hipError_t)sweep2_t<T>(C, src(C.phi), C.tmp, s));
+    std::swap(C.phi, C.tmp);
   }
+  int q = 2 * npair;
   if (C.tmp) {
     for (; q + 1 < nsweeps; q += 2) {
       WF_TRY((hipError_t)sweep_t<T>(C, src(C.phi), C.tmp, s));
@@ -2550,6 +2567,34 @@ int relax_t(const wf_mg_level& L, int nsweeps, hipStream_t s, bool allow_swap = 
     WF_TRY((hipError_t)launch_rbgs<T>(C, 1, 1, s));
   }
   if (swapped) *swapped = C.phi != L.phi;
+  return 0;
+}
+
+// wf_mg_relax_plan: the choices relax_t makes without allow_swap.
+template <class T>
+int relax_plan_t(const wf_mg_level& L, int nsweeps, int32_t* out) {
+  out[0] = out[1] = out[2] = out[3] = 0;
+  if (nsweeps <= 0) return 0;
+  BlockPlan P;
+  const RelaxPath path = relax_path<T>(L, nsweeps, true, P);
+  if (path == RelaxPath::BLOCKS) {
+    out[0] = WF_RELAX_BLOCKS;
+    out[1] = P.launches;
+    return block_kernel<T>(P, [&](auto K) {
+      out[2] = K.RI * K.NSEG;
+      out[3] = K.PART;
+      return 0;
+    });
+  }
+  if (path != RelaxPath::SWEEPS) {
+    out[0] = WF_RELAX_LDS;
+    out[1] = 1;
+    return 0;
+  }
+  const int npair = sweep_pairs<T>(L, nsweeps, false), rest = nsweeps - 2 * npair;
+  const int full = L.tmp ? rest & ~1 : 0;  // one-sweep launches
+  out[0] = npair ? WF_RELAX_SWEEP2 : full ? WF_RELAX_SWEEP : WF_RELAX_HALF;
+  out[1] = npair + full + 2 * (rest - full);
   return 0;
 }
 
@@ -2952,6 +2997,12 @@ int wf_mg_refill(const wf_mg_level* L, void* stream) {
 int wf_mg_relax(const wf_mg_level* L, int nsweeps, void* stream) {
   if (!level_ok(L) || nsweeps < 0) return WF_EINVAL;
   return relax_any(*L, nsweeps, S_(stream));
+}
+
+int wf_mg_relax_plan(const wf_mg_level* L, int nsweeps, int32_t* out) {
+  if (!level_ok(L) || nsweeps < 0 || !out) return WF_EINVAL;
+  return L->prec == 8 ? relax_plan_t<double>(*L, nsweeps, out)
+                      : relax_plan_t<float>(*L, nsweeps, out);
 }
 
 int wf_mg_restrict(const wf_mg_level* F, const wf_mg_level* C, void* stream) {

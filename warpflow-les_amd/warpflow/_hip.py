@@ -141,6 +141,7 @@ _SIGS = {
     "wf_mg_rbgs": [_L, _I, _P],
     "wf_mg_refill": [_L, _P],
     "wf_mg_relax": [_L, _I, _P],
+    "wf_mg_relax_plan": [_L, _I, C.POINTER(C.c_int32)],
     "wf_mg_restrict": [_L, _L, _P],
     "wf_mg_prolong": [_L, _L, _P],
     "wf_mg_copy_in": [_P, _G, _L, _P],
