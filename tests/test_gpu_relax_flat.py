@@ -53,9 +53,11 @@ def test_flat_levels_equal_one_sweep_launches(gpu, prec, n3):
         autotune.reset()
 
 
-# through the V-cycle: the flat level 1 takes its interpolation in the first launch
+# through the V-cycle: a level may relax by another kernel before the coarse
+# correction than after it, where blocks also add the interpolation
 @pytest.mark.parametrize("prec", PRECS)
-@pytest.mark.parametrize("n3", [(16, 160, 160), (16, 62, 512)])
+@pytest.mark.parametrize("n3", [(16, 160, 160), (16, 62, 512), (8, 1024, 1024), (4, 48, 40),
+                                (2, 20, 40), (40, 16, 24)])
 def test_flat_hierarchy_equals_one_sweep_launches(gpu, prec, n3):
     from warpflow import _hip, autotune
     from warpflow.multigrid import _Level

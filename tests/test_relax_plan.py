@@ -33,3 +33,19 @@ def test_block_planes_fit_the_level(prec, tmp):
                         blocks += 1
                         assert (n0 <= planes) if part else (n0 >= planes), (n0, n1, n2, n)
     assert blocks
+
+
+# small levels with an extent above 16 (one LDS launch takes every sweep) and
+# levels of a few planes with many columns (blocks would be mostly halo) keep
+# the launches that are faster there; blocks elsewhere
+@pytest.mark.parametrize("n3,prec,nsweeps,kind", [
+    ((4, 8, 64), 8, 300, LDS), ((2, 8, 24), 4, 300, LDS), ((20, 20, 20), 4, 300, LDS),
+    ((24, 12, 32), 4, 300, BLOCKS), ((27, 27, 27), 8, 300, BLOCKS),
+    ((2, 20, 6), 4, 6, LDS), ((1, 10, 20), 8, 6, LDS), ((24, 24, 24), 4, 6, BLOCKS),
+    ((1, 1024, 1024), 4, 6, SWEEP), ((2, 512, 512), 8, 6, SWEEP), ((4, 512, 512), 4, 6, SWEEP),
+    ((4, 512, 512), 8, 6, SWEEP), ((4, 256, 256), 4, 6, BLOCKS), ((8, 256, 256), 8, 6, BLOCKS),
+    ((16, 256, 256), 4, 6, BLOCKS), ((512, 2, 512), 4, 6, BLOCKS), ((512, 512, 2), 8, 6, BLOCKS),
+    ((12, 12, 12), 8, 300, BLOCKS), ((16, 16, 16), 4, 6, BLOCKS), ((32, 32, 32), 4, 300, BLOCKS),
+    ((128, 128, 128), 4, 6, BLOCKS), ((80, 80, 80), 8, 6, BLOCKS)])
+def test_faster_smoother_is_taken(n3, prec, nsweeps, kind):
+    assert plan(n3, prec, nsweeps)[0] == kind

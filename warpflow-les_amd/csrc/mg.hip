@@ -2208,6 +2208,11 @@ int launch_relax_lds(const wf_mg_level& L, int nsweeps, size_t bytes, hipStream_
 constexpr size_t LDS_RELAX_MAX_CELLS = 4096;
 constexpr int LDS_RELAX_MIN_SWEEPS = 32;
 
+// i-planes per workgroup of the one-sweep launches where none was tuned
+inline int sweep_ich(int64_t tiles, int n0) {
+  return (int)std::max<int64_t>(4, std::min<int64_t>(16, tiles * n0 / 2048));
+}
+
 template <class T, int TJ, int TK>
 int launch_sweep(const wf_mg_level& L, const void* pin, void* pout, hipStream_t s) {
   const MgDev d = mg_dev(L);
@@ -2232,8 +2237,7 @@ int launch_sweep(const wf_mg_level& L, const void* pin, void* pout, hipStream_t 
     WF_LAUNCHED();
     return 0;
   }
-  int ich = tuned > 0 ? tuned
-                      : (int)std::max<int64_t>(4, std::min<int64_t>(16, tiles * d.n0 / 2048));
+  int ich = tuned > 0 ? tuned : sweep_ich(tiles, d.n0);
   // the kernel's plane offsets within a chunk ((ich + 3) planes) stay below 2^30
   if ((int64_t)4 * pb >= ((int64_t)1 << 30)) return WF_EINVAL;
   ich = (int)std::min<int64_t>(ich, ((int64_t)1 << 30) / pb - 3);
@@ -2331,6 +2335,7 @@ struct BlockPlan {
   int ri = 0, rj = 0, rk = 0;
   bool part = false, seg = false;
   int launches = 0;
+  double us = 0;  // estimate for this level (block_cheaper); 0: one block, in place
 };
 
 template <class T, int RI, int NSEG, int RJK, bool PART, bool PRO>
@@ -2367,8 +2372,8 @@ int launch_relax_block(const wf_mg_level& L, const void* pin, void* pout, int ns
 }
 
 // The plan for n sweeps; even: the launches come in even numbers (the result
-// in phi).  False where blocks don't apply: a level tuned to another kernel,
-// one streaming is faster on, a level without tmp that is more than one block.
+// in phi).  False where blocks don't apply: a level tuned to another kernel, one
+// of many cells, a level without tmp that is more than one block.
 template <class T>
 bool block_plan(const wf_mg_level& L, int n, bool even, BlockPlan& P) {
   constexpr bool f64 = sizeof(T) == 8;
@@ -2421,6 +2426,13 @@ bool block_plan(const wf_mg_level& L, int n, bool even, BlockPlan& P) {
     if (P.launches == 0 || cost < best) {
       P = Q;
       best = cost;
+      // a block that the level fills in part costs less: its launch in
+      // proportion, a further block half by its planes and by its columns
+      constexpr double b0 = f64 ? 4.4 : 3.85;
+      const double cf = (double)(Q.rj * Q.rk) / (S.rjk * S.rjk), pf = (double)Q.ri / S.ri;
+      P.us = Q.launches * (b0 + (S.base - b0) * pf * cf +
+                           1e-3 * S.more * std::max(0.0, b - 256.0) * (1 + pf) / 2 *
+                               (0.2 + 0.8 * cf));
     }
   }
   return P.launches > 0;
@@ -2455,16 +2467,10 @@ int relax_block(const wf_mg_level& L, const BlockPlan& P, const void* pin, void*
   });
 }
 
-// nsweeps RBGS sweeps of L.  Pairs of sweeps run as two-sweep launches
-// (phi -> tmp, then tmp -> phi, ...); with allow_swap an odd number of them
-// may leave the result in tmp, which *swapped reports (the caller then
-// treats tmp as the level's phi); without it the pairs go in even numbers
-// and the rest as one-sweep launches, so the result is in phi.
-// Which smoother relax_t runs for nsweeps sweeps of level L.
 enum class RelaxPath { BLOCKS, LDS2, LDS_RHS, LDS, SWEEPS };
+// The smoother of nsweeps sweeps where blocks are not taken.
 template <class T>
-RelaxPath relax_path(const wf_mg_level& L, int nsweeps, bool even, BlockPlan& P) {
-  if (block_plan<T>(L, nsweeps, even, P)) return RelaxPath::BLOCKS;
+RelaxPath stream_path(const wf_mg_level& L, int nsweeps) {
   const size_t cells = (size_t)L.n0 * L.n1 * L.n2;
   const size_t lds = (size_t)max_lds();
   // levels whose zero-ringed copy fits LDS: all sweeps in one workgroup
@@ -2477,12 +2483,54 @@ RelaxPath relax_path(const wf_mg_level& L, int nsweeps, bool even, BlockPlan& P)
   if (cells <= LDS_RELAX_MAX_CELLS && cells * sizeof(T) <= lds) return RelaxPath::LDS;
   return RelaxPath::SWEEPS;
 }
-// True when relax_t's first launch for nsweeps sweeps of L is a full-sweep or
-// block kernel, which can take a zero iterate without reading it (zero_start).
+// Whether the blocks of plan P take nsweeps sweeps faster than stream_path does.
+// Blocks lose on two kinds of level.  Small ones with an extent above 16, whose
+// sweeps take one LDS launch however many they are, while blocks are launched
+// every third (300 sweeps of 4 x 8 x 64 cells in FP64: 124 us against 474; six
+// of 2 x 20 x 6: 5.5 against 7.8 in FP32).  And levels of a few planes with many
+// columns, where a block is mostly halo (six sweeps of 1 x 1024 x 1024 in FP32 92
+// us streamed, 299 by blocks; 4 x 512 x 512 57 and 82; 8 x 256 x 256 45 and 27).
+// The estimates are fits to 1600 levels of each type with 6, 12 and 300 sweeps
+// (wrong by more than 10% in time on 3% of them); one block in place is faster
+// than both from a few sweeps on.
+// fused: blocks also save the prolongation's launch.
+template <class T>
+bool block_cheaper(const wf_mg_level& L, int nsweeps, const BlockPlan& P, bool fused) {
+  constexpr bool f64 = sizeof(T) == 8;
+  if (P.us == 0) return true;
+  const double us = P.us - (fused ? 4.0 : 0.0);
+  switch (stream_path<T>(L, nsweeps)) {
+    case RelaxPath::LDS2: {  // cells per thread: loads and stores, then two passes a sweep
+      const int c = relax_lds2_cpt(L);
+      return us <= (f64 ? 3.5 : 3.2) + 1.8 * c +
+                       nsweeps * (f64 ? 0.16 + 0.40 * c : 0.11 + 0.32 * c);
+    }
+    case RelaxPath::SWEEPS: {  // a chunk's planes, and each further round of workgroups
+      const int64_t tiles = L.n2 > 32 ? (int64_t)div_up(L.n2, 64) * div_up(L.n1, 8)
+                                      : (int64_t)div_up(L.n2, 32) * div_up(L.n1, 16);
+      const int ich = sweep_ich(tiles, L.n0), p = std::min(ich, L.n0);
+      const double more = std::max<double>(0, (double)tiles * div_up(L.n0, ich) / 256 - 1);
+      return us <= nsweeps * (f64 ? 5.6 + 0.75 * p + (2.0 + 0.25 * p) * more
+                                  : 4.9 + 0.6 * p + (1.1 + 0.22 * p) * more);
+    }
+    default:  // 1700 to 3500 us for 300 sweeps that take blocks 500 to 700
+      return true;
+  }
+}
+// Which smoother relax_t runs for nsweeps sweeps of level L.
+template <class T>
+RelaxPath relax_path(const wf_mg_level& L, int nsweeps, bool even, bool fused, BlockPlan& P) {
+  if (block_plan<T>(L, nsweeps, even, P) && block_cheaper<T>(L, nsweeps, P, fused))
+    return RelaxPath::BLOCKS;
+  return stream_path<T>(L, nsweeps);
+}
+// True when relax_t's first launch for nsweeps sweeps of L (allow_swap) is a
+// full-sweep or block kernel, which can take a zero iterate without reading it
+// (zero_start).
 template <class T>
 bool relax_zero_start_ok(const wf_mg_level& L, int nsweeps) {
   BlockPlan P;
-  const RelaxPath p = relax_path<T>(L, nsweeps, true, P);
+  const RelaxPath p = relax_path<T>(L, nsweeps, false, false, P);
   return nsweeps >= 2 && L.tmp && (p == RelaxPath::BLOCKS || p == RelaxPath::SWEEPS);
 }
 
@@ -2492,7 +2540,7 @@ bool relax_zero_start_ok(const wf_mg_level& L, int nsweeps) {
 template <class T>
 bool relax_prolong_ok(const wf_mg_level& L, int nsweeps) {
   BlockPlan P;
-  return nsweeps > 0 && relax_path<T>(L, nsweeps, false, P) == RelaxPath::BLOCKS;
+  return nsweeps > 0 && relax_path<T>(L, nsweeps, false, true, P) == RelaxPath::BLOCKS;
 }
 
 // Two-sweep launches of nsweeps sweeps by full-sweep kernels; without allow_swap
@@ -2508,6 +2556,11 @@ int sweep_pairs(const wf_mg_level& L, int nsweeps, bool allow_swap) {
   return allow_swap ? nsweeps / 2 : (nsweeps / 2) & ~1;
 }
 
+// nsweeps RBGS sweeps of L.  Pairs of sweeps run as two-sweep launches
+// (phi -> tmp, then tmp -> phi, ...); with allow_swap an odd number of them
+// may leave the result in tmp, which *swapped reports (the caller then
+// treats tmp as the level's phi); without it the pairs go in even numbers
+// and the rest as one-sweep launches, so the result is in phi.
 // zero_start: the iterate in L.phi is to be taken as zero (the caller has
 // not zeroed it); only valid when relax_zero_start_ok.  coarse: the next level's
 // iterate, still to be prolonged onto L; only when relax_prolong_ok.
@@ -2517,8 +2570,9 @@ int relax_t(const wf_mg_level& L, int nsweeps, hipStream_t s, bool allow_swap = 
   if (swapped) *swapped = false;
   if (nsweeps <= 0) return 0;
   const size_t cells = (size_t)L.n0 * L.n1 * L.n2;
+  if (zero_start && !relax_zero_start_ok<T>(L, nsweeps)) return WF_EINVAL;
   BlockPlan P;
-  switch (relax_path<T>(L, nsweeps, !allow_swap, P)) {
+  switch (relax_path<T>(L, nsweeps, !allow_swap, coarse != nullptr, P)) {
     case RelaxPath::BLOCKS: {
       const void* in = zero_start ? nullptr : L.phi;
       if (P.launches == 1 && L.n0 <= 16 && L.n1 <= 16 && L.n2 <= 16)
@@ -2542,7 +2596,6 @@ int relax_t(const wf_mg_level& L, int nsweeps, hipStream_t s, bool allow_swap = 
     case RelaxPath::SWEEPS:
       break;
   }
-  if (zero_start && !relax_zero_start_ok<T>(L, nsweeps)) return WF_EINVAL;
   wf_mg_level C = L;  // C.phi holds the current iterate
   // the first launch reads the zero iterate through an empty descriptor
   auto src = [&](const void* p) -> const void* {
@@ -2576,7 +2629,7 @@ int relax_plan_t(const wf_mg_level& L, int nsweeps, int32_t* out) {
   out[0] = out[1] = out[2] = out[3] = 0;
   if (nsweeps <= 0) return 0;
   BlockPlan P;
-  const RelaxPath path = relax_path<T>(L, nsweeps, true, P);
+  const RelaxPath path = relax_path<T>(L, nsweeps, true, false, P);
   if (path == RelaxPath::BLOCKS) {
     out[0] = WF_RELAX_BLOCKS;
     out[1] = P.launches;
