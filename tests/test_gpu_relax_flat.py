@@ -79,3 +79,14 @@ def test_flat_hierarchy_equals_one_sweep_launches(gpu, prec, n3):
             assert np.array_equal(a, b)
     finally:
         autotune.reset()
+
+
+# planes of 121 MB: one-sweep launches, where two-sweep ones would be refused
+def test_wide_planes_relax(gpu):
+    from warpflow import _hip
+    from warpflow.device import zeros
+    n3 = (10, 5500, 5500)
+    phi, rhs, tmp = [zeros(tuple(n + 2 for n in n3), np.float32) for _ in range(3)]
+    d = _hip.WfMgLevel(phi.ptr, rhs.ptr, *n3, 4, *(1.0 / n for n in n3), tmp.ptr, None, 0, 0)
+    _hip.call("wf_mg_relax", C.byref(d), 2, None)
+    _hip.call("wf_synchronize")

@@ -49,3 +49,11 @@ def test_block_planes_fit_the_level(prec, tmp):
     ((128, 128, 128), 4, 6, BLOCKS), ((80, 80, 80), 8, 6, BLOCKS)])
 def test_faster_smoother_is_taken(n3, prec, nsweeps, kind):
     assert plan(n3, prec, nsweeps)[0] == kind
+
+
+# planes whose offsets in a two-sweep chunk pass 2^30 bytes take one-sweep launches
+@pytest.mark.parametrize("n3,prec,kind", [
+    ((16, 5500, 5500), 4, SWEEP), ((16, 8000, 8000), 4, SWEEP), ((16, 5400, 5400), 4, SWEEP2),
+    ((16, 3900, 3900), 8, SWEEP), ((16, 3800, 3800), 8, SWEEP2)])
+def test_wide_planes_are_not_refused(n3, prec, kind):
+    assert plan(n3, prec, 6)[0] == kind

@@ -2267,6 +2267,12 @@ int sweep_t(const wf_mg_level& L, const void* pin, void* pout, hipStream_t s) {
   }
 }
 
+// Whether the two-sweep kernel can address the level's planes.
+template <class T>
+bool sweep2_fits(const wf_mg_level& L) {
+  return 9 * mg_dev(L).s0 * (int64_t)sizeof(T) < ((int64_t)1 << 30);
+}
+
 template <class T, int TJ, int TK>
 int launch_sweep2(const wf_mg_level& L, const void* pin, void* pout, hipStream_t s) {
   const MgDev d = mg_dev(L);
@@ -2277,8 +2283,8 @@ int launch_sweep2(const wf_mg_level& L, const void* pin, void* pout, hipStream_t
   const int tuned = tune_get(sizeof(T) == 8 ? WF_TUNE_SWEEP2_ICH_F64 : WF_TUNE_SWEEP2_ICH_F32,
                              d.n0, d.n1, d.n2);
   // the kernel's plane offsets within a chunk ((ich + 8) planes) stay below 2^30
+  if (!sweep2_fits<T>(L)) return WF_EINVAL;
   const int64_t pb = d.s0 * (int64_t)sizeof(T);
-  if ((int64_t)9 * pb >= ((int64_t)1 << 30)) return WF_EINVAL;
   // Chunks that fill the chip once: a CU holds three (FP32) or two (FP64)
   // workgroups of the 8 x 64 and 16 x 32 tiles, and a chunk of ich planes runs
   // ich + 9 iterations, so the fewest chunks that occupy it lose the least to
@@ -2550,8 +2556,10 @@ int sweep_pairs(const wf_mg_level& L, int nsweeps, bool allow_swap) {
   const size_t cells = (size_t)L.n0 * L.n1 * L.n2;
   const int pairs = tune_get(sizeof(T) == 8 ? WF_TUNE_SWEEP_PAIRS_F64 : WF_TUNE_SWEEP_PAIRS_F32,
                              L.n0, L.n1, L.n2);
-  // built-in: the levels too large for blocks (block_plan)
-  const bool two = pairs == 2 || (pairs == 0 && cells >= (sizeof(T) == 8 ? 1750000u : 3500000u));
+  // built-in: the levels too large for blocks (block_plan), but for planes that
+  // only the one-sweep kernel can address
+  const bool two = pairs == 2 || (pairs == 0 && sweep2_fits<T>(L) &&
+                                  cells >= (sizeof(T) == 8 ? 1750000u : 3500000u));
   if (!L.tmp || !two) return 0;
   return allow_swap ? nsweeps / 2 : (nsweeps / 2) & ~1;
 }
