@@ -57,3 +57,15 @@ def test_faster_smoother_is_taken(n3, prec, nsweeps, kind):
     ((16, 3900, 3900), 8, SWEEP), ((16, 3800, 3800), 8, SWEEP2)])
 def test_wide_planes_are_not_refused(n3, prec, kind):
     assert plan(n3, prec, 6)[0] == kind
+
+
+# large levels of few planes or rows: a two-sweep chunk would be mostly the
+# planes and rows around it
+@pytest.mark.parametrize("n3,prec,kind", [
+    ((4, 1056, 1056), 4, SWEEP), ((8, 744, 744), 4, SWEEP), ((12, 608, 608), 4, SWEEP2),
+    ((1224, 8, 1224), 4, SWEEP), ((608, 12, 608), 4, SWEEP2), ((608, 608, 12), 4, SWEEP2),
+    ((1496, 1496, 2), 4, SWEEP2), ((2, 1048, 1048), 8, SWEEP), ((8, 520, 520), 8, SWEEP),
+    ((8, 1224, 1224), 8, SWEEP2), ((10, 464, 464), 8, SWEEP2), ((256, 256, 256), 4, SWEEP2),
+    ((128, 128, 128), 8, SWEEP2)])
+def test_large_flat_levels(n3, prec, kind):
+    assert plan(n3, prec, 6)[0] == kind

@@ -2557,9 +2557,16 @@ int sweep_pairs(const wf_mg_level& L, int nsweeps, bool allow_swap) {
   const int pairs = tune_get(sizeof(T) == 8 ? WF_TUNE_SWEEP_PAIRS_F64 : WF_TUNE_SWEEP_PAIRS_F32,
                              L.n0, L.n1, L.n2);
   // built-in: the levels too large for blocks (block_plan), but for planes that
-  // only the one-sweep kernel can address
+  // only the one-sweep kernel can address, and for levels of few planes or rows: a
+  // chunk runs nine planes, and a tile four rows on each side, past its own.  Six
+  // sweeps, one- / two-sweep launches: FP32 4 x 1056 x 1056 135 / 170 us, 1224 x 8
+  // x 1224 213 / 320, 8 x 1224 x 1224 236 / 267, 12 x 1000 x 1000 346 / 222; FP64 8 x
+  // 520 x 520 126 / 138, 10 x 464 x 464 133 / 96, 4 x 1728 x 1728 671 / 725, 8 x
+  // 1224 x 1224 570 / 489.
+  const int few = sizeof(T) == 8 && cells >= ((size_t)1 << 23) ? 5 : 8;
   const bool two = pairs == 2 || (pairs == 0 && sweep2_fits<T>(L) &&
-                                  cells >= (sizeof(T) == 8 ? 1750000u : 3500000u));
+                                  cells >= (sizeof(T) == 8 ? 1750000u : 3500000u) &&
+                                  std::min(L.n0, L.n1) > few);
   if (!L.tmp || !two) return 0;
   return allow_swap ? nsweeps / 2 : (nsweeps / 2) & ~1;
 }
