@@ -140,6 +140,7 @@ struct BatchRelax {
   bool single = false;  // every member is one block: all sweeps in one launch, in place
   int rjk = 0, ns = 0;  // blocks: rows and columns, sweeps per launch
   int ich = 0;          // > 0: two-sweep launches in chunks of ich planes instead
+  double us = 0;        // estimate of a launch
 };
 
 // Host side of a batch (defined in batch.hip).

@@ -1219,12 +1219,15 @@ relax_block_kernel(const T* __restrict__ pin, T* pout, const T* __restrict__ rhs
                                                reinterpret_cast<T*>(smem_raw), pc);
 }
 
+constexpr int LDS_RELAX_MAX_CELLS = 4096;
+
 // n sweeps of RBGS on one small level held in LDS by one workgroup
 // (multigrid.py:289-299 with the refill folded in).  The real cells of phi
 // live in LDS; ring terms carry zero coefficients and are skipped.  rhs is
-// in LDS too when RHS_LDS, else read from global memory (L2-resident).
+// in LDS too when RHS_LDS, else read from global memory (L2-resident).  pin: phi,
+// or nullptr for an iterate of zeros.
 template <class T, bool RHS_LDS>
-__device__ inline void relax_lds_body(T* __restrict__ phi, const T* __restrict__ rhs,
+__device__ inline void relax_lds_body(const T* pin, T* phi, const T* __restrict__ rhs,
                                       const MgDev& d, T c0, T c1, T c2, int nsweeps, T* sp) {
   const int n0 = d.n0, n1 = d.n1, n2 = d.n2;
   const int ncell = n0 * n1 * n2;
@@ -1233,7 +1236,7 @@ __device__ inline void relax_lds_body(T* __restrict__ phi, const T* __restrict__
   for (int l = tid; l < ncell; l += nt) {
     const int k = l % n2, j = (l / n2) % n1, i = l / (n1 * n2);
     const int64_t x = mg_at(d, i, j, k);
-    sp[l] = phi[x];
+    sp[l] = pin ? pin[x] : T(0);
     if (RHS_LDS) sr[l] = rhs[x];
   }
   __syncthreads();
@@ -1275,7 +1278,7 @@ __global__ void __launch_bounds__(1024)
 relax_lds_kernel(T* __restrict__ phi, const T* __restrict__ rhs, MgDev d, T c0, T c1, T c2,
                  int nsweeps) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  relax_lds_body<T, RHS_LDS>(phi, rhs, d, c0, c1, c2, nsweeps, reinterpret_cast<T*>(smem_raw));
+  relax_lds_body<T, RHS_LDS>(phi, phi, rhs, d, c0, c1, c2, nsweeps, reinterpret_cast<T*>(smem_raw));
 }
 
 // n sweeps of RBGS on one level held in LDS by one workgroup of 1024 threads,
@@ -1912,6 +1915,20 @@ batch_sweep2_kernel(BView V, const int4* item, int l, int ich, const float* pin,
                              M->lc[l][1], M->lc[l][2], ich, B);
 }
 
+// n sweeps of level l in LDS, a workgroup per member (levels of at most
+// LDS_RELAX_MAX_CELLS cells; batch_relax_in_lds)
+__global__ void __launch_bounds__(1024)
+batch_relax_lds_kernel(BView V, int l, const float* pin, float* phi, const float* rhs,
+                       int nsweeps, const int* active) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int m = blockIdx.x;
+  if (active && !active[m]) return;  // uniform per workgroup
+  const MemDev& M = V.mem[m];
+  const int64_t o = M.loff[l];
+  relax_lds_body<float, true>(pin ? pin + o : nullptr, phi + o, rhs + o, level_dev(M, l),
+                              M.lc[l][0], M.lc[l][1], M.lc[l][2], nsweeps,
+                              reinterpret_cast<float*>(smem_raw));
+}
 // phi = M rhs on the coarsest level l, a workgroup per member and COP_ROWS rows
 // (one per member took 177 us where a member's M is 1728^2, as long as that
 // member alone)
@@ -1971,6 +1988,7 @@ void batch_relax_plan(const MemDev* mem, int nmem, int l, BatchRelax& P,
       best = cost;
       P.rjk = S.rjk;
       P.ns = S.ns;
+      P.us = cost * S.ns / 6;
     }
     if (P.single) break;
   }
@@ -1990,6 +2008,7 @@ void batch_relax_plan(const MemDev* mem, int nmem, int l, BatchRelax& P,
     if (cost < best) {
       best = cost;
       P.ich = ich;
+      P.us = cost / 3;
     }
   }
   if (P.ich) P.ns = 2;
@@ -2011,6 +2030,23 @@ void batch_relax_plan(const MemDev* mem, int nmem, int l, BatchRelax& P,
   P.total = (int)items.size();
 }
 
+// Whether n sweeps of level l run in LDS, all in one launch of a workgroup per
+// member: where that is faster than the plan's launches, and where the plan has
+// none for an odd sweep.  300 sweeps, plan / LDS: 64 members of 32 x 8 x 8 cells 708
+// / 445 us, of 24 x 12 x 12 545 / 708; 300 of 2 x 24 x 48 2805 / 891; six sweeps of
+// 300 of 4 x 8 x 64 33 / 24, of 8 x 16 x 24 13 / 33.  fused: blocks also save the
+// prolongation's launch.
+static bool batch_relax_in_lds(const Batch& B, int l, int n, bool fused) {
+  const BatchRelax& P = B.relax[l];
+  if (P.single || B.max_lds_cells[l] > LDS_RELAX_MAX_CELLS) return false;
+  if (P.ich && n % 2) return true;
+  // the loads, then two passes a sweep; further rounds of workgroups overlap a little
+  const double c = B.max_lds_cells[l] / 1024.0;
+  const double lds = (1.0 + 1.1 * c + n * (0.55 + 0.545 * c)) *
+                     (1.0 + 0.85 * (div_up(B.nmem, 256) - 1));
+  return lds < div_up(n, P.ns) * P.us - (fused ? 4.0 : 0.0);
+}
+
 // One batched V-cycle of the FP32 levels (vcycle_any's order); zero0: level 0's
 // iterate is taken as zero without being read (its first relaxation has sweeps).
 int batch_vcycle(const Batch& B, float* const* phi_, float* const* rhs, float* const* tmp_,
@@ -2028,17 +2064,22 @@ int batch_vcycle(const Batch& B, float* const* phi_, float* const* rhs, float* c
   auto relax = [&](int l, int n, bool zero, const float* pc) -> int {
     if (n <= 0) return 0;
     const BatchRelax& P = B.relax[l];
-    if (n % 2 && B.max_lds_cells[l] > 4096) return WF_EINVAL;
+    if (n % 2 && B.max_lds_cells[l] > LDS_RELAX_MAX_CELLS) return WF_EINVAL;
     const float* in = zero ? nullptr : phi[l];
+    if (!pc && batch_relax_in_lds(B, l, n, false)) {
+      hipLaunchKernelGGL(batch_relax_lds_kernel, dim3(B.nmem), dim3(1024),
+                         2 * B.max_lds_cells[l] * sizeof(float), s, V, l, in, phi[l],
+                         (const float*)rhs[l], n, active);
+      WF_LAUNCHED();
+      return 0;
+    }
     const int launches = P.single ? 1 : div_up(n, P.ns);
     for (int q = 0; q < launches; ++q) {
       const int ns = n / launches + (q < n % launches);
       float* const out = P.single ? phi[l] : tmp[l];
-      if (P.ich && ns == 2) {
+      if (P.ich) {  // ns = 2: an odd n has gone to LDS or been refused
         hipLaunchKernelGGL(batch_sweep2_kernel, dim3(P.total), dim3(256), 0, s, V, P.item, l,
                            P.ich, in, out, (const float*)rhs[l], active);
-      } else if (P.ich) {
-        return WF_EINVAL;  // (levels this large take even numbers of sweeps)
       } else {
         auto run = [&](auto kern, int nt, int words) {
           hipLaunchKernelGGL(kern, dim3(P.total), dim3(nt), words * sizeof(float), s, V, P.item,
@@ -2081,7 +2122,7 @@ int batch_vcycle(const Batch& B, float* const* phi_, float* const* rhs, float* c
   }
   for (int l = nlev - 2; l >= 0; --l) {
     // blocks add the interpolation as they read the iterate
-    const bool fused = npost > 0 && !B.relax[l].ich;
+    const bool fused = npost > 0 && !B.relax[l].ich && !batch_relax_in_lds(B, l, npost, true);
     if (!fused) {
       const Plan& P = B.plan[PK_LCELLS0 + l + 1];
       hipLaunchKernelGGL(batch_prolong8_kernel, dim3(P.total), dim3(64, 4), 0, s, V, P, l,
@@ -2213,7 +2254,6 @@ int launch_relax_lds(const wf_mg_level& L, int nsweeps, size_t bytes, hipStream_
 // asked for many sweeps (the coarsest solve) -- relax in one LDS-resident
 // workgroup; the rest in fused full-sweep launches (or half-sweep launches
 // without tmp).
-constexpr size_t LDS_RELAX_MAX_CELLS = 4096;
 constexpr int LDS_RELAX_MIN_SWEEPS = 32;
 
 // i-planes per workgroup of the one-sweep launches where none was tuned
@@ -2491,10 +2531,10 @@ RelaxPath stream_path(const wf_mg_level& L, int nsweeps) {
   if (relax_lds2_cpt(L) > 0 && relax_lds2_bytes(L, sizeof(T)) <= lds) return RelaxPath::LDS2;
   // many sweeps in one workgroup pay off only with rhs in LDS too: with rhs
   // read from global memory every colour pass waits on its latency
-  if ((cells <= LDS_RELAX_MAX_CELLS || nsweeps >= LDS_RELAX_MIN_SWEEPS) &&
+  if ((cells <= (size_t)LDS_RELAX_MAX_CELLS || nsweeps >= LDS_RELAX_MIN_SWEEPS) &&
       2 * cells * sizeof(T) <= lds)
     return RelaxPath::LDS_RHS;
-  if (cells <= LDS_RELAX_MAX_CELLS && cells * sizeof(T) <= lds) return RelaxPath::LDS;
+  if (cells <= (size_t)LDS_RELAX_MAX_CELLS && cells * sizeof(T) <= lds) return RelaxPath::LDS;
   return RelaxPath::SWEEPS;
 }
 // Whether the blocks of plan P take nsweeps sweeps faster than stream_path does.
