@@ -1209,9 +1209,8 @@ sweep2_kernel(const T* __restrict__ pin, T* __restrict__ pout, const T* __restri
 template <class T, int RI, int NSEG, int PL, int NT, bool PART, bool PRO>
 __global__ void __launch_bounds__(NT)
     __attribute__((amdgpu_waves_per_eu(NT / 256, sizeof(T) == 4 && !PRO ? 5 : 4)))
-relax_block_kernel(const T* __restrict__ pin, T* pout, const T* __restrict__ rhs, MgDev d, T c0,
-                   T c1, T c2, int ns, int rj, int rk, int tj, int tk,
-                   const T* __restrict__ pc) {
+relax_block_kernel(const T* pin, T* pout, const T* __restrict__ rhs, MgDev d, T c0, T c1, T c2,
+                   int ns, int rj, int rk, int tj, int tk, const T* __restrict__ pc) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int b = xcd_linear(blockIdx.x, gridDim.x);
   relax_block_body<T, RI, NSEG, PL, PART, PRO>(pin, pout, rhs, d, c0, c1, c2, ns, 2 * ns, rj, rk,

@@ -90,9 +90,10 @@ __device__ inline void add_prolonged(T* E, const T* __restrict__ pc, const MgDev
 // RI planes each (the block has NSEG RI planes).  PART: the level may have fewer
 // planes than the block (one block along i then); the planes past it stay zero
 // under a zero reciprocal diagonal, kept per cell.  PRO: the iterate is pin plus
-// the interpolation of pc.
+// the interpolation of pc.  pout may be pin where one block is the level: the
+// barriers after the loads come before any store.
 template <class T, int RI, int NSEG, int PL, bool PART, bool PRO = false>
-__device__ inline void relax_block_body(const T* __restrict__ pin, T* __restrict__ pout,
+__device__ inline void relax_block_body(const T* pin, T* pout,
                                         const T* __restrict__ rhs, const MgDev& d, T c0, T c1,
                                         T c2, int ns, int h, int rj, int rk, Blk B,
                                         T* __restrict__ sm, const T* __restrict__ pc = nullptr) {
