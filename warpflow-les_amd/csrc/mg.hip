@@ -1762,14 +1762,13 @@ coarse_op_sym_even_kernel(double* __restrict__ phi, const double* __restrict__ r
   if (!colour_cell(d, 1, i, j, k)) return;
   const int64_t x = mg_at(d, i, j, k);
   const Coef<double> c = mg_coef(d, i, j, k, c0, c1, c2);
-  // nb_sum, but for the ring: this cell's images there are still phi's old ones
+  // zeros for the ring: this cell's images there are still phi's old ones
   auto nb = [&](int64_t o, bool in) {
     const double q = phi[x + o];
     return in ? q : 0.0;
   };
-  const double sum = c.aw * nb(-d.s0, i > 0) + c.ae * nb(d.s0, i + 1 < d.n0) +
-                     c.as * nb(-d.s1, j > 0) + c.an * nb(d.s1, j + 1 < d.n1) +
-                     c.ab * nb(-1, k > 0) + c.at * nb(1, k + 1 < d.n2);
+  const double sum = nb6(c0, c1, c2, nb(-d.s0, i > 0), nb(d.s0, i + 1 < d.n0), nb(-d.s1, j > 0),
+                         nb(d.s1, j + 1 < d.n1), nb(-1, k > 0), nb(1, k + 1 < d.n2));
   const double v = *any != 0.0 ? (rhs[x] - sum) * (1.0 / c.ap) : 0.0;
   phi[x] = v;
   ring_images(phi, d, i, j, k, x, v);
