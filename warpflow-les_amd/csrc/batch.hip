@@ -201,7 +201,7 @@ int create(const wf_member* mem, int nmem, int nlev, Batch** out) {
   for (int ich = 2; ich <= BATCH_ICH; ich *= 2) {
     int64_t w = 0;
     for (int m = 0; m < nmem; ++m) w += member_count(PK_CELLS, B->mem_host[m], ich);
-    if (w >= 8 * 256) el_ich = ich;
+    if (w >= 8 * cu_count()) el_ich = ich;
   }
   for (int m = 0; m < nmem; ++m) {
     B->mem_host[m].red0 = red;

@@ -1954,7 +1954,7 @@ int batch_mg_init() {
 }
 
 // The relaxation of level l of every member: the tiles and the cheapest of the
-// launches below, costs as in BLOCK_SHAPES (us for the first 256 blocks, ns for
+// launches below, costs as in BLOCK_SHAPES (us for a block per CU, ns for
 // each further one; two-sweep launches: us per plane iteration of a round of
 // three workgroups per CU).
 void batch_relax_plan(const MemDev* mem, int nmem, int l, BatchRelax& P,
@@ -1972,6 +1972,7 @@ void batch_relax_plan(const MemDev* mem, int nmem, int l, BatchRelax& P,
     t[2] = relax_block_tiles(n[2], std::min(n[2], rjk), h);
     return (int64_t)t[0] * t[1] * t[2];
   };
+  const double cus = cu_count();
   int t[3];
   double best = 0;
   P.single = true;
@@ -1981,7 +1982,7 @@ void batch_relax_plan(const MemDev* mem, int nmem, int l, BatchRelax& P,
     int64_t nb = 0;
     for (int m = 0; m < nmem; ++m) nb += blocks(m, S.rjk, 2 * S.ns, t);
     // per six sweeps
-    const double cost = 6 / S.ns * (S.base + 1e-3 * S.more * std::max(0.0, (double)nb - 256.0));
+    const double cost = 6 / S.ns * (S.base + 1e-3 * S.more * std::max(0.0, nb - cus));
     if (P.ns == 0 || cost < best) {
       best = cost;
       P.rjk = S.rjk;
@@ -1993,7 +1994,7 @@ void batch_relax_plan(const MemDev* mem, int nmem, int l, BatchRelax& P,
   // two-sweep launches: the chunk of least total plane iterations
   int nmax = 0;
   for (int m = 0; m < nmem; ++m) nmax = std::max(nmax, mem[m].ln[l][0]);
-  const double slots = 3 * 256;
+  const double slots = 3 * cus;
   for (int ich = 8; ich <= 64 && !P.single; ich += 4) {
     int64_t w = 0;
     for (int m = 0; m < nmem; ++m) {
@@ -2041,7 +2042,7 @@ static bool batch_relax_in_lds(const Batch& B, int l, int n, bool fused) {
   // the loads, then two passes a sweep; further rounds of workgroups overlap a little
   const double c = B.max_lds_cells[l] / 1024.0;
   const double lds = (1.0 + 1.1 * c + n * (0.55 + 0.545 * c)) *
-                     (1.0 + 0.85 * (div_up(B.nmem, 256) - 1));
+                     (1.0 + 0.85 * (div_up(B.nmem, cu_count()) - 1));
   return lds < div_up(n, P.ns) * P.us - (fused ? 4.0 : 0.0);
 }
 
@@ -2086,7 +2087,7 @@ int batch_vcycle(const Batch& B, float* const* phi_, float* const* rhs, float* c
         if (P.rjk == 32)
           run(pc ? batch_relax_block_kernel<32, false, true>
                  : batch_relax_block_kernel<32, false, false>, 1024, 16 * 1152);
-        else if (P.total <= 256)  // one block per CU
+        else if (P.total <= cu_count())  // one block per CU
           run(pc ? batch_relax_block_kernel<16, true, true>
                  : batch_relax_block_kernel<16, true, false>, 1024, 18 * 320);
         else
@@ -2363,8 +2364,8 @@ int sweep2_t(const wf_mg_level& L, const void* pin, void* pout, hipStream_t s) {
 // Relaxation by overlapping blocks (relax_block_kernel): the block shapes, and
 // the choice of shape and sweeps per launch for a level.
 //
-// A launch costs `base` us up to 256 blocks (one per CU) and `more` ns for each
-// further block, both measured (six sweeps, back to back, 24^3 .. 256^3); the
+// A launch costs `base` us up to a block per CU and `more` ns for each
+// further block, both measured on 256 CUs (six sweeps, back to back, 24^3 .. 256^3); the
 // plan with the least total is taken.  Blocks of 16^3 cells (256 threads)
 // relax three times per launch while they fit the CUs once and twice above (once:
 // 1024 threads, six sweeps 12.6 us at 24^3 .. 32^3 in FP32 and 13.7 in FP64, with
@@ -2373,7 +2374,7 @@ int sweep2_t(const wf_mg_level& L, const void* pin, void* pout, hipStream_t s) {
 // in 32 instead of in 16), of 16 planes while they fit the CUs once, else 20.
 struct BlockShape {
   int ri, rjk, ns;   // planes, rows and columns, sweeps per launch
-  double base, more; // us, ns per block past 256
+  double base, more; // us, ns per block past one per CU
 };
 template <class T>
 constexpr BlockShape BLOCK_SHAPES[] = {
@@ -2452,6 +2453,7 @@ bool block_plan(const wf_mg_level& L, int n, bool even, BlockPlan& P) {
     return true;
   }
   if (!L.tmp || (even && n < 2)) return false;
+  const double cus = cu_count();
   double best = 0;
   for (const BlockShape& S : BLOCK_SHAPES<T>) {
     BlockPlan Q;
@@ -2471,10 +2473,10 @@ bool block_plan(const wf_mg_level& L, int n, bool even, BlockPlan& P) {
     const double blocks = (double)relax_block_tiles(L.n0, Q.ri, h) *
                           relax_block_tiles(L.n1, Q.rj, h) * relax_block_tiles(L.n2, Q.rk, h);
     // 32 x 32 columns fill a CU's registers: its second block waits for the first
-    const double b = S.rjk == 32 ? std::ceil(blocks / 256.0) * 256.0 : blocks;
-    const double cost = Q.launches * (S.base + 1e-3 * S.more * std::max(0.0, b - 256.0));
+    const double b = S.rjk == 32 ? std::ceil(blocks / cus) * cus : blocks;
+    const double cost = Q.launches * (S.base + 1e-3 * S.more * std::max(0.0, b - cus));
     // (eight planes: the part kernel, also where the level has all eight)
-    Q.seg = Q.part || Q.ri == 8 || (S.rjk == 16 && blocks <= 256);
+    Q.seg = Q.part || Q.ri == 8 || (S.rjk == 16 && blocks <= cus);
     if (P.launches == 0 || cost < best) {
       P = Q;
       best = cost;
@@ -2483,7 +2485,7 @@ bool block_plan(const wf_mg_level& L, int n, bool even, BlockPlan& P) {
       constexpr double b0 = f64 ? 4.4 : 3.85;
       const double cf = (double)(Q.rj * Q.rk) / (S.rjk * S.rjk), pf = (double)Q.ri / S.ri;
       P.us = Q.launches * (b0 + (S.base - b0) * pf * cf +
-                           1e-3 * S.more * std::max(0.0, b - 256.0) * (1 + pf) / 2 *
+                           1e-3 * S.more * std::max(0.0, b - cus) * (1 + pf) / 2 *
                                (0.2 + 0.8 * cf));
     }
   }
@@ -2561,7 +2563,7 @@ bool block_cheaper(const wf_mg_level& L, int nsweeps, const BlockPlan& P, bool f
       const int64_t tiles = L.n2 > 32 ? (int64_t)div_up(L.n2, 64) * div_up(L.n1, 8)
                                       : (int64_t)div_up(L.n2, 32) * div_up(L.n1, 16);
       const int ich = sweep_ich(tiles, L.n0), p = std::min(ich, L.n0);
-      const double more = std::max<double>(0, (double)tiles * div_up(L.n0, ich) / 256 - 1);
+      const double more = std::max<double>(0, (double)tiles * div_up(L.n0, ich) / cu_count() - 1);
       return us <= nsweeps * (f64 ? 5.6 + 0.75 * p + (2.0 + 0.25 * p) * more
                                   : 4.9 + 0.6 * p + (1.1 + 0.22 * p) * more);
     }
