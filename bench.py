@@ -208,13 +208,26 @@ class Flush:
         copy(self.b, self.a)
 
 
+def smoother(level, nsweeps, ctype):
+    """The kernel and the launches of nsweeps sweeps of a level (wf_mg_relax)."""
+    from warpflow import _hip
+    plan = (C.c_int32 * 4)()
+    _hip.call("wf_mg_relax_plan", C.byref(level), nsweeps, plan)
+    kern = {1: "relax_block_kernel<%s> (several RBGS sweeps per launch)",
+            2: "relax_lds2_kernel<%s> (every RBGS sweep in one launch)",
+            3: "sweep2_kernel<%s> (two RBGS sweeps per launch)",
+            4: "sweep_kernel<%s> (one RBGS sweep per launch)",
+            5: "rbgs_kernel<%s> (half an RBGS sweep per launch)"}[plan[0]]
+    return kern % ctype, plan[1]
+
+
 def hot_kernels(a, s64, smx):
     """The hot kernels and launch groups of one step on the solvers' own
     arrays: dicts with the launch (fn), the kernel it runs, launches and
     algorithmic bytes per call, and calls per step of each form with two
     outer iterations (one pressure solve: 4 V-cycles in the FP64 form,
     --mixed-cycles in the mixed form)."""
-    from warpflow import _hip, autotune
+    from warpflow import _hip
     from warpflow import kernels as K
     from warpflow.device import copy, current_stream
     from warpflow.topology import NPL
@@ -284,18 +297,14 @@ def hot_kernels(a, s64, smx):
     for tag, mg, eb, cyc64, cycmx in (("fp64", s64.mg, 8, nv, 0), ("fp32", smx.mg, 4, 0, nm)):
         lv0, lv1 = mg.levels[0], mg.levels[1]
         L0, L1 = lv0.desc(), lv1.desc()
-        knob = autotune.SWEEP_PAIRS_F64 if eb == 8 else autotune.SWEEP_PAIRS_F32
-        pairs = autotune.get_shape(knob, lv0.n3)
-        two = pairs == 2 or (pairs == 0 and cells >= (1750000 if eb == 8 else 3500000))
         ctype = "double" if eb == 8 else "float"
-        kern = ("sweep2_kernel<%s> (two RBGS sweeps per launch)" % ctype if two
-                else "sweep_kernel<%s> (one RBGS sweep per launch)" % ctype)
+        kern, nlaunch = smoother(L0, nsw, ctype)
         # one cycle's level-0 smoothing (6 pre + 6 post sweeps) as one group of
         # launches: the first reads arrays another kernel touched long before,
         # the others read what the previous sweep wrote, as in a V-cycle
         out.append(row("rbgs %d sweeps L0 (%s)" % (nsw, tag), kern,
                        lambda L0=L0: _hip.call("wf_mg_relax", C.byref(L0), nsw, st),
-                       nsw * (4 * eb) * cells, cyc64, cycmx, nsw // 2 if two else nsw))
+                       nsw * (4 * eb) * cells, cyc64, cycmx, nlaunch))
         out.append(row("restrict L0 (%s)" % tag, "restrict_kernel<%s>" % ctype,
                        lambda L0=L0, L1=L1: _hip.call("wf_mg_restrict", C.byref(L0),
                                                       C.byref(L1), st),
@@ -436,10 +445,12 @@ ROW_KERNELS = {
     "add_ring": ("add_kernel(",),
     "copy (u -> uoo)": ("copy16_kernel(",),
     "bc_fill (u)": ("bc_axis_kernel(",),
-    "rbgs 12 sweeps L0 (fp64)": ("sweep2_kernel<double", "sweep_kernel<double"),
+    "rbgs 12 sweeps L0 (fp64)": ("sweep2_kernel<double", "sweep_kernel<double",
+                                 "relax_block_kernel<double"),
     "restrict L0 (fp64)": ("restrict_kernel<double>",),
     "prolong L0 (fp64)": ("prolong8_kernel<double>", "prolong_kernel<double>"),
-    "rbgs 12 sweeps L0 (fp32)": ("sweep2_kernel<float", "sweep_kernel<float"),
+    "rbgs 12 sweeps L0 (fp32)": ("sweep2_kernel<float", "sweep_kernel<float",
+                                 "relax_block_kernel<float"),
     "restrict L0 (fp32)": ("restrict_kernel<float>",),
     "prolong L0 (fp32)": ("prolong8_kernel<float>", "prolong_kernel<float>"),
 }
