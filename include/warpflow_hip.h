@@ -52,9 +52,10 @@ typedef struct wf_grid {
  * Coefficients are matrix-free: 1/h^2 per face, 0 across the six physical
  * faces of the single cavity domain, ap = -(aw+ae+as+an+ab+at)
  * (multigrid.py:23-67).  tmp (nullable) is a second array of phi's shape,
- * zero-initialised: with it, smoothing runs as fused full sweeps that
- * ping-pong phi -> tmp -> phi (results always end in phi); without it, as
- * two in-place half-sweep launches per sweep. */
+ * zero-initialised: with it, smoothing runs as full sweeps or as blocks of
+ * several, which ping-pong phi -> tmp -> phi (results always end in phi); without
+ * it in place, as one block or in LDS where the level fits, else as two
+ * half-sweep launches per sweep. */
 typedef struct wf_mg_level {
   void* phi;
   void* rhs;
@@ -354,8 +355,8 @@ int wf_mg_rbgs(const wf_mg_level* lev, int color, void* stream);
 int wf_mg_refill(const wf_mg_level* lev, void* stream);
 
 /* Multigrid._relax, multigrid.py:289-299: nsweeps x (colour 0, colour 1,
- * refill).  Levels whose arrays fit the workgroup's LDS run all sweeps in one
- * single-workgroup launch. */
+ * refill), by the smoother that is estimated to be the fastest for the level's
+ * extents and the count (wf_mg_relax_plan); every one gives the same bits. */
 int wf_mg_relax(const wf_mg_level* lev, int nsweeps, void* stream);
 
 /* How wf_mg_relax runs nsweeps sweeps of lev (no arrays are touched):
@@ -578,7 +579,8 @@ int wf_batch_add_ring(wf_batch b, double* p, const double* pp, const int* active
                       void* stream);
 /* wf_mg_solve_mixed with a fixed ncycles (no tolerance test, no host sync):
  * phi/rhs/tmp = FP32 level pools (nlev each), cop = operator pool or NULL
- * (NULL: n_coarse sweeps on the coarsest level), flags 2 = remove the mean. */
+ * (NULL: n_coarse sweeps on the coarsest level), flags 2 = remove the mean.
+ * Levels of more than 4096 cells in some member take even sweep counts. */
 int wf_batch_mg_solve_mixed(wf_batch b, float* const* phi, float* const* rhs, float* const* tmp,
                             const float* cop, const double* su, double* pp, int ncycles,
                             int n_pre, int n_post, int n_coarse, int flags, const int* active,
@@ -624,8 +626,10 @@ int wf_batch_set_int(int* p, int n, int value, void* stream);
  *   WF_TUNE_SWEEP_PAIRS_F64/F32 pairs of sweeps of this level as 1 = two
  *                               one-sweep launches, 2 = one two-sweep launch
  * A level with none of the SWEEP tile, ICH and PAIRS knobs set takes the
- * built-in smoother: blocks relaxed several times per launch on levels of
- * fewer than 1.75e6 (FP64) or 3.5e6 (FP32) cells, two-sweep launches above.
+ * built-in smoother (wf_mg_relax_plan): on levels of fewer than 1.75e6 (FP64) or
+ * 3.5e6 (FP32) cells blocks relaxed several times per launch, or the LDS or
+ * one-sweep launches where those are estimated to be faster; two-sweep
+ * launches above, one-sweep launches for levels of few planes or rows.
  *   WF_TUNE_PROJ_ICH            i-planes per workgroup of wf_calvel3_calmas
  *                               (raised where needed to keep the workgroup
  *                               count within the reduction's partial slots)

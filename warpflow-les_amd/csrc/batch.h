@@ -4,11 +4,12 @@
 // Every field of every member lives in one pool per field name (member m's
 // (n0+6)(n1+6)(n2+6) array at element offset off); every multigrid level l
 // in one pool per level array (member m's (n_l+2)^3 array at loff[l]).  A
-// batched launch walks a list of work items -- (member, local block) pairs
-// numbered member after member -- with a grid-stride loop: the grid is at
-// most the number of workgroups the device holds at once (a persistent
-// launch), and each item is decoded into the block coordinates the
-// single-domain kernel body expects, so both paths run the same arithmetic.
+// batched launch covers a list of work items -- (member, block coordinates),
+// numbered member after member -- and runs the single-domain kernel body on
+// them, so both paths run the same arithmetic.  The passes over whole fields and
+// levels launch a workgroup per entry of a table made at creation; the others
+// are a grid-stride loop of at most the workgroups the device holds at once,
+// which finds an item's member by search, or a workgroup per member.
 // A per-member `active` mask (nullable) lets converged members skip the
 // projection iterations of the others inside one captured graph.
 #pragma once

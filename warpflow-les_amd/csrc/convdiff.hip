@@ -1445,10 +1445,11 @@ int batch_convdiff(const Batch& B, int comp, const double* u, const double* v,
   return 0;
 }
 
-// Launch of the fused operator on box b (checked by the caller).
 // conv4th alone on the fused pass's tiles: a thread per cell with every tap from
 // global memory took about fifty loads and three FP64 divisions, 25 us for 96 x 80
-// x 112 cells in the caches; here 14 us (the traffic's floor is 5).
+// x 112 cells in the caches; here 14 us (the traffic's floor is 5).  Up to 48^3
+// cells the two took the same 6 us; boxes of one or two rows leave most of a
+// tile idle (512 x 2 x 512: 19 us for 14).
 int conv_launch(int comp, const double* u, const double* v, const double* w, const double* coo,
                 double* cstar, const wf_grid& g, const Box3& b, double dx, double dy, double dz,
                 double dta, hipStream_t s) {
@@ -1474,6 +1475,7 @@ int conv_launch(int comp, const double* u, const double* v, const double* w, con
   return 0;
 }
 
+// Launch of the fused operator on box b (checked by the caller).
 int convdiff_launch(int comp, const double* u, const double* v, const double* w,
                     const double* coo, const double* vis, double* cstar, const wf_grid& g,
                     const Box3& b, double dx, double dy, double dz, double dta, int ich,

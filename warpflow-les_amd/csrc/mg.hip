@@ -2249,10 +2249,10 @@ int launch_relax_lds(const wf_mg_level& L, int nsweeps, size_t bytes, hipStream_
   return 0;
 }
 
-// Levels up to LDS_RELAX_MAX_CELLS cells -- or any level that fits LDS when
-// asked for many sweeps (the coarsest solve) -- relax in one LDS-resident
-// workgroup; the rest in fused full-sweep launches (or half-sweep launches
-// without tmp).
+// Where blocks are not taken (stream_path): levels up to LDS_RELAX_MAX_CELLS cells
+// -- or any level that fits LDS when asked for many sweeps (the coarsest solve) --
+// relax in one LDS-resident workgroup; the rest in fused full-sweep launches (or
+// half-sweep launches without tmp).
 constexpr int LDS_RELAX_MIN_SWEEPS = 32;
 
 // i-planes per workgroup of the one-sweep launches where none was tuned
