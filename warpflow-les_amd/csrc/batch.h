@@ -107,7 +107,6 @@ enum PlanKind : int {
   PK_STREAM,        // the same tiles, other chunks: WALE and calvel3_calmas
   PK_CDE,           // u's edge planes 0 and ni-2: 8 x 32 (j, k) tiles x 2
   PK_XG,            // w's cross-ghost cells of each real plane, 256 per item
-  PK_MEMBER,        // one item per member
   PK_COP,           // 32-row blocks of the coarsest level's operator
   PK_LCELLS0,       // 64x4 tiles over single planes of level l, l = 0 .. 7
   PK_COUNT = PK_LCELLS0 + BATCH_MAX_LEVELS

@@ -80,8 +80,6 @@ int member_count(int kind, const MemDev& M, int ich) {
       return ((n2 + 31) / 32) * ((n1 + 7) / 8) * (n0 - 1 > 1 ? 2 : (n0 - 1 > 0 ? 1 : 0));
     case PK_XG:
       return ((2 * (n2 + 3) + 4 * n1 + 255) / 256) * n0;
-    case PK_MEMBER:
-      return 1;
     case PK_COP: {
       const int* c = M.ln[M.nlev - 1];
       return (c[0] * c[1] * c[2] + 31) / 32;
